@@ -61,6 +61,29 @@ def test_bruteforce_boxes_subset_matches_oracle():
     assert rel_l2(got, ref) <= 1e-4
 
 
+@pytest.mark.parametrize("diffuse_only", [True, False])
+@pytest.mark.parametrize("width,height,read,wide", [(9, 7, 8, 0), (250, 131, 16, 1), (65, 63, 1, 0), (8, 8, 2, 0)])
+def test_bruteforce_tile_and_group_edges_match_oracle(width, height, read, wide, diffuse_only):
+    """Pixel tiles cut by the window's edge, VAL counts from one (fewer than a
+    group of four) to 2:1, every wave's share of the groups empty or not."""
+    from dataclasses import replace
+
+    from dynamicradiancevolume_amd import workloads as W
+    from oracle import orc
+
+    light = replace(W.BOXES_1080P.light, rsm_resolution=read, rsm_read_lod=0, rsm_wide=wide, indirect_shadow_lod=0)
+    fi = frame_inputs("boxes_1080p", n_objects=60, tess=3, width=width, height=height, light=light)
+    announce(f"brute force {width}x{height}, read level {read}, wide {wide}, diffuse_only={diffuse_only}")
+    r, df = _setup(fi)
+    out = torch.full((height, width, 3), 7.0, device="cuda")
+    rm = None if diffuse_only else df.groughmetal
+    r.bruteforce_rsm(df.gbuffer(), df.rsm(), fi.light, out, diffuse_only, rm)
+    got = out.cpu().numpy().reshape(-1, 3)
+    ref = orc.bruteforce_rsm(fi, diffuse_only, None if diffuse_only else fi.groughmetal)
+    assert np.linalg.norm(ref) > 0 and rel_l2(got, ref) <= 1e-4
+    assert np.all(got[fi.depth.reshape(-1) < 1e-5] == 0)
+
+
 @pytest.mark.parametrize("sh_bands", [1, 2])
 def test_cache_path_vs_bruteforce_end_to_end(sh_bands):
     """The unshadowed cache path (SH interpolation of the diffuse irradiance)
