@@ -32,7 +32,8 @@ constexpr uint32_t kMaxSplits = 256;  // VPL splits of the SH gather (each at le
 // One VPL ("LightInfo", cacheLightingRSM.comp:34-40) packed for LDS staging.
 struct Vpl {
   float px, py, pz, disc_area;
-  float fr, fg, fb, pad0;
+  float fr, fg, fb;
+  uint32_t quad_flux;  // the bits of all flux of the aligned group of four VPLs or'ed: 0 = the group is dark
   float nx, ny, nz, pad1;
 };
 

@@ -27,6 +27,7 @@
 // all views.  Small views no longer leave the GPU idle behind their own
 // launches, and no view waits for another's tail.
 #include <algorithm>
+#include <type_traits>
 #include <cstring>
 
 #include "drv_internal.hpp"
@@ -418,9 +419,17 @@ __global__ __launch_bounds__(256) void k_split_gather(const SplitDev* views, uin
     const SplitDev& d = views[v];
     const uint32_t groups = (d.splits + 3u) / 4u;
     const uint32_t local = item - d.gather_begin;
-    const uint32_t tile = local / groups, group = local - tile * groups;
-    gather_item<kSh2, kShadow>(d.caches, stride, d.live, d.prep.vpls, d.n_vpl, d.vis, d.vis_pitch, d.interval,
-                               d.partial, d.partial_pitch, d.splits, tile, group, part);
+    const uint32_t group = local / d.tiles, tile = local - group * d.tiles;  // group-major, as k_gather
+    auto gather = [&](auto shadow) {
+      gather_item<kSh2, decltype(shadow)::value>(d.caches, stride, d.live, d.prep.vpls, d.n_vpl, d.vis, d.vis_pitch,
+                                                 d.interval, d.partial, d.partial_pitch, d.splits, tile, group, part);
+    };
+    if (!kShadow)
+      gather(std::integral_constant<int, kShadowNone>());
+    else if (d.interval < 4u)  // a view with shadow LOD 0
+      gather(std::integral_constant<int, kShadowUnits>());
+    else
+      gather(std::integral_constant<int, kShadowBlocks>());
     __syncthreads();  // part is rewritten by the next item
   }
 }

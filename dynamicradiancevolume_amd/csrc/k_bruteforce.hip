@@ -18,7 +18,7 @@
 //  - groups that face away from, or lie behind, the surface of every pixel of
 //    the tile are skipped after the two cosines' signs: 59 % of the groups
 //    with flux on boxes_1080p, 39 % on a 637x359 view of 300 boxes.
-// 1920x1080 x 16384 VALs, diffuse: 25.6 -> 8.4 ms; 637x359 x 4096, whole BRDF:
+// 1920x1080 x 16384 VALs, diffuse: 25.6 -> 7.7 ms; 637x359 x 4096, whole BRDF:
 // 1.78 -> 0.67 ms.  Two and four pixels per lane (fewer scalar loads per pair)
 // took 15.8 and 16.6 ms against 14.9 ms with one, before the second skip.
 #include "drv_internal.hpp"
@@ -138,15 +138,13 @@ __global__ __launch_bounds__(256) void k_bruteforce(BruteArgs a) {
     for (uint32_t g = g0; g < g1; ++g) {
       const ValRecord v = vals + 12u * g;
       float4v pos[4], flux[4], nrm[4];
-      uint32_t any = 0u;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         pos[j] = v[3 * j];
         flux[j] = v[3 * j + 1];
         nrm[j] = v[3 * j + 2];
-        any |= __float_as_uint(flux[j].x) | __float_as_uint(flux[j].y) | __float_as_uint(flux[j].z);
       }
-      if (any == 0u) continue;
+      if (__float_as_uint(flux[0].w) == 0u) continue;  // Vpl::quad_flux
       BrutePair e[4];
       float m[4];
 #pragma unroll

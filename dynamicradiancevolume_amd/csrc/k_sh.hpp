@@ -27,19 +27,19 @@ __device__ __forceinline__ void sh_zero(ShSums& a) {
   for (int k = 0; k < 27; ++k) a.s[k] = 0.0f;
 }
 
-// One cache.VPL interaction with the block's shadowing term.
+// One cache.VPL interaction with the block's shadowing term: (tx0, ty0, tz0)
+// leads from the cache to the VPL, nd0 is its unnormalized cosine with the
+// VPL's normal.
 template <bool kSh2>
-__device__ __forceinline__ void sh_accumulate(ShSums& a, const Vpl& v, float wx, float wy, float wz,
-                                              float shadowing) {
-  const float tx0 = v.px - wx, ty0 = v.py - wy, tz0 = v.pz - wz;
+__device__ __forceinline__ void sh_accumulate(ShSums& a, float disc_area, float fr, float fg, float fb, float tx0,
+                                              float ty0, float tz0, float nd0, float shadowing) {
   const float d2 = __builtin_fmaf(tz0, tz0, __builtin_fmaf(ty0, ty0, tx0 * tx0));
   const float inv = __builtin_amdgcn_rsqf(d2);
   const float tx = tx0 * inv, ty = ty0 * inv, tz = tz0 * inv;
-  const float nd = -__builtin_fmaf(v.nz, tz, __builtin_fmaf(v.ny, ty, v.nx * tx));
-  float k = fminf(1.0f, fmaxf(0.0f, nd));
+  float k = fminf(1.0f, fmaxf(0.0f, nd0 * inv));
   k = k * shadowing;
-  const float f = k * __builtin_amdgcn_rcpf(d2 + v.disc_area);
-  const float rad[3] = {v.fr * f, v.fg * f, v.fb * f};
+  const float f = k * __builtin_amdgcn_rcpf(d2 + disc_area);
+  const float rad[3] = {fr * f, fg * f, fb * f};
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
     a.s[c] += rad[c];
@@ -59,6 +59,15 @@ __device__ __forceinline__ void sh_accumulate(ShSums& a, const Vpl& v, float wx,
       a.s[24 + c] = __builtin_fmaf(bdd, rad[c], a.s[24 + c]);
     }
   }
+}
+
+// The same from the cache's position.
+template <bool kSh2>
+__device__ __forceinline__ void sh_accumulate(ShSums& a, const Vpl& v, float wx, float wy, float wz,
+                                              float shadowing) {
+  const float tx = v.px - wx, ty = v.py - wy, tz = v.pz - wz;
+  const float nd = -__builtin_fmaf(v.nz, tz, __builtin_fmaf(v.ny, ty, v.nx * tx));
+  sh_accumulate<kSh2>(a, v.disc_area, v.fr, v.fg, v.fb, tx, ty, tz, nd, shadowing);
 }
 
 // Adds coefficient j (0..8), channel ch of raw sums v (v0 = the channel's

@@ -339,6 +339,39 @@ def test_gather_cornell_unshadowed():
     _gather_case("cornell_256", indirect_shadow=0, sh_bands=2)
 
 
+@pytest.mark.parametrize("read,lod,wide,sh_bands", [(8, 0, 0, 2), (16, 0, 1, 1), (32, 1, 0, 2), (32, 4, 0, 1)])
+def test_gather_shadow_block_sizes_match_oracle(read, lod, wide, sh_bands):
+    """Blocks of one VPL (each with its own visibility), of exactly one group
+    of four, and of more VPLs than a wave has lanes; alone and as the view of
+    a batch's queued gather, whose blocks differ from its neighbour's."""
+    from dynamicradiancevolume_amd import workloads as W
+    from dynamicradiancevolume_amd.pipeline import Batch, DeviceFrame, Renderer, entries_sh
+
+    orc = _orc()
+    c = W.CORNELL_256.with_(sh_bands=sh_bands, width=96, height=64, max_caches=8192)
+    light = W.replace(c.light, rsm_resolution=read, rsm_read_lod=0, rsm_wide=wide, indirect_shadow_lod=lod)
+    frames = [W.make_inputs(c.with_(light=light)), W.make_inputs(c)]
+    announce(f"gather read level {read}, wide {wide}, shadow LOD {lod}, SH{sh_bands}")
+    dfs = [DeviceFrame(fi) for fi in frames]
+    alone, view, other = (Renderer(c.config()) for _ in range(3))
+    alone.render_frame(dfs[0])
+    batch = Batch([view, other])
+    batch.set_tuning(-2, 1024)
+    batch.render_frame(dfs)
+    fi, cfg = frames[0], c.config()
+    vol = orc.update_volume(cfg, c.eye, fi.bbox[:3], fi.bbox[3:])
+    _, mips = orc.voxelize(c.voxel_resolution, vol, fi.positions, adaption_factor=1.0)
+    for r in (alone, view):
+        _, live = r.cache_count()
+        got = r.read_caches(live)
+        ref = got.copy()
+        ref[:, 4:] = 0.0
+        orc.gather_f32(cfg, vol, orc.sh_constants(), fi.light, fi, mips, ref, n=live)
+        err = rel_l2(entries_sh(got, sh_bands), entries_sh(ref, sh_bands))
+        assert err < SH_TOL, f"SH relative L2 {err:.3e}"
+    batch.close()
+
+
 def test_gather_boxes_all_caches():
     """Every cache of the 1080p frame (6.5M cone traces) against the oracle."""
     announce("gather boxes_1080p, all caches")
