@@ -851,7 +851,8 @@ int prepare_light(drv_ctx* ctx, const drv_rsm* rsm, const drv_spot_light* light,
     dev_free(ctx->march);
     ctx->block_cap = 0;
     if ((rc = dev_alloc(ctx, &ctx->blocks, n_blocks)) != DRV_OK) return rc;
-    if ((rc = dev_alloc(ctx, &ctx->march, static_cast<size_t>(n_blocks) * drvk::kMarchSteps)) != DRV_OK) return rc;
+    // One record more: a march loads a step ahead.
+    if ((rc = dev_alloc(ctx, &ctx->march, static_cast<size_t>(n_blocks) * drvk::kMarchSteps + 1)) != DRV_OK) return rc;
     ctx->block_cap = n_blocks;
   }
   return DRV_OK;

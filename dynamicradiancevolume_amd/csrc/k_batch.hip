@@ -392,15 +392,15 @@ __global__ __launch_bounds__(256) void k_split_visibility(const SplitDev* views,
       const bool valid = cache < w.live;
       const float* e = w.caches + static_cast<size_t>(valid ? cache : w.live - 1u) * stride;
       const f3 wp = make3(e[0], e[1], e[2]);
-      const float vsz = w.voxel_size * static_cast<float>(w.vox.res);
-      // cacheLightingRSM.comp:103-104
-      const f3 vpos = make3((wp.x - w.vmin[0]) / vsz, (wp.y - w.vmin[1]) / vsz, (wp.z - w.vmin[2]) / vsz);
+      const float vsz = w.voxel_size * static_cast<float>(w.vox.res), inv_vsz = 1.0f / vsz;
+      const f3 vpos = make3(volume_coord(wp.x - w.vmin[0], vsz, inv_vsz), volume_coord(wp.y - w.vmin[1], vsz, inv_vsz),
+                            volume_coord(wp.z - w.vmin[2], vsz, inv_vsz));
       const __amdgpu_buffer_rsrc_t cr = corner_rsrc(w.vox);
       const uint32_t b0 = group * kSplitBpi, b1 = min(w.n_blocks, b0 + kSplitBpi);
       for (uint32_t b = b0; b < b1; ++b) {
-        Trace t = trace_setup(w.vox, w.voxel_size, wp, vpos, block_record(w.blocks, b));
-        if (w.fidx) trace_planned<false, true>(march_steps(w.march, b), cr, t, valid);
-        else trace_planned<false, false>(march_steps(w.march, b), cr, t, valid);
+        const Trace t =
+            w.fidx ? trace_planned<false, true>(w.vox, cr, w.blocks, w.march, b, w.voxel_size, wp, vpos, valid)
+                   : trace_planned<false, false>(w.vox, cr, w.blocks, w.march, b, w.voxel_size, wp, vpos, valid);
         if (valid) w.vis[static_cast<size_t>(b) * w.pitch + cache] = trace_visibility(t);
       }
     }

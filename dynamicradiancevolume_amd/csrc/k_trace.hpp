@@ -141,13 +141,14 @@ __device__ __forceinline__ ShadowBlock block_record(const ShadowBlock* blocks, u
   const BlockRecord r = (BlockRecord)(blocks + block);  // NOLINT(old-style-cast)
   return ShadowBlock{r->x, r->y, r->z, r->rho, r->nx, r->ny, r->nz, r->k};
 }
-// One 64-byte record, one s_load_dwordx16.  (Elements are copied to scalars
-// before the bit casts: a bit cast of an ext_vector element lvalue read the
-// vector's first element on this compiler.)
-__device__ __forceinline__ MarchStep march_step(MarchSteps pl, int n) {
+// The 64-byte record at byte `offset` of a plan, one s_load_dwordx16.
+// (Elements are copied to scalars before the bit casts: a bit cast of an
+// ext_vector element lvalue read the vector's first element on this compiler.)
+__device__ __forceinline__ MarchStep march_step(MarchSteps pl, uint32_t offset) {
   typedef uint32_t u32x16 __attribute__((ext_vector_type(16)));
   typedef const __attribute__((address_space(4))) u32x16* Raw;
-  const u32x16 v = *((Raw)(pl + n));  // NOLINT(old-style-cast)
+  typedef const __attribute__((address_space(4))) char* Bytes;
+  const u32x16 v = *((Raw)((Bytes)pl + offset));  // NOLINT(old-style-cast)
   uint32_t w[16];
 #pragma unroll
   for (int i = 0; i < 16; ++i) w[i] = v[i];
@@ -175,24 +176,29 @@ __device__ __forceinline__ MarchStep march_step(MarchSteps pl, int n) {
 // (samples taken) is kept only with kCount: it costs a VALU instruction per
 // sample and only the step counters read it.
 template <bool kCount = false, bool kFloatIndex = false>
-__device__ __forceinline__ bool march_planned(MarchSteps pl, __amdgpu_buffer_rsrc_t cr, Trace& t, int n0, int n1) {
+__device__ __forceinline__ bool march_planned(MarchSteps pl, const MarchStep& first, __amdgpu_buffer_rsrc_t cr,
+                                              Trace& t, int n0, int n1) {
   // The lanes that march stay in lockstep (all start at sample n0 and take
   // one sample per iteration until they stop), so the sample index is
   // wave-uniform and the record load is scalar.
   bool stopped = false;
-  MarchStep next = march_step(pl, __builtin_amdgcn_readfirstlane(n0));
+  uint32_t off = __builtin_amdgcn_readfirstlane(n0) * sizeof(MarchStep);
+  MarchStep next = first;
   for (int n = n0; n < n1; ++n) {
     const MarchStep cur = next;
-    next = march_step(pl, __builtin_amdgcn_readfirstlane(min(n + 1, kMarchSteps - 1)));  // a step ahead
+    off += sizeof(MarchStep);  // past sample 31: the next block's record, or the padding one, not used
     t.px = __builtin_fmaf(t.dx, cur.step, t.px);
     t.py = __builtin_fmaf(t.dy, cur.step, t.py);
     t.pz = __builtin_fmaf(t.dz, cur.step, t.pz);
-    // Both loads are issued before either record is blended.
     const Footprint f1 = footprint<kFloatIndex>(cur.lv[0], t.px, t.py, t.pz);
-    const Footprint f2 = footprint<kFloatIndex>(cur.lv[1], t.px, t.py, t.pz);
     const corner_t c1 = corner_load(cr, f1.offset);
-    corner_t c2;  // read only when loaded (cur.two is wave-uniform)
-    if (cur.two) c2 = corner_load(cr, f2.offset);
+    Footprint f2;
+    corner_t c2;
+    if (cur.two) {  // wave-uniform; both loads are issued before either record is blended
+      f2 = footprint<kFloatIndex>(cur.lv[1], t.px, t.py, t.pz);
+      c2 = corner_load(cr, f2.offset);
+    }
+    next = march_step(pl, off);  // a step ahead
     const float o1 = blend_corner(c1, f1.ax, f1.ay, f1.az);
     float o = o1;
     if (cur.two) o = __builtin_fmaf(cur.frac, blend_corner(c2, f2.ax, f2.ay, f2.az) - o1, o1);
@@ -206,11 +212,27 @@ __device__ __forceinline__ bool march_planned(MarchSteps pl, __amdgpu_buffer_rsr
   return stopped;
 }
 
-// The whole trace (samples 0 .. 31) of a ray; lanes with live = false take
-// no samples.
+// (wp - vmin) / vsz of a cache (cacheLightingRSM.comp:103-104) with inv = 1 / vsz
+// correctly rounded: a quotient estimate corrected by its exact remainder is
+// the correctly rounded quotient (Markstein), the value of the division.
+__device__ __forceinline__ float volume_coord(float d, float vsz, float inv) {
+  const float q = d * inv;
+  return __builtin_fmaf(__builtin_fmaf(-q, vsz, d), inv, q);
+}
+
+// The whole trace (samples 0 .. 31) of cache wp towards block b, the same for
+// every lane of the wave; lanes with live = false take no samples.
 template <bool kCount = false, bool kFloatIndex = false>
-__device__ __forceinline__ void trace_planned(MarchSteps pl, __amdgpu_buffer_rsrc_t cr, Trace& t, bool live) {
-  if (live) march_planned<kCount, kFloatIndex>(pl, cr, t, 0, kMarchSteps);
+__device__ __forceinline__ Trace trace_planned(const VoxelView& vox, __amdgpu_buffer_rsrc_t cr, const ShadowBlock* blocks,
+                                               const MarchStep* march, uint32_t b, float voxel_size, f3 wp, f3 vpos,
+                                               bool live) {
+  const MarchSteps pl = march_steps(march, b);
+  const MarchStep first = march_step(pl, 0u);
+  const ShadowBlock rec = block_record(blocks, b);
+  Trace t = trace_setup(vox, voxel_size, wp, vpos, rec);
+  asm volatile("" ::"s"(first.step));  // keeps the load above the branch, beside the ones before it
+  if (live) march_planned<kCount, kFloatIndex>(pl, first, cr, t, 0, kMarchSteps);
+  return t;
 }
 
 // Steps the reference takes for a ray traced by trace_planned (geometry
