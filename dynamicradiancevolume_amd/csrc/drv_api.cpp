@@ -83,9 +83,9 @@ struct drv_ctx {
   float* mlp_v = nullptr;
   float* mlp_grad = nullptr;  // reduced gradient [kMlpParams + 1] (last: loss)
   void* mlp_pack = nullptr;   // inference operands
-  void* mlp_train_w = nullptr;  // training LDS images
+  void* mlp_back = nullptr;  // packed backward operands
   float* mlp_partial = nullptr;
-  size_t mlp_partial_waves = 0;
+  size_t mlp_partial_cap = 0;
   uint32_t* mlp_idx = nullptr;
   size_t mlp_idx_cap = 0;
   uint32_t* mlp_pairs = nullptr;
@@ -543,7 +543,7 @@ int drv_destroy(drv_ctx* ctx) {
   dev_free(ctx->mlp_v);
   dev_free(ctx->mlp_grad);
   dev_free(ctx->mlp_pack);
-  dev_free(ctx->mlp_train_w);
+  dev_free(ctx->mlp_back);
   dev_free(ctx->mlp_partial);
   dev_free(ctx->mlp_idx);
   dev_free(ctx->mlp_pairs);
@@ -1276,7 +1276,7 @@ int mlp_alloc(drv_ctx* ctx) {
   if ((rc = dev_alloc(ctx, &ctx->mlp_v, drvk::kMlpParams)) != DRV_OK) return rc;
   if ((rc = dev_alloc(ctx, &ctx->mlp_grad, drvk::kMlpParams + 1)) != DRV_OK) return rc;
   if ((rc = dev_alloc(ctx, reinterpret_cast<uint8_t**>(&ctx->mlp_pack), drvk::kMlpPackBytes)) != DRV_OK) return rc;
-  if ((rc = dev_alloc(ctx, reinterpret_cast<uint16_t**>(&ctx->mlp_train_w), drvk::kMlpTrainW)) != DRV_OK) return rc;
+  if ((rc = dev_alloc(ctx, reinterpret_cast<uint8_t**>(&ctx->mlp_back), drvk::kMlpBackBytes)) != DRV_OK) return rc;
   if ((rc = dev_alloc(ctx, &ctx->mlp_n, 1)) != DRV_OK) return rc;
   return DRV_OK;
 }
@@ -1292,26 +1292,26 @@ int require_features(drv_ctx* ctx) {
   return DRV_OK;
 }
 
-// Gradient of the mean loss over the `batch` samples listed in mlp_idx: the
-// training kernel's per-wave partials, reduced in a fixed order into mlp_grad
+// Gradient of the mean loss over the `batch` samples idx lists (null: all): the
+// training kernel's per-workgroup partials, reduced in a fixed order into mlp_grad
 // (last entry: summed loss), and for lr > 0 one Adam step plus a repack.
-int mlp_step(drv_ctx* ctx, const float* x, const float* y, uint32_t batch, float lr) {
-  const uint32_t waves = drvk::mlp_train_waves(batch, ctx->cu_count);
+int mlp_step(drv_ctx* ctx, const float* x, const float* y, const uint32_t* idx, uint32_t batch, float lr) {
+  const uint32_t groups = drvk::mlp_train_groups(batch, ctx->cu_count);
   int rc;
-  if ((rc = ensure(ctx, &ctx->mlp_partial, &ctx->mlp_partial_waves, static_cast<size_t>(waves) * (drvk::kMlpParams + 1))) !=
+  if ((rc = ensure(ctx, &ctx->mlp_partial, &ctx->mlp_partial_cap, static_cast<size_t>(groups) * (drvk::kMlpParams + 1))) !=
       DRV_OK)
     return rc;
-  drvk::launch_mlp_train(x, y, ctx->mlp_idx, batch, ctx->mlp_params, ctx->mlp_train_w, ctx->mlp_partial, waves,
-                         ctx->stream);
+  drvk::launch_mlp_train(x, y, idx, batch, ctx->mlp_params, ctx->mlp_pack, ctx->mlp_back, ctx->mlp_partial,
+                         groups, ctx->stream);
   float bc1 = 1.0f, bc2 = 1.0f;
   if (lr > 0.0f) {
     ctx->adam_t += 1;
     bc1 = 1.0f - static_cast<float>(std::pow(0.9, ctx->adam_t));
     bc2 = 1.0f - static_cast<float>(std::pow(0.999, ctx->adam_t));
   }
-  drvk::launch_mlp_adam(ctx->mlp_partial, waves, ctx->mlp_params, ctx->mlp_m, ctx->mlp_v, ctx->mlp_grad, lr, 0.9f,
+  drvk::launch_mlp_adam(ctx->mlp_partial, groups, ctx->mlp_params, ctx->mlp_m, ctx->mlp_v, ctx->mlp_grad, lr, 0.9f,
                         0.999f, 1e-8f, bc1, bc2, ctx->stream);
-  if (lr > 0.0f) drvk::launch_mlp_pack(ctx->mlp_params, ctx->mlp_pack, ctx->mlp_train_w, ctx->stream);
+  if (lr > 0.0f) drvk::launch_mlp_pack(ctx->mlp_params, ctx->mlp_pack, ctx->mlp_back, ctx->stream);
   return check_hip(ctx, hipGetLastError(), "mlp_step");
 }
 
@@ -1324,7 +1324,7 @@ int drv_mlp_set_params(drv_ctx* ctx, const float* host_params, uint32_t count) {
   DRV_HIP(ctx, hipMemcpyAsync(ctx->mlp_params, host_params, sizeof(float) * count, hipMemcpyHostToDevice, ctx->stream));
   drvk::launch_fill_u32(reinterpret_cast<uint32_t*>(ctx->mlp_m), drvk::kMlpParams, 0u, ctx->stream);
   drvk::launch_fill_u32(reinterpret_cast<uint32_t*>(ctx->mlp_v), drvk::kMlpParams, 0u, ctx->stream);
-  drvk::launch_mlp_pack(ctx->mlp_params, ctx->mlp_pack, ctx->mlp_train_w, ctx->stream);
+  drvk::launch_mlp_pack(ctx->mlp_params, ctx->mlp_pack, ctx->mlp_back, ctx->stream);
   DRV_HIP(ctx, hipStreamSynchronize(ctx->stream));
   ctx->adam_t = 0;
   ctx->mlp_ready = true;
@@ -1418,9 +1418,7 @@ int drv_mlp_gradient(drv_ctx* ctx, const float* x_dev, const float* y_dev, uint3
   if (!ctx || !x_dev || !y_dev || !grad_host || n == 0) return DRV_ERR_INVALID_ARG;
   int rc;
   if ((rc = require_net(ctx)) != DRV_OK) return rc;
-  if ((rc = ensure(ctx, &ctx->mlp_idx, &ctx->mlp_idx_cap, n)) != DRV_OK) return rc;
-  drvk::launch_mlp_batch_indices(n, n, 0u, ctx->mlp_idx, true, ctx->stream);
-  if ((rc = mlp_step(ctx, x_dev, y_dev, n, 0.0f)) != DRV_OK) return rc;
+  if ((rc = mlp_step(ctx, x_dev, y_dev, nullptr, n, 0.0f)) != DRV_OK) return rc;
   DRV_HIP(ctx, hipMemcpyAsync(grad_host, ctx->mlp_grad, sizeof(float) * (drvk::kMlpParams + 1), hipMemcpyDeviceToHost,
                               ctx->stream));
   DRV_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -1434,8 +1432,8 @@ int drv_mlp_train(drv_ctx* ctx, const float* x_dev, const float* y_dev, uint32_t
   if ((rc = require_net(ctx)) != DRV_OK) return rc;
   if ((rc = ensure(ctx, &ctx->mlp_idx, &ctx->mlp_idx_cap, batch)) != DRV_OK) return rc;
   for (uint32_t t = 0; t < steps; ++t) {
-    drvk::launch_mlp_batch_indices(n, batch, seed * 0x9e3779b1u + t, ctx->mlp_idx, false, ctx->stream);
-    if ((rc = mlp_step(ctx, x_dev, y_dev, batch, lr)) != DRV_OK) return rc;
+    drvk::launch_mlp_batch_indices(n, batch, seed * 0x9e3779b1u + t, ctx->mlp_idx, ctx->stream);
+    if ((rc = mlp_step(ctx, x_dev, y_dev, ctx->mlp_idx, batch, lr)) != DRV_OK) return rc;
   }
   if (mean_loss_host) {
     float loss = 0.0f;
@@ -1958,7 +1956,7 @@ int drv_batch_mlp_finetune(drv_batch* b, uint32_t n_samples, uint32_t batch, uin
     if (hipMemcpyAsync(ctx->mlp_params, owner->mlp_params, sizeof(float) * drvk::kMlpParams, hipMemcpyDeviceToDevice,
                        b->stream) != hipSuccess)
       return bfail(b, DRV_ERR_HIP, "batch_mlp_finetune: parameter copy failed");
-    drvk::launch_mlp_pack(ctx->mlp_params, ctx->mlp_pack, ctx->mlp_train_w, b->stream);
+    drvk::launch_mlp_pack(ctx->mlp_params, ctx->mlp_pack, ctx->mlp_back, b->stream);
     ctx->mlp_ready = true;
   }
   const hipError_t e = hipGetLastError();

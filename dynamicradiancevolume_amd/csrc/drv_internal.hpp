@@ -114,7 +114,7 @@ constexpr int kMlpW4 = 10432;
 constexpr int kMlpB4 = 10496;
 constexpr int kMlpParams = 10497;
 constexpr int kMlpPackBytes = 1280 * 16;       // inference A operands
-constexpr int kMlpTrainW = 64 * 40 + 4 * 64 * 72;  // bf16 LDS images for training
+constexpr int kMlpBackBytes = 1024 * 16;  // packed BF16 backward operands (W2, W3)
 
 // Inputs of the surrogate's feature extraction.
 struct FeatureArgsHost {
@@ -261,8 +261,7 @@ void launch_reduce_sh(const drv_sh_constants& shc, int sh_bands, float* caches, 
                       const float* partial, uint32_t partial_pitch, int grid, hipStream_t s);
 
 FeatureArgsHost make_feature_args(const drv_volume& vol, const float* cam, const VoxelView& vox);
-size_t mlp_train_lds_bytes();
-void launch_mlp_pack(const float* params, void* pack, void* train_w, hipStream_t s);
+void launch_mlp_pack(const float* params, void* pack, void* back, hipStream_t s);
 void launch_visibility_mlp(const FeatureArgsHost& fh, const void* pack, const float* params, const float* caches,
                            int stride, const Counter* counter, const Counter* first, const ShadowBlock* blocks,
                            uint32_t n_blocks, float* vis, uint32_t pitch, int grid, hipStream_t s);
@@ -273,11 +272,12 @@ void launch_mlp_features(const FeatureArgsHost& fh, const float* caches, int str
                          const float* vis, uint32_t pitch, float* y, hipStream_t s);
 void launch_mlp_forward(const void* pack, const float* params, const float* x, uint32_t n, float* p, int grid,
                         hipStream_t s);
-void launch_mlp_batch_indices(uint32_t n, uint32_t batch, uint32_t seed, uint32_t* idx, bool all, hipStream_t s);
-uint32_t mlp_train_waves(uint32_t batch, int cu_count);
+void launch_mlp_batch_indices(uint32_t n, uint32_t batch, uint32_t seed, uint32_t* idx, hipStream_t s);
+// partial: one gradient (kMlpParams + 1 floats) per workgroup.
+uint32_t mlp_train_groups(uint32_t batch, int cu_count);
 void launch_mlp_train(const float* x, const float* y, const uint32_t* idx, uint32_t batch, const float* params,
-                      const void* train_w, float* partial, uint32_t n_waves, hipStream_t s);
-void launch_mlp_adam(const float* partial, uint32_t n_waves, float* params, float* m, float* v, float* grad_out,
+                      const void* pack, const void* back, float* partial, uint32_t groups, hipStream_t s);
+void launch_mlp_adam(const float* partial, uint32_t rows, float* params, float* m, float* v, float* grad_out,
                      float lr, float beta1, float beta2, float eps, float bc1, float bc2, hipStream_t s);
 
 void launch_batch(BatchView* views, uint32_t n_views, BatchQueue* q, int stride, int sh_bands, int shadow,

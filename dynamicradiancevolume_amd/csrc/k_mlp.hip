@@ -14,11 +14,13 @@
 // layers.  The slot -> k assignment of the hardware is irrelevant: A and B
 // use the same one.
 //
-// Training (k_mlp_train) stages operands in LDS and runs the forward pass,
-// the backward pass and the weight-gradient GEMMs (K = samples) with the same
-// MFMA; every wave writes its partial gradient and k_mlp_adam reduces them in
-// a fixed order and applies Adam to the FP32 master weights.
+// Training (k_mlp_train) chains the forward and the backward layers the same
+// way; only the weight-gradient GEMMs (K = samples) need their operands
+// transposed, through LDS.  A workgroup sums its waves' gradients, and
+// k_mlp_adam reduces the workgroups' in a fixed order and applies Adam to the
+// FP32 master weights.
 #include <algorithm>
+#include <type_traits>
 
 #include "drv_internal.hpp"
 #include "k_common.hpp"
@@ -467,93 +469,78 @@ __global__ __launch_bounds__(64 * kInferWaves) void k_mlp_forward(const bf16x8* 
 // Hidden unit held in slot (kb, g, e) of a lane: 16(2kb + e/4) + 4g + e%4.
 __device__ __forceinline__ int slot_unit(int kb, int g, int e) { return 16 * (2 * kb + e / 4) + 4 * g + (e & 3); }
 
-// From the FP32 master parameters: (1) the inference A operands, (2) the
-// training LDS images W1T [64][40], W2T/W3T [64][72] ([out][in], padded), and
-// W2/W3 [64][72] ([in][out]).
-__global__ void k_mlp_pack(const float* params, bf16x8* pack, __bf16* train_w) {
+// From the FP32 master parameters: the forward A operands, W^T with K in slot
+// order (pack: W1, then (tile, kb) of W2 and W3), and the backward ones, W
+// itself with K = output units in slot order (back: (tile, kb) of W2 and W3).
+__global__ void k_mlp_pack(const float* params, bf16x8* pack, bf16x8* back) {
   const float* W1 = params + kMlpW1;
   const float* W2 = params + kMlpW2;
   const float* W3 = params + kMlpW3;
   const int tid = blockIdx.x * blockDim.x + threadIdx.x;
-  if (tid < 1280) {
-    const int lane = tid & 63;
-    const int row = lane & 15, g = lane >> 4;
-    bf16x8 v;
-    if (tid < 256) {
-      const int t = tid >> 6;
-      for (int e = 0; e < 8; ++e) v[e] = to_bf16(W1[(8 * g + e) * 64 + 16 * t + row]);
-    } else {
-      const int q = (tid - 256) >> 6;  // 0..15: layer 2 (0..7) or 3 (8..15)
-      const int layer = q >> 3, t = (q & 7) >> 1, kb = q & 1;
-      const float* W = layer == 0 ? W2 : W3;
-      for (int e = 0; e < 8; ++e) v[e] = to_bf16(W[slot_unit(kb, g, e) * 64 + 16 * t + row]);
-    }
+  if (tid >= 1280 + 1024) return;
+  const int lane = tid & 63;
+  const int row = lane & 15, g = lane >> 4;
+  bf16x8 v;
+  if (tid < 256) {
+    const int t = tid >> 6;
+    for (int e = 0; e < 8; ++e) v[e] = to_bf16(W1[(8 * g + e) * 64 + 16 * t + row]);
     pack[tid] = v;
+    return;
   }
-  // Training images.
-  for (int i = tid; i < kMlpTrainW; i += gridDim.x * blockDim.x) {
-    float v = 0.0f;
-    if (i < 64 * 40) {
-      const int o = i / 40, c = i % 40;
-      v = c < 32 ? W1[c * 64 + o] : 0.0f;
-    } else {
-      const int r = i - 64 * 40;
-      const int m = r / (64 * 72);  // 0: W2T, 1: W3T, 2: W2, 3: W3
-      const int rr = r % (64 * 72);
-      const int a = rr / 72, c = rr % 72;
-      if (c < 64) {
-        const float* W = (m == 0 || m == 2) ? W2 : W3;
-        v = (m < 2) ? W[c * 64 + a] : W[a * 64 + c];
-      }
-    }
-    train_w[i] = to_bf16(v);
+  const int q = ((tid - 256) >> 6) & 15;  // 0..15: layer 2 (0..7) or 3 (8..15)
+  const int layer = q >> 3, t = (q & 7) >> 1, kb = q & 1;
+  const float* W = layer == 0 ? W2 : W3;
+  if (tid < 1280) {
+    for (int e = 0; e < 8; ++e) v[e] = to_bf16(W[slot_unit(kb, g, e) * 64 + 16 * t + row]);
+    pack[tid] = v;
+  } else {
+    for (int e = 0; e < 8; ++e) v[e] = to_bf16(W[(16 * t + row) * 64 + slot_unit(kb, g, e)]);
+    back[tid - 1280] = v;
   }
 }
 
 // ---- training -----------------------------------------------------------------
 
-constexpr int kTrainChain = 32;  // samples per wave per chain
-constexpr int kTrainWaves = 2;   // waves per workgroup
-constexpr int LD32 = 40, LD64 = 72;
+constexpr int kTrainChain = 32;  // samples per wave per chain (two MFMA columns tiles)
+constexpr int kTrainWaves = 4;   // waves per workgroup, one per SIMD
+constexpr int LD32 = 40;         // padded row of 32 samples (16-byte reads of 16 rows spread over the banks)
+constexpr int LDW = 68;          // padded row of 64 weights in the gradient sum
 
 struct TrainLds {
-  __bf16 w1t[64 * LD32];
-  __bf16 w2t[64 * LD64];
-  __bf16 w3t[64 * LD64];
-  __bf16 w2[64 * LD64];
-  __bf16 w3[64 * LD64];
+  // Per wave, all [unit][sample]: what the weight-gradient GEMMs read.
   struct Wave {
-    __bf16 x[kTrainChain * LD32];    // [s][f]
-    __bf16 xt[32 * LD32];            // [f][s]
-    __bf16 h[3][kTrainChain * LD64];   // [s][u]
-    __bf16 ht[3][64 * LD32];           // [u][s]
-    __bf16 dz[kTrainChain * LD64];   // [s][u]
-    __bf16 dzt[64 * LD32];           // [u][s]
-    float y[kTrainChain];
-    float wgt[kTrainChain];
-    float dz4[kTrainChain];
+    __bf16 xt[32 * LD32];
+    __bf16 h1t[64 * LD32];
+    __bf16 h2t[64 * LD32];
+    __bf16 dzt[64 * LD32];
   } wv[kTrainWaves];
 };
+// A gradient in LDS, after the last chain: W1, W2, W3 as [in][LDW], then b1,
+// b2, b3, w4 (64 each), b4 and the loss.
+constexpr int kSumW2 = 32 * LDW, kSumW3 = kSumW2 + 64 * LDW, kSumB = kSumW3 + 64 * LDW, kSumEnd = kSumB + 260;
+// Two gradients at a time take the chains' memory.
+constexpr size_t kTrainLdsBytes = std::max(sizeof(TrainLds), 2 * kSumEnd * sizeof(float));
 
-// acc[mt][nt] += A[16mt.., :] . B[:, 16nt..] with A row-major [M][K] (lda)
-// and B given as B^T row-major [N][K] (ldbt), K = 32 * KB.
-template <int MT, int NT, int KB>
-__device__ __forceinline__ void wave_gemm(f32x4 (&acc)[MT][NT], const __bf16* A, int lda, const __bf16* Bt, int ldbt,
-                                          int lane) {
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// acc[mt][nt] += A[16mt.., :] . B[:, 16nt..] over 32 samples, A row-major
+// [M][32] and B given as B^T row-major [N][32], rows of LD32.
+template <int MT, int NT>
+__device__ __forceinline__ void grad_gemm(f32x4 (&acc)[MT][NT], const __bf16* A, const __bf16* Bt, int lane) {
   const int row = lane & 15, kg = (lane >> 4) * 8;
+  bf16x8 a[MT], b[NT];
 #pragma unroll
-  for (int kb = 0; kb < KB; ++kb) {
-    bf16x8 a[MT], b[NT];
+  for (int mt = 0; mt < MT; ++mt) a[mt] = *reinterpret_cast<const bf16x8*>(A + (16 * mt + row) * LD32 + kg);
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) a[mt] = *reinterpret_cast<const bf16x8*>(A + (16 * mt + row) * lda + 32 * kb + kg);
+  for (int nt = 0; nt < NT; ++nt) b[nt] = *reinterpret_cast<const bf16x8*>(Bt + (16 * nt + row) * LD32 + kg);
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-      b[nt] = *reinterpret_cast<const bf16x8*>(Bt + (16 * nt + row) * ldbt + 32 * kb + kg);
+  for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = mfma(a[mt], b[nt], acc[mt][nt]);
-  }
+    for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = mfma(a[mt], b[nt], acc[mt][nt]);
 }
 
 template <int MT, int NT>
@@ -564,41 +551,112 @@ __device__ __forceinline__ void zero(f32x4 (&acc)[MT][NT]) {
     for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 }
 
-// Writes relu(acc + bias) of a [64 units] x [32 samples] D tile set as
-// bf16 [s][u] and [u][s].
-__device__ __forceinline__ void store_hidden(const f32x4 (&acc)[4][2], const float* bias, __bf16* h, __bf16* ht,
-                                             int lane) {
-  const int j = lane & 15, g = lane >> 4;
+// Sum over the 16 lanes of a row, in every lane (DPP: neighbour, pair, then
+// the row's halves and the row mirrored).
+__device__ __forceinline__ float row_sum(float v) {
+  auto dpp = [](float x, auto ctrl) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), decltype(ctrl)::value,
+                                                                 0xf, 0xf, true));
+  };
+  v += dpp(v, std::integral_constant<int, 0xB1>());   // quad_perm 1,0,3,2
+  v += dpp(v, std::integral_constant<int, 0x4E>());   // quad_perm 2,3,0,1
+  v += dpp(v, std::integral_constant<int, 0x141>());  // row_half_mirror
+  v += dpp(v, std::integral_constant<int, 0x140>());  // row_mirror
+  return v;
+}
+
+__device__ __forceinline__ f32x4 load4(const float* p, int t, int g) {
+  return *reinterpret_cast<const f32x4*>(p + 16 * t + 4 * g);
+}
+
+// A chain's hidden layer: the lane's units 16t + 4g + r of samples 16nt + j
+// as the bf16 values v[t / 2][nt][4 (t % 2) + r], which are also the B operand
+// of the next layer.
+struct Hidden {
+  bf16x8 v[2][2];
+  __device__ __forceinline__ float at(int t, int nt, int r) const { return from_bf16(v[t >> 1][nt][4 * (t & 1) + r]); }
+  __device__ __forceinline__ void set(int t, int nt, int r, float x) { v[t >> 1][nt][4 * (t & 1) + r] = to_bf16(x); }
+};
+
+// The layer as [unit][sample] rows in LDS.
+__device__ __forceinline__ void store_rows(__bf16* rows, const Hidden& h, int j, int g) {
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
+  for (int t = 0; t < 4; ++t)
 #pragma unroll
-    for (int nt = 0; nt < 2; ++nt) {
-      const int s = 16 * nt + j;
-      bf16x4 v;
+    for (int nt = 0; nt < 2; ++nt)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int u = 16 * mt + 4 * g + r;
-        const __bf16 q = to_bf16(fmaxf(acc[mt][nt][r] + bias[u], 0.0f));
-        v[r] = q;
-        ht[u * LD32 + s] = q;
-      }
-      *reinterpret_cast<bf16x4*>(h + s * LD64 + 16 * mt + 4 * g) = v;
+      for (int r = 0; r < 4; ++r) rows[(16 * t + 4 * g + r) * LD32 + 16 * nt + j] = h.v[t >> 1][nt][4 * (t & 1) + r];
+}
+
+// acc[t][nt] += (packed 64x64 operand) . in
+__device__ __forceinline__ void layer64(f32x4 (&acc)[4][2], const bf16x8* w, const Hidden& in, int lane) {
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+      const bf16x8 a = w[(t * 2 + kb) * 64 + lane];
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt) acc[t][nt] = mfma(a, in.v[kb][nt], acc[t][nt]);
     }
 }
+
+__device__ __forceinline__ void bias_init(f32x4 (&acc)[4][2], const float* b, int g) {
+#pragma unroll
+  for (int t = 0; t < 4; ++t) acc[t][0] = acc[t][1] = load4(b, t, g);
+}
+
+__device__ __forceinline__ Hidden relu(const f32x4 (&acc)[4][2]) {
+  Hidden h;
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) h.set(t, nt, r, fmaxf(acc[t][nt][r], 0.0f));
+  return h;
+}
+
+// dZ = dH where the unit was positive, its bias gradient summed.
+__device__ __forceinline__ Hidden relu_back(const f32x4 (&dh)[4][2], const Hidden& h, f32x4 (&gb)[4]) {
+  Hidden d;
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float dz = h.at(t, nt, r) > 0.0f ? dh[t][nt][r] : 0.0f;
+        gb[t][r] += dz;
+        d.set(t, nt, r, dz);
+      }
+  return d;
+}
+
+// Four floats at a 4-byte aligned address (one 16-byte load).
+struct __attribute__((aligned(4))) Float4u {
+  float v[4];
+};
 
 struct TrainArgs {
   const float* x;        // [n][32]
   const float* y;        // [n]
-  const uint32_t* idx;   // minibatch sample indices [n_batch]
+  const uint32_t* idx;   // minibatch sample indices [n_batch], or null: samples 0 .. n_batch - 1
   uint32_t n_batch;
   const float* params;   // FP32 master
-  const __bf16* train_w; // packed LDS images
-  float* partial;        // [n_waves][kMlpParams + 1] (last: loss)
+  const bf16x8* pack;    // forward operands
+  const bf16x8* back;    // backward operands
+  float* partial;        // [workgroup][kMlpParams + 1] (last: loss)
   float inv_batch;
   uint32_t chains_per_wave;
 };
 
-__global__ __launch_bounds__(128) void k_mlp_train(TrainArgs a) {
+// One wave per SIMD with its gradient accumulators (160 registers) and the
+// chain's layers in registers; LDS holds only the transposed operands (18 KiB
+// per wave).  Bound by the latency of a chain's ten dependent stages (8.5 us a
+// chain, 15 us before and after).  The first version kept every layer and the
+// weights in 129 KiB of LDS per two waves, stored each layer in both orders
+// and wrote a gradient per wave: 104 against 32 us for 65536 samples.
+__global__ __launch_bounds__(64 * kTrainWaves, 1) void k_mlp_train(TrainArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
   TrainLds& L = *reinterpret_cast<TrainLds*>(smem);
   const int lane = static_cast<int>(threadIdx.x & 63u);
@@ -606,195 +664,216 @@ __global__ __launch_bounds__(128) void k_mlp_train(TrainArgs a) {
   const int j = lane & 15, g = lane >> 4;
   const uint32_t gwave = blockIdx.x * kTrainWaves + wid;
   const uint32_t n_waves = gridDim.x * kTrainWaves;
-  // weights -> LDS
-  {
-    const uint4* src = reinterpret_cast<const uint4*>(a.train_w);
-    uint4* dst = reinterpret_cast<uint4*>(L.w1t);
-    for (int i = threadIdx.x; i < kMlpTrainW / 8; i += blockDim.x) dst[i] = src[i];
-  }
-  __syncthreads();
   auto& W = L.wv[wid];
-  const float* b1 = a.params + kMlpB1;
-  const float* b2 = a.params + kMlpB2;
-  const float* b3 = a.params + kMlpB3;
-  const float* w4 = a.params + kMlpW4;
+  const bf16x8* w1 = a.pack;
+  const bf16x8* w2 = a.pack + 256;
+  const bf16x8* w3 = a.pack + 768;
+  f32x4 w4[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) w4[t] = load4(a.params + kMlpW4, t, g);
   const float b4 = a.params[kMlpB4];
   f32x4 gw1[4][2], gw2[4][4], gw3[4][4];
   zero(gw1);
   zero(gw2);
   zero(gw3);
-  float gb1[4][4], gb2[4][4];
+  f32x4 gb1[4], gb2[4], gb3[4], gw4[4];
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) gb1[mt][r] = gb2[mt][r] = 0.0f;
-  float gb3 = 0.0f, gw4 = 0.0f, gb4 = 0.0f, loss = 0.0f;
+  for (int t = 0; t < 4; ++t) gb1[t] = gb2[t] = gb3[t] = gw4[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  float gb4 = 0.0f, loss = 0.0f;
 
   for (uint32_t c = 0; c < a.chains_per_wave; ++c) {
     const uint32_t chain = gwave + c * n_waves;
-    // 1. samples -> LDS (lanes 0..31: one sample each)
-    if (lane < kTrainChain) {
-      const uint32_t bi = chain * kTrainChain + lane;
+    if (chain * kTrainChain >= a.n_batch) break;  // wave-uniform
+    // 1. The lane's samples 16nt + j, features 8g .. 8g + 7.
+    bf16x8 xb[2];
+    float yv[2], wv[2];
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) {
+      const uint32_t bi = chain * kTrainChain + 16 * nt + j;
       const bool ok = bi < a.n_batch;
-      const uint32_t si = ok ? a.idx[bi] : 0u;
-      for (int f = 0; f < 32; ++f) {
-        const __bf16 q = to_bf16(ok ? a.x[static_cast<size_t>(si) * 32 + f] : 0.0f);
-        W.x[lane * LD32 + f] = q;
-        W.xt[f * LD32 + lane] = q;
+      const uint32_t si = !ok ? 0u : a.idx ? a.idx[bi] : bi;
+      const Float4u* src = reinterpret_cast<const Float4u*>(a.x + static_cast<size_t>(si) * 32 + 8 * g);
+      const Float4u lo = src[0], hi = src[1];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        xb[nt][e] = to_bf16(ok ? lo.v[e] : 0.0f);
+        xb[nt][4 + e] = to_bf16(ok ? hi.v[e] : 0.0f);
       }
-      W.y[lane] = ok ? a.y[si] : 0.0f;
-      W.wgt[lane] = ok ? 1.0f : 0.0f;
+      yv[nt] = ok ? a.y[si] : 0.0f;
+      wv[nt] = ok ? 1.0f : 0.0f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) W.xt[(8 * g + e) * LD32 + 16 * nt + j] = xb[nt][e];
     }
-    __syncthreads();
-    // 2-4. forward
-    {
-      f32x4 acc[4][2];
-      zero(acc);
-      wave_gemm<4, 2, 1>(acc, L.w1t, LD32, W.x, LD32, lane);
-      store_hidden(acc, b1, W.h[0], W.ht[0], lane);
+    // 2-4. Forward.
+    f32x4 acc[4][2];
+    bias_init(acc, a.params + kMlpB1, g);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const bf16x8 w = w1[t * 64 + lane];
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt) acc[t][nt] = mfma(w, xb[nt], acc[t][nt]);
     }
-    __syncthreads();
-    {
-      f32x4 acc[4][2];
-      zero(acc);
-      wave_gemm<4, 2, 2>(acc, L.w2t, LD64, W.h[0], LD64, lane);
-      store_hidden(acc, b2, W.h[1], W.ht[1], lane);
-    }
-    __syncthreads();
-    {
-      f32x4 acc[4][2];
-      zero(acc);
-      wave_gemm<4, 2, 2>(acc, L.w3t, LD64, W.h[1], LD64, lane);
-      store_hidden(acc, b3, W.h[2], W.ht[2], lane);
-    }
-    __syncthreads();
-    // 5. output unit, loss, dz4: lane = (sample s = lane % 32, half = lane / 32)
-    {
-      const int s = lane & 31, half = lane >> 5;
+    const Hidden h1 = relu(acc);
+    store_rows(W.h1t, h1, j, g);
+    bias_init(acc, a.params + kMlpB2, g);
+    layer64(acc, w2, h1, lane);
+    const Hidden h2 = relu(acc);
+    store_rows(W.h2t, h2, j, g);
+    bias_init(acc, a.params + kMlpB3, g);
+    layer64(acc, w3, h2, lane);
+    const Hidden h3 = relu(acc);
+    // 5. Output unit, loss and dz4, the same in the sample's four lanes; dW4,
+    // db3 and dZ3 = (w4 dz4) * (h3 > 0).
+    Hidden dz;
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) {
       float z = 0.0f;
-      for (int u = 32 * half; u < 32 * half + 32; ++u) z = __builtin_fmaf(w4[u], from_bf16(W.h[2][s * LD64 + u]), z);
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) z = __builtin_fmaf(w4[t][r], h3.at(t, nt, r), z);
+      z += __shfl_xor(z, 16);
       z += __shfl_xor(z, 32);
       z += b4;
       const float p = 1.0f / (1.0f + __expf(-z));
-      if (half == 0) {
-        const float yv = W.y[s], wv = W.wgt[s];
+      const float d4 = wv[nt] * (p - yv[nt]) * a.inv_batch;
+      if (g == 0) {
         const float pc = fminf(fmaxf(p, 1e-7f), 1.0f - 1e-7f);
-        loss += -wv * (yv * __logf(pc) + (1.0f - yv) * __logf(1.0f - pc));
-        W.dz4[s] = wv * (p - yv) * a.inv_batch;
+        loss += -wv[nt] * (yv[nt] * __logf(pc) + (1.0f - yv[nt]) * __logf(1.0f - pc));
+        gb4 += d4;
       }
-    }
-    __syncthreads();
-    // 6. lane u: dW4, db3 and dZ3 = (w4 dz4) * (h3 > 0)
-    {
-      const int u = lane;
-      float acc4 = 0.0f, accb = 0.0f;
-      for (int s = 0; s < kTrainChain; ++s) {
-        const float d4 = W.dz4[s];
-        const float h = from_bf16(W.ht[2][u * LD32 + s]);
-        acc4 = __builtin_fmaf(d4, h, acc4);
-        const float dz = h > 0.0f ? w4[u] * d4 : 0.0f;
-        accb += dz;
-        const __bf16 q = to_bf16(dz);
-        W.dzt[u * LD32 + s] = q;
-        W.dz[s * LD64 + u] = q;
-      }
-      gw4 += acc4;
-      gb3 += accb;
-      if (lane == 0)
-        for (int s = 0; s < kTrainChain; ++s) gb4 += W.dz4[s];
-    }
-    __syncthreads();
-    // 7. dW3^T += dZ3^T . H2
-    wave_gemm<4, 4, 1>(gw3, W.dzt, LD32, W.ht[1], LD32, lane);
-    // 8. dH2^T = W3 . dZ3^T  ([in][out] x [out][s])
-    f32x4 dh[4][2];
-    zero(dh);
-    wave_gemm<4, 2, 2>(dh, L.w3, LD64, W.dz, LD64, lane);
-    __syncthreads();
-    // 9. dZ2 = dH2 * (h2 > 0), db2
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-      for (int nt = 0; nt < 2; ++nt) {
-        const int s = 16 * nt + j;
+      for (int t = 0; t < 4; ++t)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int u = 16 * mt + 4 * g + r;
-          const float dz = from_bf16(W.h[1][s * LD64 + u]) > 0.0f ? dh[mt][nt][r] : 0.0f;
-          gb2[mt][r] += dz;
-          const __bf16 q = to_bf16(dz);
-          W.dzt[u * LD32 + s] = q;
-          W.dz[s * LD64 + u] = q;
+          const float h = h3.at(t, nt, r);
+          gw4[t][r] = __builtin_fmaf(d4, h, gw4[t][r]);
+          const float d = h > 0.0f ? w4[t][r] * d4 : 0.0f;
+          gb3[t][r] += d;
+          dz.set(t, nt, r, d);
         }
-      }
-    __syncthreads();
-    // 10. dW2^T += dZ2^T . H1 ; 11. dH1^T = W2 . dZ2^T
-    wave_gemm<4, 4, 1>(gw2, W.dzt, LD32, W.ht[0], LD32, lane);
-    zero(dh);
-    wave_gemm<4, 2, 2>(dh, L.w2, LD64, W.dz, LD64, lane);
-    __syncthreads();
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-      for (int nt = 0; nt < 2; ++nt) {
-        const int s = 16 * nt + j;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int u = 16 * mt + 4 * g + r;
-          const float dz = from_bf16(W.h[0][s * LD64 + u]) > 0.0f ? dh[mt][nt][r] : 0.0f;
-          gb1[mt][r] += dz;
-          W.dzt[u * LD32 + s] = to_bf16(dz);
-        }
-      }
-    __syncthreads();
-    // 12. dW1^T += dZ1^T . X
-    wave_gemm<4, 2, 1>(gw1, W.dzt, LD32, W.xt, LD32, lane);
-    __syncthreads();
+    }
+    store_rows(W.dzt, dz, j, g);
+    wave_sync();
+    // 6. dW3^T += dZ3^T . H2, dH2^T = W3 . dZ3^T, dZ2
+    grad_gemm(gw3, W.dzt, W.h2t, lane);
+    zero(acc);
+    layer64(acc, a.back + 512, dz, lane);
+    dz = relu_back(acc, h2, gb2);
+    wave_sync();
+    store_rows(W.dzt, dz, j, g);
+    wave_sync();
+    // 7. dW2^T += dZ2^T . H1, dH1^T = W2 . dZ2^T, dZ1
+    grad_gemm(gw2, W.dzt, W.h1t, lane);
+    zero(acc);
+    layer64(acc, a.back, dz, lane);
+    dz = relu_back(acc, h1, gb1);
+    wave_sync();
+    store_rows(W.dzt, dz, j, g);
+    wave_sync();
+    // 8. dW1^T += dZ1^T . X
+    grad_gemm(gw1, W.dzt, W.xt, lane);
+    wave_sync();
   }
 
-  // Per-wave partial gradient in the parameter layout.
-  float* out = a.partial + static_cast<size_t>(gwave) * (kMlpParams + 1);
+  // The workgroup's sum, (w0 + w2) + (w1 + w3): a lane's places are the same
+  // in every wave, so waves 2 and 3 leave theirs in LDS, waves 0 and 1 add
+  // them to their registers, and so on; all threads then write it out in the
+  // parameter layout.
+  f32x4 tail = f32x4{gb4, loss, 0.0f, 0.0f};
+  for (int off = 1; off < 64; off <<= 1) {
+    tail[0] += __shfl_xor(tail[0], off);
+    tail[1] += __shfl_xor(tail[1], off);
+  }
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
+  for (int t = 0; t < 4; ++t)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int o = 16 * mt + 4 * g + r;
+      gb1[t][r] = row_sum(gb1[t][r]);
+      gb2[t][r] = row_sum(gb2[t][r]);
+      gb3[t][r] = row_sum(gb3[t][r]);
+      gw4[t][r] = row_sum(gw4[t][r]);
+    }
+  float* sum = reinterpret_cast<float*>(smem);
+  // f(place, four values) for all of the lane's values
+  auto each = [&](float* base, auto&& f) {
 #pragma unroll
-      for (int nt = 0; nt < 2; ++nt) out[kMlpW1 + (16 * nt + j) * 64 + o] = gw1[mt][nt][r];
+    for (int t = 0; t < 4; ++t) {
+      float* o = base + 16 * t + 4 * g;
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt) f(o + (16 * nt + j) * LDW, gw1[t][nt]);
 #pragma unroll
       for (int nt = 0; nt < 4; ++nt) {
-        out[kMlpW2 + (16 * nt + j) * 64 + o] = gw2[mt][nt][r];
-        out[kMlpW3 + (16 * nt + j) * 64 + o] = gw3[mt][nt][r];
-      }
-      // bias sums over the 16 sample lanes of this lane group
-      float v1 = gb1[mt][r], v2 = gb2[mt][r];
-      for (int off = 1; off < 16; off <<= 1) {
-        v1 += __shfl_xor(v1, off);
-        v2 += __shfl_xor(v2, off);
+        f(o + kSumW2 + (16 * nt + j) * LDW, gw2[t][nt]);
+        f(o + kSumW3 + (16 * nt + j) * LDW, gw3[t][nt]);
       }
       if (j == 0) {
-        out[kMlpB1 + o] = v1;
-        out[kMlpB2 + o] = v2;
+        f(o + kSumB, gb1[t]);
+        f(o + kSumB + 64, gb2[t]);
+        f(o + kSumB + 128, gb3[t]);
+        f(o + kSumB + 192, gw4[t]);
       }
     }
-  out[kMlpB3 + lane] = gb3;
-  out[kMlpW4 + lane] = gw4;
-  float lsum = loss;
-  for (int off = 1; off < 64; off <<= 1) lsum += __shfl_xor(lsum, off);
-  if (lane == 0) {
-    out[kMlpB4] = gb4;
-    out[kMlpParams] = lsum;
+    if (lane == 0) f(base + kSumB + 256, tail);
+  };
+  auto store = [](float* p, f32x4& v) { *reinterpret_cast<f32x4*>(p) = v; };
+  auto add = [](float* p, f32x4& v) { v += *reinterpret_cast<const f32x4*>(p); };
+  __syncthreads();
+  if (wid >= 2) each(sum + (wid - 2) * kSumEnd, store);
+  __syncthreads();
+  if (wid < 2) each(sum + wid * kSumEnd, add);
+  __syncthreads();
+  if (wid == 1) each(sum, store);
+  __syncthreads();
+  if (wid == 0) {
+    each(sum, add);
+    each(sum, store);
+  }
+  __syncthreads();
+  float* out = a.partial + static_cast<size_t>(blockIdx.x) * (kMlpParams + 1);
+  const int t0 = static_cast<int>(threadIdx.x);
+  for (int i = t0; i < 2048; i += 64 * kTrainWaves) out[kMlpW1 + i] = sum[(i >> 6) * LDW + (i & 63)];
+  for (int i = t0; i < 4096; i += 64 * kTrainWaves) {
+    out[kMlpW2 + i] = sum[kSumW2 + (i >> 6) * LDW + (i & 63)];
+    out[kMlpW3 + i] = sum[kSumW3 + (i >> 6) * LDW + (i & 63)];
+  }
+  if (t0 < 64) {
+    out[kMlpB1 + t0] = sum[kSumB + t0];
+    out[kMlpB2 + t0] = sum[kSumB + 64 + t0];
+    out[kMlpB3 + t0] = sum[kSumB + 128 + t0];
+    out[kMlpW4 + t0] = sum[kSumB + 192 + t0];
+  }
+  if (t0 == 0) {
+    out[kMlpB4] = sum[kSumB + 256];
+    out[kMlpParams] = sum[kSumB + 257];
   }
 }
 
-// Fixed-order reduction of the per-wave partials, then Adam on the FP32
+// Fixed-order reduction of the workgroups' partials, then Adam on the FP32
 // master weights (step t >= 1).  With lr = 0 only the gradient is produced.
-__global__ void k_mlp_adam(const float* partial, uint32_t n_waves, float* params, float* m, float* v, float* grad_out,
-                           float lr, float beta1, float beta2, float eps, float bc1, float bc2) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i > static_cast<uint32_t>(kMlpParams)) return;
+// A workgroup takes 64 parameters, its waves interleaved rows: one thread per
+// parameter summing all rows left 42 workgroups with a chain of up to 1024
+// loads each (242 us against 4 us with the 256 rows of 65536 samples).
+constexpr int kAdamWaves = 8;
+__global__ __launch_bounds__(64 * kAdamWaves) void k_mlp_adam(const float* partial, uint32_t rows, float* params,
+                                                             float* m, float* v, float* grad_out, float lr,
+                                                             float beta1, float beta2, float eps, float bc1,
+                                                             float bc2) {
+  __shared__ float part[kAdamWaves][64];
+  const uint32_t lane = threadIdx.x & 63u, wid = threadIdx.x >> 6;
+  const uint32_t i = blockIdx.x * 64u + lane;
+  const bool in = i <= static_cast<uint32_t>(kMlpParams);
+  float s = 0.0f;
+  if (in) {
+#pragma unroll 8
+    for (uint32_t w = wid; w < rows; w += kAdamWaves) s += partial[static_cast<size_t>(w) * (kMlpParams + 1) + i];
+  }
+  part[wid][lane] = s;
+  __syncthreads();
+  if (wid != 0u || !in) return;
   float gsum = 0.0f;
-  for (uint32_t w = 0; w < n_waves; ++w) gsum += partial[static_cast<size_t>(w) * (kMlpParams + 1) + i];
+#pragma unroll
+  for (int w = 0; w < kAdamWaves; ++w) gsum += part[w][lane];
   if (grad_out) grad_out[i] = gsum;
   if (i == static_cast<uint32_t>(kMlpParams) || lr == 0.0f) return;
   const float mi = beta1 * m[i] + (1.0f - beta1) * gsum;
@@ -808,10 +887,6 @@ __global__ void k_mlp_adam(const float* partial, uint32_t n_waves, float* params
 __global__ void k_mlp_batch_indices(uint32_t n, uint32_t batch, uint32_t seed, uint32_t* idx) {
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < batch; i += gridDim.x * blockDim.x)
     idx[i] = hash32(i * 0x9e3779b9u + seed * 0x85ebca6bu + 7u) % n;
-}
-
-__global__ void k_iota(uint32_t n, uint32_t* idx) {
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) idx[i] = i;
 }
 
 // ---- spot check ---------------------------------------------------------------
@@ -894,8 +969,6 @@ __global__ __launch_bounds__(256) void k_spot_error(const float* spot, uint32_t 
 
 }  // namespace
 
-size_t mlp_train_lds_bytes() { return sizeof(TrainLds); }
-
 void launch_spot_select(const Counter* counter, uint32_t k, const float* caches, int stride, float* spot,
                         uint32_t spot_cap, Counter* spot_ctr, hipStream_t s) {
   hipLaunchKernelGGL(k_spot_select, dim3((spot_cap + 255) / 256), dim3(256), 0, s, counter, k, caches, stride, spot,
@@ -931,9 +1004,9 @@ static FeatureCtx to_ctx(const FeatureArgsHost& h) {
   return c;
 }
 
-void launch_mlp_pack(const float* params, void* pack, void* train_w, hipStream_t s) {
-  hipLaunchKernelGGL(k_mlp_pack, dim3(64), dim3(256), 0, s, params, static_cast<bf16x8*>(pack),
-                     static_cast<__bf16*>(train_w));
+void launch_mlp_pack(const float* params, void* pack, void* back, hipStream_t s) {
+  hipLaunchKernelGGL(k_mlp_pack, dim3(9), dim3(256), 0, s, params, static_cast<bf16x8*>(pack),
+                     static_cast<bf16x8*>(back));
 }
 
 void launch_visibility_mlp(const FeatureArgsHost& fh, const void* pack, const float* params, const float* caches,
@@ -986,47 +1059,45 @@ void launch_mlp_forward(const void* pack, const float* params, const float* x, u
   hipLaunchKernelGGL(k_mlp_forward, dim3(grid), dim3(64 * kInferWaves), 0, s, static_cast<const bf16x8*>(pack), params, x, n, p);
 }
 
-void launch_mlp_batch_indices(uint32_t n, uint32_t batch, uint32_t seed, uint32_t* idx, bool all, hipStream_t s) {
+void launch_mlp_batch_indices(uint32_t n, uint32_t batch, uint32_t seed, uint32_t* idx, hipStream_t s) {
   const unsigned blocks = std::max(1u, std::min(4096u, (batch + 255u) / 256u));
-  if (all)
-    hipLaunchKernelGGL(k_iota, dim3(blocks), dim3(256), 0, s, batch, idx);
-  else
-    hipLaunchKernelGGL(k_mlp_batch_indices, dim3(blocks), dim3(256), 0, s, n, batch, seed, idx);
+  hipLaunchKernelGGL(k_mlp_batch_indices, dim3(blocks), dim3(256), 0, s, n, batch, seed, idx);
 }
 
-uint32_t mlp_train_waves(uint32_t batch, int cu_count) {
+// Workgroups of the training kernel: one chain per wave until every SIMD has
+// a wave, then more chains per wave.
+uint32_t mlp_train_groups(uint32_t batch, int cu_count) {
   const uint32_t chains = (batch + kTrainChain - 1) / kTrainChain;
-  const uint32_t max_waves = static_cast<uint32_t>(cu_count) * 2u * kTrainWaves;
-  const uint32_t waves = std::min(chains, max_waves);
-  return ((waves + kTrainWaves - 1) / kTrainWaves) * kTrainWaves;
+  return std::min((chains + kTrainWaves - 1) / kTrainWaves, static_cast<uint32_t>(cu_count));
 }
 
 void launch_mlp_train(const float* x, const float* y, const uint32_t* idx, uint32_t batch, const float* params,
-                      const void* train_w, float* partial, uint32_t n_waves, hipStream_t s) {
+                      const void* pack, const void* back, float* partial, uint32_t groups, hipStream_t s) {
   TrainArgs a;
   a.x = x;
   a.y = y;
   a.idx = idx;
   a.n_batch = batch;
   a.params = params;
-  a.train_w = static_cast<const __bf16*>(train_w);
+  a.pack = static_cast<const bf16x8*>(pack);
+  a.back = static_cast<const bf16x8*>(back);
   a.partial = partial;
   a.inv_batch = 1.0f / static_cast<float>(batch);
   const uint32_t chains = (batch + kTrainChain - 1) / kTrainChain;
-  a.chains_per_wave = (chains + n_waves - 1) / n_waves;
+  a.chains_per_wave = (chains + groups * kTrainWaves - 1) / (groups * kTrainWaves);
   static bool lds_raised = false;  // the training kernel needs more than 64 KiB of LDS
   if (!lds_raised) {
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_mlp_train), hipFuncAttributeMaxDynamicSharedMemorySize,
-                              static_cast<int>(sizeof(TrainLds)));
+                              static_cast<int>(kTrainLdsBytes));
     lds_raised = true;
   }
-  hipLaunchKernelGGL(k_mlp_train, dim3(n_waves / kTrainWaves), dim3(64 * kTrainWaves), sizeof(TrainLds), s, a);
+  hipLaunchKernelGGL(k_mlp_train, dim3(groups), dim3(64 * kTrainWaves), kTrainLdsBytes, s, a);
 }
 
-void launch_mlp_adam(const float* partial, uint32_t n_waves, float* params, float* m, float* v, float* grad_out,
+void launch_mlp_adam(const float* partial, uint32_t rows, float* params, float* m, float* v, float* grad_out,
                      float lr, float beta1, float beta2, float eps, float bc1, float bc2, hipStream_t s) {
-  hipLaunchKernelGGL(k_mlp_adam, dim3((kMlpParams + 1 + 255) / 256), dim3(256), 0, s, partial, n_waves, params, m, v,
-                     grad_out, lr, beta1, beta2, eps, bc1, bc2);
+  hipLaunchKernelGGL(k_mlp_adam, dim3((kMlpParams + 1 + 63) / 64), dim3(64 * kAdamWaves), 0, s, partial, rows, params,
+                     m, v, grad_out, lr, beta1, beta2, eps, bc1, bc2);
 }
 
 }  // namespace drvk

@@ -111,6 +111,35 @@ def test_mlp_gradient_matches_oracle(cornell):
         assert e <= 1e-2, (names[k], e)
 
 
+@pytest.mark.parametrize("n", [1, 31, 33, 129, 32773])
+def test_mlp_gradient_chain_and_workgroup_edges(cornell, n):
+    """One sample, chains of 32 cut short, workgroups with idle waves, and a
+    second chain in some waves only; the samples at a 4-byte aligned address.
+    Per tensor 1e-2 like the 3000-sample gradient (BF16 roundings of hidden
+    values that differ in the last FP32 bits), of the whole gradient's norm
+    where the tensor's own is tiny."""
+    from dynamicradiancevolume_amd.surrogate import OFFSETS, init_params
+    from oracle import mlp
+
+    announce(f"mlp gradient of {n} samples vs oracle")
+    r = _renderer(cornell)
+    params = init_params(13)
+    r.mlp_set_params(params)
+    rng = np.random.default_rng(n)
+    x = _random_features(n, n)
+    y = rng.uniform(0, 1, n).astype(np.float32)
+    buf = torch.zeros(32 * n + 1, device=DEV)
+    xd = buf[1:].view(n, 32)
+    xd.copy_(torch.from_numpy(x))
+    g = r.mlp_gradient(xd, torch.from_numpy(y).to(DEV))
+    loss, ref = mlp.loss_and_grad(params, x, y, bf16=True)
+    assert g[-1] == pytest.approx(loss, rel=1e-3)
+    bounds = list(OFFSETS.values()) + [mlp.N_PARAMS]
+    for lo, hi in zip(bounds[:-1], bounds[1:]):
+        scale = max(np.linalg.norm(ref[lo:hi]), 1e-2 * np.linalg.norm(ref))
+        assert np.linalg.norm(g[lo:hi] - ref[lo:hi]) <= 1e-2 * scale, (lo, n)
+
+
 def test_mlp_adam_step_matches_oracle(cornell):
     from dynamicradiancevolume_amd.surrogate import init_params
     from oracle import mlp
