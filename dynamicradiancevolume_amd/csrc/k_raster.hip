@@ -8,12 +8,12 @@
 // near plane in FP64, pixel centres are sampled, both windings are accepted,
 // a fragment with reverse-Z depth z in (0, 1] is kept, and of all fragments
 // of a pixel the one with the largest depth wins, the lowest triangle index
-// among equal depths.  On the GPU that is a two-pass visibility buffer: pass
-// 1 takes the 64-bit atomic max of the depth bits (non-negative doubles
-// order like their bit patterns), pass 2 the atomic min of the index among
-// the fragments that reached that depth; a resolve pass then shades each
-// pixel from its winning triangle.  One thread rasterizes a small triangle;
-// triangles with a large pixel box are listed and rasterized by a workgroup.
+// among equal depths.  Small windows (most RSMs) take a two-pass visibility
+// buffer: pass 1 takes the 64-bit atomic max of the depth bits (non-negative
+// doubles order like their bit patterns), pass 2 the atomic min of the index
+// among the fragments that reached that depth.  Larger ones are rasterized tile
+// by tile in registers.  A resolve pass then shades each pixel from its
+// winning triangle.
 #include <algorithm>
 
 #include "drv_internal.hpp"
@@ -85,10 +85,13 @@ struct RasterArgs {
   uint32_t* n_big;
 };
 
-// Triangles covering more pixel-box area than this are rasterized by a whole
-// workgroup instead of one thread (a ground plane's few large triangles would
-// otherwise serialize the pass).
-constexpr uint32_t kBigPixels = 512;
+// Triangles of a larger pixel box than this are listed and rasterized by a
+// wave each (a thread's loop over them holds up the other 63), above the second
+// bound by the workgroup.  256x256, 1.0M triangles of 3 box pixels: both passes
+// 174 us at 512 with a workgroup for each listed triangle, 54 us at 24 (8: 107,
+// 64: 59); nearly all of what is left is reading and projecting.
+constexpr uint32_t kBigPixels = 24;
+constexpr uint32_t kHugePixels = 4096;
 
 // Screen-space setup of one clipped triangle piece: pixel box and edge data.
 struct Setup {
@@ -124,10 +127,11 @@ __device__ __forceinline__ Setup setup_piece(const ScreenTri& q, int w, int h) {
 template <typename F>
 __device__ __forceinline__ void raster_piece(const Setup& st, int w, uint32_t start, uint32_t step, F&& f) {
   const ScreenTri& q = st.q;
-  const uint32_t npix = static_cast<uint32_t>(st.bw) * static_cast<uint32_t>(st.bh);
-  for (uint32_t k = start; k < npix; k += step) {
-    const int px = st.px0 + static_cast<int>(k % static_cast<uint32_t>(st.bw));
-    const int py = st.py0 + static_cast<int>(k / static_cast<uint32_t>(st.bw));
+  const int rows = static_cast<int>(step / static_cast<uint32_t>(st.bw)), cols = static_cast<int>(step % static_cast<uint32_t>(st.bw));
+  int px = st.px0 + static_cast<int>(start % static_cast<uint32_t>(st.bw));
+  int py = st.py0 + static_cast<int>(start / static_cast<uint32_t>(st.bw));
+  const int end_x = st.px0 + st.bw, end_y = st.py0 + st.bh;
+  for (; py < end_y; px += cols, py += rows + (px >= end_x ? 1 : 0), px -= px >= end_x ? st.bw : 0) {
     const double cy = py + 0.5, cx = px + 0.5;
     const double e0 = ((q.x[2] - q.x[1]) * (cy - q.y[1]) - (q.y[2] - q.y[1]) * (cx - q.x[1])) * st.inv;
     const double e1 = ((q.x[0] - q.x[2]) * (cy - q.y[2]) - (q.y[0] - q.y[2]) * (cx - q.x[2])) * st.inv;
@@ -139,38 +143,91 @@ __device__ __forceinline__ void raster_piece(const Setup& st, int w, uint32_t st
   }
 }
 
-// Small triangles: one thread each.  Large ones are listed (first pass) or
-// skipped (second pass) for the workgroup kernel.
+// The screen triangle of a triangle wholly in front of the near plane (the
+// operations project_clip performs for it).  Returns the vertices in front.
+__device__ __forceinline__ int project_front(const float* p, const double* vp, int w, int h, ScreenTri& out,
+                                             bool& degenerate) {
+  int front = 0;
+  degenerate = false;
+#pragma unroll
+  for (int v = 0; v < 3; ++v) {
+    double c[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      c[r] = vp[4 * r + 0] * p[3 * v + 0] + vp[4 * r + 1] * p[3 * v + 1] + vp[4 * r + 2] * p[3 * v + 2] +
+             vp[4 * r + 3];
+    front += c[3] - c[2] >= 0 ? 1 : 0;
+    degenerate = degenerate || c[3] <= 1e-12;
+    out.x[v] = (c[0] / c[3] * 0.5 + 0.5) * w;
+    out.y[v] = (c[1] / c[3] * 0.5 + 0.5) * h;
+    out.z[v] = c[2] / c[3];
+  }
+  return front;
+}
+
+// Small triangles: one thread each.  Large ones and those that reach behind
+// the near plane are listed (first pass) or skipped (second pass) for the
+// workgroup kernel, which clips them.
 template <typename F>
 __device__ __forceinline__ void raster_small(const RasterArgs& a, uint32_t t, bool list_big, F&& f) {
-  ScreenTri sc[2];
-  const int m = project_clip(a.positions + 9 * static_cast<size_t>(t), a.vp, a.w, a.h, sc);
-  Setup st[2];
-  bool big = false;
-  for (int s = 0; s < m; ++s) {
-    st[s] = setup_piece(sc[s], a.w, a.h);
-    if (st[s].ok && static_cast<uint32_t>(st[s].bw) * static_cast<uint32_t>(st[s].bh) > kBigPixels) big = true;
+  float p[9];
+#pragma unroll
+  for (int i = 0; i < 9; ++i) p[i] = a.positions[9 * static_cast<size_t>(t) + i];
+  ScreenTri sc;
+  bool degenerate;
+  const int front = project_front(p, a.vp, a.w, a.h, sc, degenerate);
+  if (front == 0) return;
+  bool list = front < 3;
+  if (!list && degenerate) return;
+  Setup st;
+  st.ok = false;
+  if (!list) {
+    st = setup_piece(sc, a.w, a.h);
+    list = st.ok && static_cast<uint32_t>(st.bw) * static_cast<uint32_t>(st.bh) > kBigPixels;
   }
-  if (big) {
+  if (list) {
     if (list_big) a.big[atomicAdd(a.n_big, 1u)] = t;
     return;
   }
-  for (int s = 0; s < m; ++s)
-    if (st[s].ok) raster_piece(st[s], a.w, 0u, 1u, f);
+  if (st.ok) raster_piece(st, a.w, 0u, 1u, f);
 }
 
-// Large triangles: workgroup-strided pixel loops, persistent over the list.
+// Large triangles: a wave each, the huge ones among them the workgroup.
 template <typename F>
 __device__ __forceinline__ void raster_big(const RasterArgs& a, F&& f) {
-  const uint32_t n = *a.n_big;
-  for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
-    const uint32_t t = a.big[i];
-    ScreenTri sc[2];
-    const int m = project_clip(a.positions + 9 * static_cast<size_t>(t), a.vp, a.w, a.h, sc);
-    for (int s = 0; s < m; ++s) {
-      const Setup st = setup_piece(sc[s], a.w, a.h);
-      if (st.ok) raster_piece(st, a.w, threadIdx.x, blockDim.x, [&](size_t px, double z) { f(t, px, z); });
+  __shared__ uint32_t huge[4];
+  const uint32_t n = *a.n_big, lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+  for (uint32_t i0 = 4u * blockIdx.x; i0 < n; i0 += 4u * gridDim.x) {
+    const uint32_t i = i0 + w;
+    uint32_t later = 0u;  // pieces
+    if (i < n) {
+      const uint32_t t = a.big[i];
+      ScreenTri sc[2];
+      const int m = project_clip(a.positions + 9 * static_cast<size_t>(t), a.vp, a.w, a.h, sc);
+      for (int s = 0; s < m; ++s) {
+        const Setup st = setup_piece(sc[s], a.w, a.h);
+        if (!st.ok) continue;
+        if (static_cast<uint64_t>(st.bw) * static_cast<uint64_t>(st.bh) > kHugePixels)
+          later |= 1u << s;
+        else
+          raster_piece(st, a.w, lane, 64u, [&](size_t px, double z) { f(t, px, z); });
+      }
     }
+    if (lane == 0u) huge[w] = later;
+    __syncthreads();
+    for (uint32_t k = 0; k < 4u; ++k) {
+      const uint32_t pieces = huge[k];
+      if (pieces == 0u) continue;
+      const uint32_t t = a.big[i0 + k];
+      ScreenTri sc[2];
+      const int m = project_clip(a.positions + 9 * static_cast<size_t>(t), a.vp, a.w, a.h, sc);
+      for (int s = 0; s < m; ++s) {
+        if (!(pieces >> s & 1u)) continue;
+        const Setup st = setup_piece(sc[s], a.w, a.h);
+        raster_piece(st, a.w, threadIdx.x, 256u, [&](size_t px, double z) { f(t, px, z); });
+      }
+    }
+    __syncthreads();
   }
 }
 
@@ -200,6 +257,400 @@ __global__ __launch_bounds__(256) void k_raster_id_big(RasterArgs a) {
   raster_big(a, [&](uint32_t t, size_t i, double z) {
     if (static_cast<unsigned long long>(__double_as_longlong(z)) == a.zbits[i]) atomicMin(&a.tri[i], t);
   });
+}
+
+// ---- the tiled raster ----------------------------------------------------
+//
+// For windows of many tiles.  Triangles are binned to the 16x16-pixel tiles
+// their pixel boxes touch (count, scan, fill); then one workgroup per tile
+// keeps the tile's pixels in registers, one pixel per lane (a wave owns 8x8),
+// and walks the tile's triangles, 256 at a time: every thread sets up one
+// triangle in LDS, then every wave tests those that may touch it.  A pixel
+// keeps the greatest FP64 depth and the lowest index at it, as the two passes
+// above find with atomics.  The triangle's thread settles for each wave by FP32
+// planes with an error margin whether all its pixels are outside or behind, the
+// wave then for its lanes; the FP64 test, with the operations of raster_piece,
+// runs when a lane is left.
+//
+// 1920x1080, 1.0M triangles in 2000 boxes (74M box pixels, 18 layers deep):
+// the two passes 1660 us, of it atomics and FP64 tests of hidden fragments;
+// count 47, near-plane pieces 11, scan 9, fill 8, tiles 129 us, bound by vector
+// instructions (60 % of the cycles issue one, four waves on a SIMD).
+
+constexpr int kTile = 16;
+constexpr uint32_t kTileSpan = 64;  // triangles that touch more tiles go to the records that every tile looks through
+constexpr int kTileGroups = 16;     // tiles of which a wave adds up the pairs before its atomics
+
+struct TileRecord {
+  uint32_t x, y;  // first | last << 16 tile
+  uint32_t tri;
+  uint32_t piece;  // 0, 1: piece of a triangle cut by the near plane; 2: not cut
+};
+constexpr uint32_t kRecordItem = 0x80000000u;  // an item of a tile's list: a triangle, or this and a record
+
+struct TilePair {
+  uint32_t item, tile, rank;  // rank: place in the tile's list
+};
+constexpr uint32_t kNoTile = 0xffffffffu;
+
+struct TileArgs {
+  RasterArgs r;
+  int tiles_x, tiles_y;
+  uint32_t capacity;    // pairs
+  uint32_t* head;       // {wide records, clipped triangles, pairs, records in lists}, then the counts
+  uint32_t* count;      // [tiles]
+  uint32_t* start;      // [tiles]
+  uint32_t* clip;       // [n_tri] triangles that reach behind the near plane
+  TilePair* pairs;      // [capacity]
+  uint32_t* lists;      // [capacity] items by tile
+  TileRecord* records;  // [2 n_tri] from the front the wide ones, which every tile looks at, from the back those in lists
+};
+
+__device__ __forceinline__ TileRecord tile_record(const Setup& st, uint32_t t, uint32_t piece) {
+  const uint32_t x0 = st.px0 / kTile, x1 = (st.px0 + st.bw - 1) / kTile;
+  const uint32_t y0 = st.py0 / kTile, y1 = (st.py0 + st.bh - 1) / kTile;
+  return TileRecord{x0 | (x1 << 16), y0 | (y1 << 16), t, piece};
+}
+
+// Tiles of a piece if they are few enough for the lists, else 0.
+__device__ __forceinline__ uint32_t list_tiles(const TileRecord& rec) {
+  const uint32_t nx = (rec.x >> 16) - (rec.x & 0xffffu) + 1u, ny = (rec.y >> 16) - (rec.y & 0xffffu) + 1u;
+  return nx > kTileSpan || ny > kTileSpan || nx * ny > kTileSpan ? 0u : nx * ny;
+}
+
+// Claimed pairs that stay unused because they pass the capacity.
+__device__ __forceinline__ void drop_pairs(const TileArgs& a, uint32_t base, uint32_t n) {
+  for (uint32_t i = base; i < a.capacity && i - base < n; ++i) a.pairs[i].tile = kNoTile;
+}
+
+// The pairs of the workgroup's triangles are spread over its threads again (a
+// thread that walked its own triangle's tiles held up its wave: 130 us, this
+// 47).  The neighbours in a mesh fall into the same tiles, so a wave adds up
+// its pairs of a tile before its atomics (125 us with an atomic for each), whose
+// results are the ranks that spare the fill a second round of them.
+__global__ __launch_bounds__(1024) void k_tile_count(TileArgs a) {
+  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t lane = __lane_id();
+  uint32_t tiles = 0;
+  TileRecord rec{};
+  bool big = false;
+  if (t < a.r.n_tri) {
+    float p[9];
+#pragma unroll
+    for (int i = 0; i < 9; ++i) p[i] = a.r.positions[9 * static_cast<size_t>(t) + i];
+    ScreenTri sc;
+    bool degenerate;
+    const int front = project_front(p, a.r.vp, a.r.w, a.r.h, sc, degenerate);
+    if (front == 1 || front == 2) {
+      a.clip[atomicAdd(&a.head[1], 1u)] = t;
+    } else if (front == 3 && !degenerate) {
+      const Setup st = setup_piece(sc, a.r.w, a.r.h);
+      if (st.ok) {
+        rec = tile_record(st, t, 2u);
+        tiles = list_tiles(rec);
+        big = tiles == 0u;
+      }
+    }
+  }
+  // Where the thread's pairs end in the workgroup's.
+  __shared__ uint32_t ends[1024], first_x[1024], first_y[1024], width[1024], wave_sum[16], group_base;
+  uint32_t upto = tiles;
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t u = __shfl_up(upto, o);
+    if (static_cast<int>(lane) >= o) upto += u;
+  }
+  const uint32_t w = threadIdx.x >> 6;
+  if (lane == 63u) wave_sum[w] = upto;
+  __syncthreads();
+  uint32_t sum = 0u;
+#pragma unroll
+  for (uint32_t k = 0; k < 16u; ++k) {
+    upto += k < w ? wave_sum[k] : 0u;
+    sum += wave_sum[k];
+  }
+  if (threadIdx.x == 0u && sum != 0u) group_base = atomicAdd(&a.head[2], sum);
+  ends[threadIdx.x] = upto;
+  first_x[threadIdx.x] = rec.x & 0xffffu;
+  first_y[threadIdx.x] = rec.y & 0xffffu;
+  width[threadIdx.x] = (rec.x >> 16) - (rec.x & 0xffffu) + 1u;
+  __syncthreads();
+  if (sum != 0u && (group_base > a.capacity || sum > a.capacity - group_base)) {
+    // Triangles whose pairs would pass the capacity are left to the records.
+    if (threadIdx.x == 0u) drop_pairs(a, group_base, sum);
+    big = big || tiles != 0u;
+    sum = 0u;
+  }
+  for (uint32_t i0 = 0; i0 < sum; i0 += 1024u) {
+    // Pair i: the first thread whose pairs end behind it, then its tile.
+    const uint32_t i = i0 + threadIdx.x;
+    const bool on = i < sum;
+    uint32_t owner = 0u;
+#pragma unroll
+    for (uint32_t step = 512u; step > 0u; step >>= 1) owner += on && ends[owner + step - 1u] <= i ? step : 0u;
+    const uint32_t nx = width[owner], q = i - (owner != 0u ? ends[owner - 1u] : 0u);
+    const uint32_t tile = (first_y[owner] + q / nx) * static_cast<uint32_t>(a.tiles_x) + first_x[owner] + q % nx;
+    uint64_t left = __ballot(on);
+    uint32_t leader = lane, rank = 0u, n = 1u;
+    for (int k = 0; k < kTileGroups && left != 0ull; ++k) {
+      const int first = __builtin_ctzll(left);
+      const uint32_t its = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(tile), first));
+      const uint64_t same = __ballot(on && tile == its);
+      if (on && tile == its) {
+        leader = static_cast<uint32_t>(first);
+        rank = static_cast<uint32_t>(__popcll(same & ((1ull << lane) - 1ull)));
+        n = static_cast<uint32_t>(__popcll(same));
+      }
+      left &= ~same;
+    }
+    uint32_t before = 0u;
+    if (on && leader == lane) before = atomicAdd(&a.count[tile], n);
+    before = __shfl(before, static_cast<int>(leader));
+    if (on) a.pairs[group_base + i] = TilePair{blockIdx.x * 1024u + owner, tile, before + rank};
+  }
+  if (big) a.records[atomicAdd(&a.head[0], 1u)] = rec;
+}
+
+// The pieces of triangles cut by the near plane.
+__global__ __launch_bounds__(256) void k_tile_clip(TileArgs a) {
+  const uint32_t n = a.head[1];
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+    const uint32_t t = a.clip[i];
+    ScreenTri sc[2];
+    const int m = project_clip(a.r.positions + 9 * static_cast<size_t>(t), a.r.vp, a.r.w, a.r.h, sc);
+    for (int k = 0; k < m; ++k) {
+      const Setup st = setup_piece(sc[k], a.r.w, a.r.h);
+      if (!st.ok) continue;
+      const TileRecord rec = tile_record(st, t, static_cast<uint32_t>(k));
+      const uint32_t tiles = list_tiles(rec);
+      uint32_t slot = tiles != 0u ? atomicAdd(&a.head[2], tiles) : 0u;
+      if (tiles == 0u || slot > a.capacity || tiles > a.capacity - slot) {
+        drop_pairs(a, slot, tiles);
+        a.records[atomicAdd(&a.head[0], 1u)] = rec;
+        continue;
+      }
+      const uint32_t r = 2u * a.r.n_tri - 1u - atomicAdd(&a.head[3], 1u);
+      a.records[r] = rec;
+      for (uint32_t y = rec.y & 0xffffu; y <= rec.y >> 16; ++y)
+        for (uint32_t x = rec.x & 0xffffu; x <= rec.x >> 16; ++x, ++slot) {
+          const uint32_t tile = y * static_cast<uint32_t>(a.tiles_x) + x;
+          a.pairs[slot] = TilePair{kRecordItem | r, tile, atomicAdd(&a.count[tile], 1u)};
+        }
+    }
+  }
+}
+
+// Where each tile's list begins: exclusive scan of the counts, one workgroup.
+__global__ __launch_bounds__(1024) void k_tile_scan(TileArgs a) {
+  __shared__ uint32_t wave_total[16];
+  const uint32_t n = static_cast<uint32_t>(a.tiles_x) * static_cast<uint32_t>(a.tiles_y);
+  const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+  uint32_t carry = 0;
+  for (uint32_t i0 = 0; i0 < n; i0 += 1024u) {
+    const uint32_t i = i0 + threadIdx.x;
+    const uint32_t c = i < n ? a.count[i] : 0u;
+    uint32_t s = c;
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t u = __shfl_up(s, o);
+      if (static_cast<int>(lane) >= o) s += u;
+    }
+    if (lane == 63u) wave_total[w] = s;
+    __syncthreads();
+    uint32_t before = carry, all = 0;
+    for (uint32_t k = 0; k < 16u; ++k) {
+      before += k < w ? wave_total[k] : 0u;
+      all += wave_total[k];
+    }
+    if (i < n) a.start[i] = before + s - c;
+    carry += all;
+    __syncthreads();
+  }
+}
+
+__global__ __launch_bounds__(256) void k_tile_fill(TileArgs a) {
+  const uint32_t n = min(a.head[2], a.capacity);
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+    const TilePair p = a.pairs[i];
+    if (p.tile != kNoTile) a.lists[a.start[p.tile] + p.rank] = p.item;
+  }
+}
+
+// A batch of triangles in LDS: what raster_piece reads, and FP32 planes
+// a X + b Y + c over the tile's pixel centres (X, Y from the tile's corner) of
+// the three edge functions and the depth, each raised above all rounding of
+// the plane and of the FP64 test: below zero, or a depth plane below the depth
+// held, is outside or behind for sure.  39 KB: four workgroups on a CU.
+struct TilePrim {
+  double x[3], y[3], z[3], inv;
+};
+struct TileBatch {
+  TilePrim prim[256];
+  float4 plane[3][256];
+  uint2 box_tri[256];   // columns | rows << 16 of the tile inside the pixel box; index
+  float zmax[4][256];   // above every depth in the wave's 8x8 pixels
+  uint8_t touch[256];   // bit per wave: may cover a pixel of it
+};
+
+// g bounds the terms that c and the FP64 test were summed from.
+__device__ __forceinline__ void tile_plane(float* out, double a, double b, double c, double g) {
+  const double m = 16.0 * (fabs(a) + fabs(b)) + fabs(c);
+  const double top = c + m * 0x1p-20 + g * 0x1p-40 + 1e-30;
+  const bool usable = m < 1e30 && g < 1e30;  // false also for NaN
+  out[0] = usable ? static_cast<float>(a) : 0.0f;
+  out[1] = usable ? static_cast<float>(b) : 0.0f;
+  out[2] = usable ? static_cast<float>(top) : 1e38f;
+}
+
+__device__ __forceinline__ float plane_at(float a, float b, float c, float x, float y) {
+  return __builtin_fmaf(a, x, __builtin_fmaf(b, y, c));
+}
+
+// Thread tid's triangle of the batch; the waves that it may touch.
+__device__ __forceinline__ uint32_t tile_prim(TileBatch& e, uint32_t tid, const ScreenTri& q, uint32_t t, int w, int h,
+                                              int ox, int oy) {
+  const Setup st = setup_piece(q, w, h);
+  if (!st.ok) return 0u;
+  const int x0 = max(st.px0 - ox, 0), x1 = min(st.px0 + st.bw - 1 - ox, kTile - 1);
+  const int y0 = max(st.py0 - oy, 0), y1 = min(st.py0 + st.bh - 1 - oy, kTile - 1);
+  if (x0 > x1 || y0 > y1) return 0u;
+  const double a0 = -(q.y[2] - q.y[1]) * st.inv, b0 = (q.x[2] - q.x[1]) * st.inv;
+  const double a1 = -(q.y[0] - q.y[2]) * st.inv, b1 = (q.x[0] - q.x[2]) * st.inv;
+  const double rx1 = ox - q.x[1], ry1 = oy - q.y[1], rx2 = ox - q.x[2], ry2 = oy - q.y[2];
+  const double c0 = b0 * ry1 + a0 * rx1, c1 = b1 * ry2 + a1 * rx2;
+  const double g0 = fabs(b0) * (fabs(ry1) + 16.0) + fabs(a0) * (fabs(rx1) + 16.0);
+  const double g1 = fabs(b1) * (fabs(ry2) + 16.0) + fabs(a1) * (fabs(rx2) + 16.0);
+  const double u = q.z[0] - q.z[2], v = q.z[1] - q.z[2];
+  const double zsum = fabs(q.z[0]) + fabs(q.z[1]) + fabs(q.z[2]);
+  float p[12];
+  tile_plane(p + 0, a0, b0, c0, g0);
+  tile_plane(p + 3, a1, b1, c1, g1);
+  tile_plane(p + 6, -(a0 + a1), -(b0 + b1), 1.0 - c0 - c1, 1.0 + g0 + g1);
+  tile_plane(p + 9, a0 * u + a1 * v, b0 * u + b1 * v, c0 * u + c1 * v + q.z[2], (1.0 + g0 + g1) * zsum);
+  const double top = fmax(fmax(q.z[0], q.z[1]), q.z[2]) + zsum * 0x1p-20 + 1e-30;
+  const float zmax = top < 1e30 ? static_cast<float>(top) : 1e38f;
+  uint32_t touch = 0u;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int kx = 8 * (k & 1), ky = 8 * (k >> 1);
+    // Each plane at the pixel centre of the 8x8 where it is greatest.
+    bool in = x0 < kx + 8 && x1 >= kx && y0 < ky + 8 && y1 >= ky;
+    float at[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      at[c] = plane_at(p[3 * c], p[3 * c + 1], p[3 * c + 2], static_cast<float>(kx) + (p[3 * c] > 0.0f ? 7.5f : 0.5f),
+                       static_cast<float>(ky) + (p[3 * c + 1] > 0.0f ? 7.5f : 0.5f));
+    in = in && !(at[0] < 0.0f) && !(at[1] < 0.0f) && !(at[2] < 0.0f) && !(at[3] < 0.0f);
+    touch |= in ? 1u << k : 0u;
+    e.zmax[k][tid] = fminf(zmax, at[3]);
+  }
+  TilePrim& d = e.prim[tid];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    d.x[k] = q.x[k];
+    d.y[k] = q.y[k];
+    d.z[k] = q.z[k];
+    e.plane[k][tid] = make_float4(p[4 * k], p[4 * k + 1], p[4 * k + 2], p[4 * k + 3]);
+  }
+  d.inv = st.inv;
+  e.box_tri[tid] = make_uint2((((2u << (x1 - x0)) - 1u) << x0) | ((((2u << (y1 - y0)) - 1u) << y0) << 16), t);
+  return touch;
+}
+
+__global__ __launch_bounds__(256, 4) void k_tile_raster(TileArgs a) {
+  __shared__ TileBatch e;
+  const int tile_x = static_cast<int>(blockIdx.x) % a.tiles_x, tile_y = static_cast<int>(blockIdx.x) / a.tiles_x;
+  const int ox = tile_x * kTile, oy = tile_y * kTile;
+  const uint32_t tid = threadIdx.x, lane = tid & 63u;
+  const uint32_t w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t lx = (lane & 7u) + 8u * (w & 1u), ly = (lane >> 3) + 8u * (w >> 1);
+  const int px = ox + static_cast<int>(lx), py = oy + static_cast<int>(ly);
+  const bool inside = px < a.r.w && py < a.r.h;
+  const double cx = px + 0.5, cy = py + 0.5;
+  const float fx = static_cast<float>(lx) + 0.5f, fy = static_cast<float>(ly) + 0.5f;
+  const uint32_t bit = (1u << lx) | (0x10000u << ly);
+  double z = 0.0;                      // a fragment must beat the cleared depth 0
+  float zlow = inside ? 0.0f : 1e38f;  // below z
+  uint32_t id = 0xffffffffu;
+
+  // First the wide records, then the tile's list.
+  const uint32_t n_wide = a.head[0], wide_span = (n_wide + 255u) & ~255u;
+  const uint32_t begin = a.start[blockIdx.x], n_list = a.count[blockIdx.x];
+  for (uint32_t i0 = 0; i0 < wide_span + n_list; i0 += 256u) {
+    const uint32_t i = i0 + tid;
+    uint32_t item = 0u, piece = 2u;
+    bool valid;
+    if (i0 < wide_span) {
+      valid = i < n_wide;
+      if (valid) {
+        const TileRecord rec = a.records[i];
+        const uint32_t tx = static_cast<uint32_t>(tile_x), ty = static_cast<uint32_t>(tile_y);
+        valid = tx >= (rec.x & 0xffffu) && tx <= (rec.x >> 16) && ty >= (rec.y & 0xffffu) && ty <= (rec.y >> 16);
+        item = rec.tri;
+        piece = rec.piece;
+      }
+      if (!__syncthreads_or(valid)) continue;
+    } else {
+      valid = i - wide_span < n_list;
+      if (valid) {
+        item = a.lists[begin + (i - wide_span)];
+        if (item & kRecordItem) {
+          const TileRecord rec = a.records[item & ~kRecordItem];
+          item = rec.tri;
+          piece = rec.piece;
+        }
+      }
+    }
+    uint32_t touch = 0u;
+    if (valid) {
+      ScreenTri q;
+      const float* pos = a.r.positions + 9 * static_cast<size_t>(item);
+      if (piece == 2u) {
+        float p[9];
+#pragma unroll
+        for (int k = 0; k < 9; ++k) p[k] = pos[k];
+        bool degenerate;
+        project_front(p, a.r.vp, a.r.w, a.r.h, q, degenerate);
+      } else {
+        ScreenTri sc[2];
+        project_clip(pos, a.r.vp, a.r.w, a.r.h, sc);
+        q = piece ? sc[1] : sc[0];
+      }
+      touch = tile_prim(e, tid, q, item, a.r.w, a.r.h, ox, oy);
+    }
+    e.touch[tid] = static_cast<uint8_t>(touch);
+    __syncthreads();
+    for (uint32_t k = 0; k < 256u; k += 64u) {
+      // The triangles that touch the wave's pixels and may lie before the farthest.
+      float far = zlow;
+      for (int o = 32; o > 0; o >>= 1) far = fminf(far, __shfl_xor(far, o));
+      uint64_t todo = __ballot((e.touch[k + lane] >> w & 1u) != 0u && !(e.zmax[w][k + lane] < far));
+      while (todo != 0ull) {
+        const uint32_t j = k + static_cast<uint32_t>(__builtin_ctzll(todo));
+        todo &= todo - 1ull;
+        const uint2 bt = e.box_tri[j];
+        const float4 p0 = e.plane[0][j], p1 = e.plane[1][j], p2 = e.plane[2][j];
+        const bool maybe = ((bt.x & bit) == bit) & !(plane_at(p0.x, p0.y, p0.z, fx, fy) < 0.0f) &
+                           !(plane_at(p0.w, p1.x, p1.y, fx, fy) < 0.0f) & !(plane_at(p1.z, p1.w, p2.x, fx, fy) < 0.0f) &
+                           !(plane_at(p2.y, p2.z, p2.w, fx, fy) < zlow);
+        if (__ballot(maybe) == 0ull) continue;
+        const TilePrim& q = e.prim[j];
+        const double e0 = ((q.x[2] - q.x[1]) * (cy - q.y[1]) - (q.y[2] - q.y[1]) * (cx - q.x[1])) * q.inv;
+        const double e1 = ((q.x[0] - q.x[2]) * (cy - q.y[2]) - (q.y[0] - q.y[2]) * (cx - q.x[2])) * q.inv;
+        const double e2 = 1.0 - e0 - e1;
+        const double f = e0 * q.z[0] + e1 * q.z[1] + e2 * q.z[2];
+        const bool hit = maybe && !(e0 < 0 || e1 < 0 || e2 < 0) && f > 0.0 && !(f > 1.0);
+        if (hit && (f > z || (f == z && bt.y < id))) {
+          z = f;
+          id = bt.y;
+          zlow = static_cast<float>(f) * (1.0f - 0x1p-20f);
+        }
+      }
+    }
+    __syncthreads();
+  }
+  if (!inside) return;
+  const size_t o = static_cast<size_t>(py) * a.r.w + px;
+  a.r.zbits[o] = static_cast<unsigned long long>(__double_as_longlong(z));
+  a.r.tri[o] = id;
 }
 
 // ---- formats (bit-exact restatements of the host producer's) ------------
@@ -363,8 +814,25 @@ __global__ __launch_bounds__(256) void k_rsm_downsample(int res, const uint16_t*
   }
 }
 
+// Windows of at least this many tiles take the tiled raster: a tile is one
+// workgroup's work, and a small window's few tiles hold many triangles each
+// and leave the chip idle.  1.0M triangles, tiled / two passes: 306 / 228 us at
+// 256x256 (256 tiles; an RSM 439 / 111), 238 / 424 at 480x270 (510), 191 / 684 at
+// 640x360, 259 / 1907 at 1920x1080; 2176 large triangles: 43 / 58, 47 / 65,
+// 54 / 74, 165 / 335.
+constexpr int kMinTiles = 384;
+
+int tile_count(int w, int h) { return ((w + kTile - 1) / kTile) * ((h + kTile - 1) / kTile); }
+// Tile coordinates have 12 bits, and the pairs of 2^24 triangles count in 32.
+bool tiled(int w, int h, uint32_t n_tri) {
+  return tile_count(w, h) >= kMinTiles && w <= 65536 && h <= 65536 && n_tri <= (1u << 24);
+}
+uint32_t pair_capacity(uint32_t n_tri) { return 4u * n_tri + 65536u; }
+
+// Depth and winning triangle of every pixel into zbits / tri; work: the
+// raster's lists (raster_work_words).
 void raster(const float* positions, uint32_t n_tri, const float* vp, int w, int h, unsigned long long* zbits,
-            uint32_t* tri, uint32_t* big, hipStream_t s) {
+            uint32_t* tri, uint32_t* work, hipStream_t s) {
   RasterArgs a;
   a.positions = positions;
   a.n_tri = n_tri;
@@ -373,14 +841,38 @@ void raster(const float* positions, uint32_t n_tri, const float* vp, int w, int 
   a.h = h;
   a.zbits = zbits;
   a.tri = tri;
-  a.n_big = big;      // big[0] counts, the list follows
-  a.big = big + 1;
+  a.n_big = work;  // work[0] counts, the list follows
+  a.big = work + 1;
+  const dim3 grid((n_tri + 255) / 256);
+  if (tiled(w, h, n_tri)) {
+    TileArgs t;
+    t.r = a;
+    t.tiles_x = (w + kTile - 1) / kTile;
+    t.tiles_y = (h + kTile - 1) / kTile;
+    const size_t tiles = static_cast<size_t>(t.tiles_x) * t.tiles_y, n = n_tri;
+    t.capacity = pair_capacity(n_tri);
+    t.records = reinterpret_cast<TileRecord*>(work);
+    t.head = work + 8 * n;
+    t.count = t.head + 4;
+    t.start = t.count + tiles;
+    t.clip = t.start + tiles;
+    t.lists = t.clip + n;
+    t.pairs = reinterpret_cast<TilePair*>(t.lists + t.capacity);
+    launch_fill_u32(t.head, 4 + tiles, 0u, s);
+    if (n_tri != 0) {
+      hipLaunchKernelGGL(k_tile_count, dim3((n_tri + 1023) / 1024), dim3(1024), 0, s, t);
+      hipLaunchKernelGGL(k_tile_clip, dim3(256), dim3(256), 0, s, t);
+    }
+    hipLaunchKernelGGL(k_tile_scan, dim3(1), dim3(1024), 0, s, t);
+    if (n_tri != 0) hipLaunchKernelGGL(k_tile_fill, dim3(1024), dim3(256), 0, s, t);
+    hipLaunchKernelGGL(k_tile_raster, dim3(static_cast<unsigned>(tiles)), dim3(256), 0, s, t);
+    return;
+  }
   const size_t n = static_cast<size_t>(w) * h;
   launch_fill_u32(reinterpret_cast<uint32_t*>(zbits), 2 * n, 0u, s);
   launch_fill_u32(tri, n, 0xffffffffu, s);
-  launch_fill_u32(big, 1, 0u, s);
+  launch_fill_u32(work, 1, 0u, s);
   if (n_tri == 0) return;
-  const dim3 grid((n_tri + 255) / 256);
   hipLaunchKernelGGL(k_raster_depth, grid, dim3(256), 0, s, a);
   hipLaunchKernelGGL(k_raster_depth_big, dim3(1024), dim3(256), 0, s, a);
   hipLaunchKernelGGL(k_raster_id, grid, dim3(256), 0, s, a);
@@ -389,10 +881,16 @@ void raster(const float* positions, uint32_t n_tri, const float* vp, int w, int 
 
 }  // namespace
 
+size_t raster_work_words(int w, int h, uint32_t n_tri) {
+  if (!tiled(w, h, n_tri)) return static_cast<size_t>(n_tri) + 1;
+  return 9 * static_cast<size_t>(n_tri) + 4 + 2 * static_cast<size_t>(tile_count(w, h)) +
+         4 * static_cast<size_t>(pair_capacity(n_tri));
+}
+
 void launch_render_gbuffer(const float* positions, const float* albedo, const float* normals, uint32_t n_tri,
                            const float* view_proj, int w, int h, unsigned long long* zbits, uint32_t* tri,
-                           uint32_t* big, float* depth, int16_t* normal, uint8_t* albedo_srgb, hipStream_t s) {
-  raster(positions, n_tri, view_proj, w, h, zbits, tri, big, s);
+                           uint32_t* work, float* depth, int16_t* normal, uint8_t* albedo_srgb, hipStream_t s) {
+  raster(positions, n_tri, view_proj, w, h, zbits, tri, work, s);
   GbufArgs a;
   a.w = w;
   a.h = h;
@@ -408,10 +906,10 @@ void launch_render_gbuffer(const float* positions, const float* albedo, const fl
 }
 
 void launch_render_rsm(const float* positions, const float* albedo, const float* normals, uint32_t n_tri,
-                       const drv_spot_light& light, unsigned long long* zbits, uint32_t* tri, uint32_t* big,
+                       const drv_spot_light& light, unsigned long long* zbits, uint32_t* tri, uint32_t* work,
                        uint16_t* flux, int16_t* normal, uint16_t* dls, float* shadow, hipStream_t s) {
   const int res = light.rsm_render_resolution;
-  raster(positions, n_tri, light.light_view_projection, res, res, zbits, tri, big, s);
+  raster(positions, n_tri, light.light_view_projection, res, res, zbits, tri, work, s);
   RsmArgs a;
   a.res = res;
   a.zbits = zbits;

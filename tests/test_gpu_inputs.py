@@ -113,3 +113,61 @@ def test_frame_from_device_inputs_matches_host_inputs():
     np.testing.assert_array_equal(e0[o0, :3], e1[o1, :3])
     assert rel_l2(entries_sh(e1[o1], w.sh_bands), entries_sh(e0[o0], w.sh_bands)) <= 1e-4
     assert rel_l2(out1.cpu().numpy(), out0.cpu().numpy()) <= 1e-4
+
+
+def _raster_scene(kind, n, w, h):
+    """Triangles [n, 3, 3] under clip = (x, y, 0.5, z): near plane at z = 0.5,
+    pixel (x / z + 1) / 2 * w."""
+    rng = np.random.default_rng(n * 7919 + w)
+    size = {"mesh": 0.05, "near": 1.5, "wide": 0.5, "ties": 0.3}[kind]
+    z = rng.uniform(0.6, 20.0, (n, 1))
+    if kind == "near":
+        z = rng.uniform(-1.0, 2.5, (n, 3))  # vertices before, on and behind the near plane
+        z[::7, 0] = 0.5
+    pos = np.empty((n, 3, 3))
+    pos[:, :, :2] = rng.uniform(-1.2, 1.2, (n, 1, 2)) + rng.uniform(-size, size, (n, 3, 2))
+    pos[:, :, 2] = z if kind == "near" else z + rng.uniform(0, 0.3, (n, 3))
+    pos[:, :, :2] *= np.maximum(pos[:, :, 2:], 0.25)
+    if kind == "ties":  # equal depths: the lowest index wins
+        pos[n // 2:] = pos[:n - n // 2][::-1]
+    pos[1] = pos[1, 0]  # no area
+    return np.ascontiguousarray(pos.astype(np.float32))
+
+
+# Windows on both sides of the tiled raster's least (384 tiles of 16x16), whole
+# and ragged tiles; triangles below and above the sizes at which one thread, a
+# wave or the workgroup takes them (24 and 4096 pixels) and past the 64 tiles
+# that the lists take; 6000 of some 23 tiles exceed the lists' capacity
+# (4 n + 65536 pairs).
+@pytest.mark.parametrize("kind,n,w,h", [
+    ("mesh", 1, 512, 256), ("mesh", 4000, 401, 300), ("mesh", 4000, 100, 37), ("near", 700, 401, 300),
+    ("near", 300, 130, 130), ("wide", 2, 1025, 481), ("wide", 6000, 400, 300), ("wide", 900, 255, 255),
+    ("ties", 1025, 512, 192), ("ties", 1025, 64, 64),
+])
+def test_raster_paths_match_host_producer(kind, n, w, h):
+    from dynamicradiancevolume_amd import _abi
+    from dynamicradiancevolume_amd.pipeline import Renderer
+
+    announce(f"raster {kind} {n} {w}x{h}")
+    pos = _raster_scene(kind, max(n, 2), w, h)[:n]
+    # The colour is the index, at the centres of the 8-bit sRGB steps.
+    code = np.stack([np.arange(n) % 251 + 1, np.arange(n) // 251 % 251 + 1, np.full(n, 7)], 1) / 255.0
+    albedo = np.where(code <= 0.04045, code / 12.92, ((code + 0.055) / 1.055) ** 2.4).astype(np.float32)
+    normals = np.tile(np.float32([0.0, 0.0, 1.0]), (n, 1))
+    vp = np.float32([1, 0, 0, 0, 0, 1, 0, 0, 0, 0, 0, 0.5, 0, 0, 1, 0])
+    depth = np.empty((h, w), np.float32)
+    gn = np.empty((h, w, 2), np.int16)
+    ga = np.empty((h, w, 3), np.uint8)
+    _abi.load_inputs().drvin_raster_gbuffer(pos.ctypes.data, albedo.ctypes.data, normals.ctypes.data, n,
+                                            vp.ctypes.data, w, h, depth.ctypes.data, gn.ctypes.data, ga.ctypes.data,
+                                            0)
+    cfg = frame_inputs("cornell_256").workload.config()
+    cfg.width, cfg.height = w, h
+    r = Renderer(cfg)
+    dev = [torch.from_numpy(x).cuda() for x in (pos, albedo, normals)]
+    scene = _abi.DrvScene(*(x.data_ptr() for x in dev), n)
+    for _ in range(2):
+        r.render_gbuffer(scene, vp)
+        got = r.read_gbuffer()
+        np.testing.assert_array_equal(got[0].view(np.uint32), depth.view(np.uint32))
+        np.testing.assert_array_equal(got[2], ga)
