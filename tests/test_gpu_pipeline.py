@@ -214,6 +214,44 @@ def test_voxelization_bit_exact(name, adapt):
         level += 1
 
 
+# Volumes without a whole 16^3 brick, of one brick and of slabs of one, two and
+# four bricks; one triangle (32 lanes share it), the smallest scene and one past
+# the last that shares lanes (2^19 of them); a blend over old voxels.
+@pytest.mark.parametrize("res,n_tri", [(2, 36), (8, 36), (16, 1), (32, 2176), (64, 8191), (128, 262145), (256, 2176)])
+def test_voxelization_sizes_bit_exact(res, n_tri):
+    orc = _orc()
+    fi = frame_inputs("cornell_256")
+    announce(f"voxelize {res} {n_tri}")
+    rng = np.random.default_rng(res)
+    src = fi.positions[np.arange(n_tri) % len(fi.positions)].reshape(n_tri, 3, 3)
+    centre = src.mean(1, keepdims=True)
+    # copies of the scene's triangles, smaller and moved beyond the first round
+    k = (np.arange(n_tri) >= len(fi.positions))[:, None, None]
+    pos = np.where(k, centre + 0.3 * (src - centre) + rng.uniform(-0.3, 0.3, (n_tri, 1, 3)), src)
+    pos = np.ascontiguousarray(pos.reshape(n_tri, 9).astype(np.float32))
+    moved = pos.copy()
+    moved[:, 1::3] += 0.4
+    r = _renderer(fi, voxel_resolution=res)
+    w = fi.workload.with_(voxel_resolution=res)
+    r.update_volume(w.eye, fi.bbox[:3], fi.bbox[3:])
+    vol = orc.update_volume(w.config(), w.eye, fi.bbox[:3], fi.bbox[3:])
+    mips = None
+    for p, adapt in ((pos, 1.0), (moved, 0.3), (pos, 0.6)):
+        dev = torch.from_numpy(p).cuda()
+        r.voxelize_scene(dev, n_tri, adaption_factor=adapt)
+        target, mips = orc.voxelize(res, vol, p, adaption_factor=adapt, previous=mips)
+        np.testing.assert_array_equal(r.read_voxels(-1), target)
+        for level in range(res.bit_length()):
+            np.testing.assert_array_equal(r.read_voxels(level), orc.mip_level(mips, res, level),
+                                          err_msg=f"mip level {level}")
+
+
+@pytest.mark.parametrize("res", [16, 32, 256])
+def test_gather_voxel_sizes_match_oracle(res):
+    announce(f"gather voxels {res}")
+    _gather_case("cornell_256", voxel_resolution=res)
+
+
 def test_voxel_blend_partial_adaption():
     """Two frames: the second voxelizes a moved scene with AdaptionFactor 0.25,
     so texels move a quarter step towards the new target."""
