@@ -58,6 +58,7 @@ struct drv_ctx {
   float4* phantoms = nullptr;        // allocation: positions of out-of-volume appends [max_caches]
   uint32_t* alloc_counts = nullptr;  // allocation: claimed cells per chunk, then of the last call [kAllocChunks + 1]
   uint32_t* alloc_claimed = nullptr; // allocation: CAV index of each claimed cell [cav_cells]
+  uint8_t* alloc_touched = nullptr;  // allocation: blocks of 64 cells that hold a claim (0 between calls)
   uint32_t* cav = nullptr;
   size_t cav_cells = 0;
   uint8_t* vox_target = nullptr;
@@ -429,6 +430,7 @@ int drv_create(const drv_config* config, drv_ctx** out_ctx) {
   ctx->cav_cells = static_cast<size_t>(c.cav_cascades) * c.cav_resolution * c.cav_resolution * c.cav_resolution;
   if ((rc = dev_alloc(ctx, &ctx->cav, ctx->cav_cells)) != DRV_OK) return bail(rc);
   if ((rc = dev_alloc(ctx, &ctx->alloc_claimed, ctx->cav_cells)) != DRV_OK) return bail(rc);
+  if ((rc = dev_alloc(ctx, &ctx->alloc_touched, drvk::alloc_touched_bytes(ctx->cav_cells))) != DRV_OK) return bail(rc);
 
   // Voxelization::SetResolution (voxelization.cpp:56-60): R8 target plus an
   // R8 volume with its full mip chain, plus the corner-expanded copy.
@@ -488,6 +490,7 @@ int drv_create(const drv_config* config, drv_ctx** out_ctx) {
   drvk::launch_fill_u32(reinterpret_cast<uint32_t*>(ctx->counter), sizeof(Counter) / 4, 0u, nullptr);
   drvk::launch_fill_u32(ctx->cav, ctx->cav_cells, 0u, nullptr);
   drvk::launch_fill_u32(ctx->alloc_counts, drvk::kAllocChunks + 1, 0u, nullptr);
+  drvk::launch_fill_u8(ctx->alloc_touched, drvk::alloc_touched_bytes(ctx->cav_cells), 0, nullptr);
   drvk::launch_fill_u8(ctx->vox_target, res3, 0, nullptr);
   drvk::launch_fill_u8(ctx->vox_mips, L.mip_bytes, 0, nullptr);
   drvk::launch_fill_u32(reinterpret_cast<uint32_t*>(ctx->vox_corners), L.corner_count * 4, 0u, nullptr);
@@ -523,6 +526,7 @@ int drv_destroy(drv_ctx* ctx) {
   dev_free(ctx->phantoms);
   dev_free(ctx->alloc_counts);
   dev_free(ctx->alloc_claimed);
+  dev_free(ctx->alloc_touched);
   dev_free(ctx->cav);
   dev_free(ctx->spec.atlas);
   dev_free(ctx->spec.vpls_lanes);
@@ -761,7 +765,7 @@ int drv_allocate_caches(drv_ctx* ctx, const drv_gbuffer* gb) {
   // renderer.cpp:969-970 (the clear of the counter and the address volume)
   // and cacheGather.comp, cachePrepareLighting.comp.
   drvk::launch_allocate(ctx->cfg, ctx->vol, ctx->frame, gb->depth, ctx->cav, ctx->caches, ctx->counter,
-                        ctx->phantoms, ctx->alloc_counts, ctx->alloc_claimed, ctx->stream);
+                        ctx->phantoms, ctx->alloc_counts, ctx->alloc_claimed, ctx->alloc_touched, ctx->stream);
   record(ctx, 4);
   ctx->allocated = true;
   ctx->spec_first = true;

@@ -210,11 +210,12 @@ void launch_fill_u8(uint8_t* p, size_t n, uint8_t v, hipStream_t s);
 // (count, assign: indices, entries, dispatch counter).  `counts` holds
 // kAllocChunks + 1 words (the last: claimed cells of the previous call,
 // zero with an all-zero CAV), `claimed` one word per CAV cell, `phantoms`
-// max_caches positions.
+// max_caches positions, `touched` a flag per 64 cells (zero at first; left zero).
 constexpr int kAllocChunks = 1024;
+inline size_t alloc_touched_bytes(size_t cells) { return ((cells + 63) / 64 + 3) & ~static_cast<size_t>(3); }
 void launch_allocate(const drv_config& cfg, const drv_volume& vol, const drv_frame& frame, const float* depth,
                      uint32_t* cav, float* caches, Counter* counter, float4* phantoms, uint32_t* counts,
-                     uint32_t* claimed, hipStream_t s);
+                     uint32_t* claimed, uint8_t* touched, hipStream_t s);
 
 void launch_voxelize(const drv_volume& vol, int res, const float* positions, const uint32_t* indices, uint32_t n_tri,
                      const float* world, uint8_t* target, hipStream_t s);

@@ -51,9 +51,9 @@ constexpr uint32_t kClaimedLeft = 0xFFFFFFFEu;  // claimed by the x = R corner o
 struct AllocArgs {
   drv_volume vol;
   float inv_vp[16];
-  float inv_size[DRV_MAX_CASCADES];  // 1 / world_voxel_size where that is a power of two (exact)
   const float* depth;
   uint32_t* cav;
+  uint8_t* touched;  // [block of 64 cells in numbering order] holds a claim; null: every block is read
   Counter* counter;
   float4* phantoms;  // positions of appended corners outside the CAV, [capacity]
   int width, height, R, C;
@@ -71,11 +71,11 @@ struct Cell {
 // (kPow2) the divisions are multiplications by the exact reciprocal: the
 // same correctly rounded quotient.
 template <bool kPow2>
-__device__ __forceinline__ Cell cell_of(const AllocArgs& a, f3 wp, int c) {
-  const drv_cascade& k = a.vol.cascades[c];
+__device__ __forceinline__ Cell cell_of(const AllocArgs& a, const drv_cascade& k, f3 wp, int c) {
   float qx, qy, qz;
   if (kPow2) {
-    const float s = a.inv_size[c];
+    // 2^-e of the size 2^e: the exponent field negated about its bias.
+    const float s = __builtin_bit_cast(float, (254u << 23) - __builtin_bit_cast(uint32_t, k.world_voxel_size));
     qx = (wp.x - k.min[0]) * s;
     qy = (wp.y - k.min[1]) * s;
     qz = (wp.z - k.min[2]) * s;
@@ -101,6 +101,27 @@ __device__ __forceinline__ float4 corner_position(const drv_volume& vol, int c, 
                      static_cast<float>(lz) * k.world_voxel_size + k.min[2], 0.0f);
 }
 
+// Bits of v at every third place.
+__device__ __forceinline__ uint32_t spread3(uint32_t v) {
+  v &= 0x000003FFu;
+  v = (v | (v << 16)) & 0x030000FFu;
+  v = (v | (v << 8)) & 0x0300F00Fu;
+  v = (v | (v << 4)) & 0x030C30C3u;
+  v = (v | (v << 2)) & 0x09249249u;
+  return v;
+}
+
+// The block of 64 cells, in numbering order (see cell_coord), that holds a cell.
+__device__ __forceinline__ uint32_t cell_block(int R, int c, int x, int y, int z) {
+  const uint32_t r = static_cast<uint32_t>(R), uc = static_cast<uint32_t>(c), ux = static_cast<uint32_t>(x),
+                 uy = static_cast<uint32_t>(y), uz = static_cast<uint32_t>(z);
+  if ((r & 3u) != 0u) return (uc * r * r * r + (uz * r + uy) * r + ux) >> 6;
+  const uint32_t nb = r >> 2, bx = ux >> 2, by = uy >> 2, bz = uz >> 2;
+  const uint32_t b = (nb & (nb - 1u)) == 0u ? spread3(bx) | (spread3(by) << 1) | (spread3(bz) << 2)
+                                            : (bz * nb + by) * nb + bx;
+  return uc * nb * nb * nb + b;
+}
+
 // AllocateCaches, cacheGather.comp:32-91, first half: the claims.  The
 // reference locks each of the 8 corner cells with a CAS and the winner
 // appends; the set of claimed cells and each cell's position do not depend
@@ -111,7 +132,8 @@ __device__ __forceinline__ float4 corner_position(const drv_volume& vol, int c, 
 // atomicAdd per wave, into the phantom list.  Called by every lane of the
 // wave (inactive lanes pass active = false) with the cell (bx, by, bz) of
 // cascade c.
-__device__ void mark_corners(const AllocArgs& a, bool active, int bx, int by, int bz, int c) {
+__device__ __forceinline__ void mark_corners(const AllocArgs& a, bool active, int bx, int by, int bz, int c) {
+  if (__ballot(active) == 0ull) return;  // three of a tile's four waves hold few leaders
   const int R = a.R;
   uint32_t outside = 0;
 #pragma unroll
@@ -120,9 +142,16 @@ __device__ void mark_corners(const AllocArgs& a, bool active, int bx, int by, in
     const int lx = bx + (i >> 2), ly = by + (i & 1), lz = bz + ((i >> 1) & 1);
     const int gx = lx + c * R;
     const bool inside = gx < a.C * R && ly < R && lz < R;  // the offsets are >= 0
-    if (active && inside) a.cav[(lz * R + ly) * (a.C * R) + gx] = lx == R ? kClaimedLeft : kClaimed;
+    if (active && inside) {
+      a.cav[(lz * R + ly) * (a.C * R) + gx] = lx == R ? kClaimedLeft : kClaimed;
+      // A corner whose block an earlier corner of the cell shares needs no flag.
+      const bool same = (R & 3) == 0 && ((lx != bx && (lx & 3) != 0) || (ly != by && (ly & 3) != 0) ||
+                                         (lz != bz && (lz & 3) != 0));
+      if (a.touched != nullptr && !same) a.touched[cell_block(R, lx == R ? c + 1 : c, lx == R ? 0 : lx, ly, lz)] = 1;
+    }
     if (active && !inside) outside |= 1u << i;
   }
+  if (__ballot(outside != 0u) == 0ull) return;
   uint64_t masks[8];
   uint32_t total = 0;
 #pragma unroll
@@ -146,7 +175,10 @@ __device__ void mark_corners(const AllocArgs& a, bool active, int bx, int by, in
   }
 }
 
-// 16x16 pixel tiles per pass-1 workgroup.
+// 16x16 pixel tiles per pass-1 workgroup (one: 4K 89 us, two: 79).  Bound by
+// instructions and the wait for the depths: 4K 97 us, 79 since waves without a
+// leader skip the marks and the cascade is found without branches; 1080p 26 and
+// 22 us.
 constexpr int kAllocTiles = 2;
 
 template <bool kPow2>
@@ -179,12 +211,13 @@ __global__ __launch_bounds__(256) void k_allocate(AllocArgs a) {
     if (d[h] > 0.0001f) {
       const f3 wp = unproject_pixel(a.inv_vp, a.width, a.height, x, y, d[h]);
       c[h] = cascade_of(a.vol, a.C, wp);
-      e[h] = cell_of<kPow2>(a, wp, c[h]);
+      const drv_cascade k = cascade_at(a.vol, c[h]);
+      e[h] = cell_of<kPow2>(a, k, wp, c[h]);
       own[h] = e[h].flat;
       if (a.transitions) {
-        const float tr = cascade_transition(a.vol, c[h], wp);
+        const float tr = cascade_transition(a.vol, k, wp);
         if (tr > 0.0f && c[h] < a.C - 1) {
-          e2[h] = cell_of<kPow2>(a, wp, c[h] + 1);
+          e2[h] = cell_of<kPow2>(a, cascade_at(a.vol, c[h] + 1), wp, c[h] + 1);
           own2[h] = e2[h].flat;
         }
       }
@@ -225,7 +258,10 @@ __global__ __launch_bounds__(256) void k_allocate(AllocArgs a) {
 // neighbours in space; the phantoms follow them.  Each workgroup numbers a
 // fixed chunk of that order: one launch counts the claims per chunk, the
 // next adds the counts of the chunks before (at most kAllocChunks of them)
-// and writes the indices, the entries and the dispatch counter.
+// and writes the indices, the entries and the dispatch counter.  Both read
+// only the blocks of 64 cells that pass 1 flagged (4 x 240^3 cells, 55k claims:
+// 85 and 92 us for a scan of all cells, 14 and 45; 4 x 96^3: 10 and 22, now 8 and
+// 22).
 
 struct AssignArgs {
   drv_volume vol;
@@ -235,8 +271,9 @@ struct AssignArgs {
   const float4* phantoms;
   uint32_t* counts;  // [gridDim.x] claims per chunk; [kAllocChunks] claimed cells of the last allocation
   uint32_t* claimed;  // flat CAV index of every claimed cell, by cache index
+  uint8_t* touched;
   int R, C, stride;
-  uint32_t n_cells, chunk, capacity;
+  uint32_t n_cells, n_blocks, chunk, capacity;  // chunk: blocks, a multiple of 4
 };
 
 // Logical cell L (cascade c, brick, cell in brick) -> cascade and local
@@ -307,13 +344,50 @@ __global__ __launch_bounds__(256) void k_allocate_clear(uint32_t* cav, const uin
   if (blockIdx.x == 0 && threadIdx.x < sizeof(Counter) / 4) reinterpret_cast<uint32_t*>(counter)[threadIdx.x] = 0u;
 }
 
-// Steps (256 cells each, 1024 with bricks) a workgroup loads ahead in the
-// count / assign scans.
+// Blocks whose flags a workgroup looks at together, and steps (256 cells each,
+// 1024 with bricks) it loads ahead.
+constexpr uint32_t kScanBlocks = 1024;
+constexpr uint32_t kChunkStep = 16;  // blocks, with bricks, in a step
 constexpr int kScanAhead = 4;
+
+// The flagged blocks among begin .. begin + kScanBlocks - 1 (below end), in
+// order, into list; returns how many.  Called by the whole workgroup.
+__device__ __forceinline__ uint32_t touched_blocks(const AssignArgs& a, uint32_t begin, uint32_t end, bool clear,
+                                                   uint32_t* list, uint32_t* wave_n) {
+  const uint32_t t = threadIdx.x, lane = t & 63u, w = t >> 6, b = begin + 4u * t;
+  if (a.touched == nullptr) return min(kScanBlocks, end - begin);
+  uint32_t f = 0u;
+  if (b < end) {  // chunks and the flags' allocation are multiples of 4
+    uint32_t* p = reinterpret_cast<uint32_t*>(a.touched + b);
+    f = *p;
+    if (clear && f != 0u) *p = 0u;
+  }
+  const uint32_t n = static_cast<uint32_t>(__popc(f));  // a flag is 0 or 1
+  uint32_t upto = n;
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t u = __shfl_up(upto, o);
+    if (static_cast<int>(lane) >= o) upto += u;
+  }
+  __syncthreads();  // the list and wave_n of the round before are read
+  if (lane == 63u) wave_n[w] = upto;
+  __syncthreads();
+  uint32_t at = upto - n;
+  for (uint32_t k = 0; k < w; ++k) at += wave_n[k];
+#pragma unroll
+  for (uint32_t k = 0; k < 4u; ++k)
+    if ((f >> (8u * k)) & 1u) list[at++] = b + k;
+  __syncthreads();
+  return (wave_n[0] + wave_n[1]) + (wave_n[2] + wave_n[3]);
+}
+
+__device__ __forceinline__ uint32_t block_cell(const AssignArgs& a, uint32_t begin, const uint32_t* list, uint32_t i) {
+  return (a.touched == nullptr ? begin + i : list[i]) * 64u;
+}
 
 // With bricks (R % 4 == 0) the 4 consecutive cells L .. L + 3 (L % 4 == 0)
 // are one brick row, 4 consecutive x at a 16-byte aligned CAV address: a
-// thread takes them with one load.  Chunks are multiples of 256 cells.
+// thread takes them with one load, 16 threads a block.  Else a wave takes a
+// block, one cell in each lane.
 __device__ __forceinline__ uint4 cav_row(const AssignArgs& a, uint32_t L, uint32_t& flat, CellCoord& k) {
   k = cell_coord(a, L);
   flat = cell_flat(a, k);
@@ -325,33 +399,35 @@ __device__ __forceinline__ uint32_t claims4(const uint4& v) {
 }
 
 __global__ __launch_bounds__(256) void k_allocate_count(AssignArgs a) {
-  __shared__ uint32_t part[4];
-  const uint32_t begin = blockIdx.x * a.chunk;
-  const uint32_t end = min(a.n_cells, begin + a.chunk);
+  __shared__ uint32_t part[4], list[kScanBlocks], wave_n[4];
+  const uint32_t begin = blockIdx.x * a.chunk, end = min(a.n_blocks, begin + a.chunk), t = threadIdx.x;
   uint32_t n = 0;
-  if ((a.R & 3) == 0) {
-    for (uint32_t L0 = begin + 4u * threadIdx.x; L0 < end; L0 += 1024u * kScanAhead) {
-      uint4 v[kScanAhead];
+  for (uint32_t b0 = begin; b0 < end; b0 += kScanBlocks) {
+    const uint32_t blocks = touched_blocks(a, b0, end, false, list, wave_n);
+    if ((a.R & 3) == 0) {
+      for (uint32_t i0 = t >> 4; i0 < blocks; i0 += 16u * kScanAhead) {
+        uint4 v[kScanAhead];
 #pragma unroll
-      for (int u = 0; u < kScanAhead; ++u) {
-        const uint32_t L = L0 + 1024u * u;
-        uint32_t flat;
-        CellCoord k;
-        v[u] = L < end ? cav_row(a, L, flat, k) : make_uint4(0u, 0u, 0u, 0u);
+        for (int u = 0; u < kScanAhead; ++u) {
+          const uint32_t i = i0 + 16u * u;
+          uint32_t flat;
+          CellCoord k;
+          v[u] = i < blocks ? cav_row(a, block_cell(a, b0, list, i) + 4u * (t & 15u), flat, k) : make_uint4(0u, 0u, 0u, 0u);
+        }
+#pragma unroll
+        for (int u = 0; u < kScanAhead; ++u) n += claims4(v[u]);
       }
+    } else {
+      for (uint32_t i0 = t >> 6; i0 < blocks; i0 += 4u * kScanAhead) {
+        uint32_t v[kScanAhead];
 #pragma unroll
-      for (int u = 0; u < kScanAhead; ++u) n += claims4(v[u]);
-    }
-  } else {
-    for (uint32_t L0 = begin + threadIdx.x; L0 < end; L0 += 256u * kScanAhead) {
-      uint32_t v[kScanAhead];
+        for (int u = 0; u < kScanAhead; ++u) {
+          const uint32_t i = i0 + 4u * u, L = i < blocks ? block_cell(a, b0, list, i) + (t & 63u) : a.n_cells;
+          v[u] = L < a.n_cells ? a.cav[cell_flat(a, cell_coord(a, L))] : 0u;
+        }
 #pragma unroll
-      for (int u = 0; u < kScanAhead; ++u) {
-        const uint32_t L = L0 + 256u * u;
-        v[u] = L < end ? a.cav[cell_flat(a, cell_coord(a, L))] : 0u;
+        for (int u = 0; u < kScanAhead; ++u) n += is_claim(v[u]);
       }
-#pragma unroll
-      for (int u = 0; u < kScanAhead; ++u) n += is_claim(v[u]);
     }
   }
   n = wave_sum(n);
@@ -378,6 +454,7 @@ __device__ __forceinline__ void assign_cell(const AssignArgs& a, const CellCoord
 __global__ __launch_bounds__(256) void k_allocate_assign(AssignArgs a) {
   __shared__ uint32_t part[2][4];
   __shared__ uint32_t wcnt[2][4];
+  __shared__ uint32_t list[kScanBlocks], wave_n[4];
   const uint32_t t = threadIdx.x, lane = t & 63u, w = t >> 6;
   // Claims before this chunk and in all chunks.
   uint32_t before = 0, all = 0;
@@ -412,86 +489,90 @@ __global__ __launch_bounds__(256) void k_allocate_assign(AssignArgs a) {
     a.counts[kAllocChunks] = n_claimed;  // the cells the next allocation clears
   }
   const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  const uint32_t begin = blockIdx.x * a.chunk;
-  const uint32_t end = min(a.n_cells, begin + a.chunk);
+  const uint32_t begin = blockIdx.x * a.chunk, end = min(a.n_blocks, begin + a.chunk);
   uint32_t step = 0;
-  if ((a.R & 3) == 0) {
-    // Bricks: a thread takes a brick row of 4 cells (one 16-byte load and,
-    // when it holds a claim, one 16-byte store of the new CAV values); cells
-    // are numbered in thread order, 1024 per step of the workgroup.
-    for (uint32_t L0 = begin; L0 < end; L0 += 1024u * kScanAhead) {
-      CellCoord k[kScanAhead];
-      uint32_t flat[kScanAhead];
-      uint4 v[kScanAhead];
+  for (uint32_t b0 = begin; b0 < end; b0 += kScanBlocks) {
+    const uint32_t blocks = touched_blocks(a, b0, end, true, list, wave_n);
+    if ((a.R & 3) == 0) {
+      // Bricks: a thread takes a brick row of 4 cells (one 16-byte load and,
+      // when it holds a claim, one 16-byte store of the new CAV values); cells
+      // are numbered in thread order, 16 blocks per step of the workgroup.
+      for (uint32_t i0 = 0; i0 < blocks; i0 += 16u * kScanAhead) {
+        CellCoord k[kScanAhead];
+        uint32_t flat[kScanAhead];
+        uint4 v[kScanAhead];
 #pragma unroll
-      for (int u = 0; u < kScanAhead; ++u) {
-        const uint32_t L = L0 + 1024u * u + 4u * t;
-        k[u] = CellCoord{};
-        flat[u] = 0u;
-        v[u] = make_uint4(0u, 0u, 0u, 0u);
-        if (L < end) v[u] = cav_row(a, L, flat[u], k[u]);
-      }
-#pragma unroll
-      for (int u = 0; u < kScanAhead; ++u, step ^= 1u) {
-        const uint32_t cv[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
-        uint64_t m[4];
-        uint32_t wave_n = 0, before_lane = 0;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          m[i] = __ballot(is_claim(cv[i]));
-          wave_n += static_cast<uint32_t>(__popcll(m[i]));
-          before_lane += static_cast<uint32_t>(__popcll(m[i] & lt_mask));
+        for (int u = 0; u < kScanAhead; ++u) {
+          const uint32_t i = i0 + 16u * u + (t >> 4);
+          k[u] = CellCoord{};
+          flat[u] = 0u;
+          v[u] = make_uint4(0u, 0u, 0u, 0u);
+          if (i < blocks) v[u] = cav_row(a, block_cell(a, b0, list, i) + 4u * (t & 15u), flat[u], k[u]);
         }
-        if (lane == 0) wcnt[step][w] = wave_n;
-        __syncthreads();  // wcnt[step] is rewritten two steps on, after the next barrier
-        uint32_t off = base + before_lane;
-        for (uint32_t j = 0; j < w; ++j) off += wcnt[step][j];
-        uint32_t nv[4] = {cv[0], cv[1], cv[2], cv[3]};
-        bool any = false;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          if (!is_claim(cv[i])) continue;
-          any = true;
-          CellCoord ki = k[u];
-          ki.x += i;
-          assign_cell(a, ki, cv[i], flat[u] + static_cast<uint32_t>(i), off);
-          nv[i] = off + 1u;  // cacheGather.comp:79
-          ++off;
-        }
-        if (any) *reinterpret_cast<uint4*>(a.cav + flat[u]) = make_uint4(nv[0], nv[1], nv[2], nv[3]);
-        base += (wcnt[step][0] + wcnt[step][1]) + (wcnt[step][2] + wcnt[step][3]);
-      }
-    }
-  } else {
-    for (uint32_t L0 = begin; L0 < end; L0 += 256u * kScanAhead) {
-      CellCoord k[kScanAhead];
-      uint32_t flat[kScanAhead], v[kScanAhead];
+        for (int u = 0; u < kScanAhead; ++u, step ^= 1u) {
+          if (i0 + 16u * u >= blocks) break;
+          const uint32_t cv[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+          uint64_t m[4];
+          uint32_t wave_claims = 0, before_lane = 0;
 #pragma unroll
-      for (int u = 0; u < kScanAhead; ++u) {
-        const uint32_t L = L0 + 256u * u + t;
-        k[u] = CellCoord{};
-        flat[u] = 0u;
-        v[u] = 0u;
-        if (L < end) {
-          k[u] = cell_coord(a, L);
-          flat[u] = cell_flat(a, k[u]);
-          v[u] = a.cav[flat[u]];
+          for (int i = 0; i < 4; ++i) {
+            m[i] = __ballot(is_claim(cv[i]));
+            wave_claims += static_cast<uint32_t>(__popcll(m[i]));
+            before_lane += static_cast<uint32_t>(__popcll(m[i] & lt_mask));
+          }
+          if (lane == 0) wcnt[step][w] = wave_claims;
+          __syncthreads();  // wcnt[step] is rewritten two steps on, after the next barrier
+          uint32_t off = base + before_lane;
+          for (uint32_t j = 0; j < w; ++j) off += wcnt[step][j];
+          uint32_t nv[4] = {cv[0], cv[1], cv[2], cv[3]};
+          bool any = false;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            if (!is_claim(cv[i])) continue;
+            any = true;
+            CellCoord ki = k[u];
+            ki.x += i;
+            assign_cell(a, ki, cv[i], flat[u] + static_cast<uint32_t>(i), off);
+            nv[i] = off + 1u;  // cacheGather.comp:79
+            ++off;
+          }
+          if (any) *reinterpret_cast<uint4*>(a.cav + flat[u]) = make_uint4(nv[0], nv[1], nv[2], nv[3]);
+          base += (wcnt[step][0] + wcnt[step][1]) + (wcnt[step][2] + wcnt[step][3]);
         }
       }
+    } else {
+      for (uint32_t i0 = 0; i0 < blocks; i0 += 4u * kScanAhead) {
+        CellCoord k[kScanAhead];
+        uint32_t flat[kScanAhead], v[kScanAhead];
 #pragma unroll
-      for (int u = 0; u < kScanAhead; ++u, step ^= 1u) {
-        const bool claim = is_claim(v[u]);  // 0 past the end
-        const uint64_t m = __ballot(claim);
-        if (lane == 0) wcnt[step][w] = static_cast<uint32_t>(__popcll(m));
-        __syncthreads();  // wcnt[step] is rewritten two steps on, after the next barrier
-        uint32_t off = base;
-        for (uint32_t j = 0; j < w; ++j) off += wcnt[step][j];
-        if (claim) {
-          const uint32_t idx = off + static_cast<uint32_t>(__popcll(m & lt_mask));
-          assign_cell(a, k[u], v[u], flat[u], idx);
-          a.cav[flat[u]] = idx + 1u;  // cacheGather.comp:79
+        for (int u = 0; u < kScanAhead; ++u) {
+          const uint32_t i = i0 + 4u * u + w, L = i < blocks ? block_cell(a, b0, list, i) + lane : a.n_cells;
+          k[u] = CellCoord{};
+          flat[u] = 0u;
+          v[u] = 0u;
+          if (L < a.n_cells) {
+            k[u] = cell_coord(a, L);
+            flat[u] = cell_flat(a, k[u]);
+            v[u] = a.cav[flat[u]];
+          }
         }
-        base += (wcnt[step][0] + wcnt[step][1]) + (wcnt[step][2] + wcnt[step][3]);
+#pragma unroll
+        for (int u = 0; u < kScanAhead; ++u, step ^= 1u) {
+          if (i0 + 4u * u >= blocks) break;
+          const bool claim = is_claim(v[u]);  // 0 past the end
+          const uint64_t m = __ballot(claim);
+          if (lane == 0) wcnt[step][w] = static_cast<uint32_t>(__popcll(m));
+          __syncthreads();  // wcnt[step] is rewritten two steps on, after the next barrier
+          uint32_t off = base;
+          for (uint32_t j = 0; j < w; ++j) off += wcnt[step][j];
+          if (claim) {
+            const uint32_t idx = off + static_cast<uint32_t>(__popcll(m & lt_mask));
+            assign_cell(a, k[u], v[u], flat[u], idx);
+            a.cav[flat[u]] = idx + 1u;  // cacheGather.comp:79
+          }
+          base += (wcnt[step][0] + wcnt[step][1]) + (wcnt[step][2] + wcnt[step][3]);
+        }
       }
     }
   }
@@ -521,13 +602,18 @@ void launch_fill_u8(uint8_t* p, size_t n, uint8_t v, hipStream_t s) {
 
 void launch_allocate(const drv_config& cfg, const drv_volume& vol, const drv_frame& frame, const float* depth,
                      uint32_t* cav, float* caches, Counter* counter, float4* phantoms, uint32_t* counts,
-                     uint32_t* claimed, hipStream_t s) {
+                     uint32_t* claimed, uint8_t* touched, hipStream_t s) {
   hipLaunchKernelGGL(k_allocate_clear, dim3(64), dim3(256), 0, s, cav, claimed, counts, counter);
   AllocArgs a;
   a.vol = vol;
   for (int i = 0; i < 16; ++i) a.inv_vp[i] = frame.inverse_view_projection[i];
   a.depth = depth;
   a.cav = cav;
+  // A volume that the chunks hold in one step each is read whole: the flags
+  // would only be another wait (4 x 32^3 cells, count: 2.7 and 3.8 us).
+  const uint64_t n_cells =
+      static_cast<uint64_t>(cfg.cav_cascades) * cfg.cav_resolution * cfg.cav_resolution * cfg.cav_resolution;
+  a.touched = n_cells <= 64u * kChunkStep * static_cast<uint64_t>(kAllocChunks) ? nullptr : touched;
   a.counter = counter;
   a.phantoms = phantoms;
   a.width = cfg.width;
@@ -537,16 +623,10 @@ void launch_allocate(const drv_config& cfg, const drv_volume& vol, const drv_fra
   a.capacity = static_cast<uint32_t>(cfg.max_caches);
   a.transitions = cfg.cav_transition_size > 0.0f ? 1 : 0;
   bool pow2 = true;
-  for (int c = 0; c < DRV_MAX_CASCADES; ++c) {
-    a.inv_size[c] = 0.0f;
-    if (c >= a.C) continue;
+  for (int c = 0; c < a.C; ++c) {
     int e = 0;
     const float m = std::frexp(vol.cascades[c].world_voxel_size, &e);  // size = m 2^e, m in [0.5, 1)
-    if (m == 0.5f && e > -120 && e < 120) {
-      a.inv_size[c] = std::ldexp(1.0f, 1 - e);
-    } else {
-      pow2 = false;
-    }
+    pow2 = pow2 && m == 0.5f && e > -120 && e < 120;
   }
   const int tiles_x = (cfg.width + 15) / 16;
   const dim3 grid((tiles_x + kAllocTiles - 1) / kAllocTiles, (cfg.height + 15) / 16);
@@ -567,12 +647,13 @@ void launch_allocate(const drv_config& cfg, const drv_volume& vol, const drv_fra
   b.R = cfg.cav_resolution;
   b.C = cfg.cav_cascades;
   b.stride = entry_stride(cfg.sh_bands);
-  b.n_cells = static_cast<uint32_t>(static_cast<uint64_t>(cfg.cav_cascades) * cfg.cav_resolution *
-                                    cfg.cav_resolution * cfg.cav_resolution);
+  b.n_cells = static_cast<uint32_t>(n_cells);
   b.capacity = static_cast<uint32_t>(cfg.max_caches);
-  const uint32_t chunks = std::min<uint32_t>((b.n_cells + 1023u) / 1024u, static_cast<uint32_t>(kAllocChunks));
-  b.chunk = ((b.n_cells + chunks - 1u) / chunks + 255u) & ~255u;
-  const uint32_t groups = (b.n_cells + b.chunk - 1u) / b.chunk;
+  b.touched = a.touched;
+  b.n_blocks = (b.n_cells + 63u) / 64u;
+  const uint32_t chunks = std::min<uint32_t>((b.n_blocks + kChunkStep - 1u) / kChunkStep, static_cast<uint32_t>(kAllocChunks));
+  b.chunk = ((b.n_blocks + chunks - 1u) / chunks + 3u) & ~3u;
+  const uint32_t groups = (b.n_blocks + b.chunk - 1u) / b.chunk;
   hipLaunchKernelGGL(k_allocate_count, dim3(groups), dim3(256), 0, s, b);
   hipLaunchKernelGGL(k_allocate_assign, dim3(groups), dim3(256), 0, s, b);
 }

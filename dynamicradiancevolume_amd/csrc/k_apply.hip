@@ -195,9 +195,9 @@ struct __attribute__((aligned(4))) CellPair {
 };
 
 template <bool kSpec>
-__device__ __forceinline__ void lighting(const ApplyArgs& a, bool active, f3 wp, f3 n, int c, const float* diffuse,
-                                         uint32_t live, const SpecPixel& sp, float* stage, float* out) {
-  const drv_cascade& k = a.vol.cascades[c];
+__device__ __forceinline__ void lighting(const ApplyArgs& a, bool active, f3 wp, f3 n, int c, const drv_cascade& k,
+                                         const float* diffuse, uint32_t live, const SpecPixel& sp, float* stage,
+                                         float* out) {
   const float acx = (wp.x - k.min[0]) / k.world_voxel_size;
   const float acy = (wp.y - k.min[1]) / k.world_voxel_size;
   const float acz = (wp.z - k.min[2]) / k.world_voxel_size;
@@ -349,6 +349,7 @@ __global__ __launch_bounds__(256) void k_apply(ApplyArgs a) {
   const uint32_t live = a.counter->live;
   const f3 wp = unproject_pixel(a.inv_vp, a.width, a.height, x, y, d);
   const int c = cascade_of(a.vol, a.C, wp);
+  const drv_cascade& k = a.vol.cascades[c];
   const f3 n = shading_normal(static_cast<int16_t>(nrm & 0xFFFFu), static_cast<int16_t>(nrm >> 16));
   float diffuse[3] = {lut[al0], lut[al1], lut[al2]};
   SpecPixel sp{};
@@ -389,13 +390,14 @@ __global__ __launch_bounds__(256) void k_apply(ApplyArgs a) {
   }
   float* st = stage[threadIdx.x >> 6];
   float col[3];
-  lighting<kSpec>(a, valid, wp, n, c, diffuse, live, sp, st, col);
+  lighting<kSpec>(a, valid, wp, n, c, k, diffuse, live, sp, st, col);
   if (a.transitions) {  // cacheApply.frag:172-185
-    const float t = valid ? cascade_transition(a.vol, c, wp) : 0.0f;
+    const float t = valid ? cascade_transition(a.vol, k, wp) : 0.0f;
     const bool two = t > 0.0f && c < a.C - 1;
     if (__ballot(two) != 0ull) {
       float col2[3];
-      lighting<kSpec>(a, two, wp, n, two ? c + 1 : c, diffuse, live, sp, st, col2);
+      const int c2 = two ? c + 1 : c;
+      lighting<kSpec>(a, two, wp, n, c2, a.vol.cascades[c2], diffuse, live, sp, st, col2);
       if (two) {
         col[0] = col[0] * (1.0f - t) + col2[0] * t;
         col[1] = col[1] * (1.0f - t) + col2[1] * t;

@@ -24,11 +24,12 @@ __device__ __forceinline__ f3 make3(float x, float y, float z) { return f3{x, y,
 
 // Saturating float -> int with NaN -> 0 (GLSL int() is undefined outside the
 // int range; this fixes one definition shared with the oracle).
+// The conversion instruction saturates and takes NaN to 0; a C cast may not
+// rely on that, and spelled out it is seven more instructions.
 __device__ __forceinline__ int to_int(float f) {
-  if (!(f == f)) return 0;
-  if (f >= 2147483647.0f) return 2147483647;
-  if (f <= -2147483648.0f) return -2147483647 - 1;
-  return static_cast<int>(f);
+  int i;
+  asm("v_cvt_i32_f32_e32 %0, %1" : "=v"(i) : "v"(f));
+  return i;
 }
 
 // `vec4(x, y, z, w) * M` with a row-major upload: out[r] = sum_c M[r][c] v[c],
@@ -56,21 +57,44 @@ __device__ __forceinline__ f3 unproject_pixel(const float* inv_vp, int w, int h,
   return make3(v[0] / v[3], v[1] / v[3], v[2] / v[3]);
 }
 
-// ComputeAddressVolumeCascade, shader/lightcache.glsl:109-122.
+// ComputeAddressVolumeCascade, shader/lightcache.glsl:109-122: the first cascade
+// whose decision box holds the point (no branch: its lanes would part).
 __device__ __forceinline__ int cascade_of(const drv_volume& vol, int n, f3 wp) {
-  int c = 0;
-  for (; c < n - 1; ++c) {
+  int found = n - 1;
+#pragma unroll
+  for (int c = DRV_MAX_CASCADES - 2; c >= 0; --c) {
     const drv_cascade& k = vol.cascades[c];
-    if (wp.x <= k.decision_max[0] && wp.y <= k.decision_max[1] && wp.z <= k.decision_max[2] &&
-        wp.x >= k.decision_min[0] && wp.y >= k.decision_min[1] && wp.z >= k.decision_min[2])
-      break;
+    const bool in = (c < n - 1) & (wp.x <= k.decision_max[0]) & (wp.y <= k.decision_max[1]) & (wp.z <= k.decision_max[2]) &
+                    (wp.x >= k.decision_min[0]) & (wp.y >= k.decision_min[1]) & (wp.z >= k.decision_min[2]);
+    found = in ? c : found;
   }
-  return c;
+  return found;
+}
+
+// The lane's cascade c of n, chosen out of scalar loads where a lookup by lane
+// would wait for a memory load of each member (the allocation; a kernel that is
+// bound by instructions is better off with the loads).  Most waves see one or
+// two cascades.
+__device__ __forceinline__ drv_cascade cascade_at(const drv_volume& vol, int c) {
+  drv_cascade k = vol.cascades[0];
+#pragma unroll
+  for (int i = 1; i < DRV_MAX_CASCADES; ++i) {
+    const bool me = c == i;
+    if (__ballot(me) == 0ull) continue;
+    const drv_cascade& s = vol.cascades[i];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      k.min[j] = me ? s.min[j] : k.min[j];
+      k.decision_min[j] = me ? s.decision_min[j] : k.decision_min[j];
+      k.decision_max[j] = me ? s.decision_max[j] : k.decision_max[j];
+    }
+    k.world_voxel_size = me ? s.world_voxel_size : k.world_voxel_size;
+  }
+  return k;
 }
 
 // ComputeAddressVolumeCascadeTransition, shader/lightcache.glsl:125-134.
-__device__ __forceinline__ float cascade_transition(const drv_volume& vol, int c, f3 wp) {
-  const drv_cascade& k = vol.cascades[c];
+__device__ __forceinline__ float cascade_transition(const drv_volume& vol, const drv_cascade& k, f3 wp) {
   const float a0 = k.decision_max[0] - wp.x, a1 = k.decision_max[1] - wp.y, a2 = k.decision_max[2] - wp.z;
   const float b0 = wp.x - k.decision_min[0], b1 = wp.y - k.decision_min[1], b2 = wp.z - k.decision_min[2];
   const float m = fminf(fminf(fminf(a0, a1), a2), fminf(fminf(b0, b1), b2));

@@ -106,6 +106,25 @@ def test_allocation_variants(overrides):
     _assert_alloc_equal(r, fi, cfg, orc)
 
 
+# Blocks of 64 cells: fewer cells than one, bricks in Morton and in row order,
+# rows that end inside a block, cascades that start inside one, and chunks of
+# more blocks than a workgroup looks at together (1024; 240^3 x 4 has 844).
+@pytest.mark.parametrize("cav,cascades", [(2, 1), (3, 4), (5, 3), (12, 4), (33, 4), (50, 2), (64, 3), (96, 4), (270, 4)])
+def test_allocation_block_sizes(cav, cascades):
+    orc = _orc()
+    fi = frame_inputs("cornell_256")
+    over = dict(cav_resolution=cav, cav_cascades=cascades, cascade0_world_size=0.6)
+    cfg = fi.workload.with_(**over).config()
+    df = _device(fi)
+    announce(f"allocate {cav}^3 x {cascades}")
+    r = _renderer(fi, **over)
+    r.set_frame(fi.frame())
+    r.update_volume(fi.workload.eye, fi.bbox[:3], fi.bbox[3:])
+    for _ in range(2):  # the second call starts from the first one's flags and claims
+        r.allocate_caches(df.gbuffer())
+        _assert_alloc_equal(r, fi, cfg, orc)
+
+
 def test_allocation_overflow_counts_and_clamps():
     """Capacity below the live count: demanded count is still exact, only
     `capacity` caches are stored, the claimed cell set is unchanged and apply
