@@ -6,7 +6,7 @@
 // blending into the HDR target.
 //
 // MI355X design: one lane per pixel over 16x16 pixel tiles (a 256-thread
-// workgroup), so the 8 corner cells of neighbouring pixels share CAV lines and
+// workgroup, 8x8 pixels in a wave), so the 8 corner cells of neighbouring pixels share CAV lines and
 // cache entries in L2.  Addresses that are unclaimed (CAV 0 -> 0xFFFFFFFF) or
 // past the live count read as zero, as robust buffer access does in GL.
 //
@@ -179,25 +179,70 @@ __device__ __forceinline__ void cache_irradiance(const ApplyArgs& a, const float
   irr[2] = fmaxf(v2, 0.0f);
 }
 
-// ComputeLightingFromCaches, cacheApply.frag:28-118.  The lanes of a wave
-// (16x4 pixels) mostly share their 8 caches (2.1 distinct addresses per
-// corner on a 1080p frame), and 8 x 7 per-lane 16-byte loads keep the
-// texture address and data units busy.  So per corner the wave's first two
-// distinct entries are fetched once - lanes 0-27 and 32-59 load one float
-// each, the 8 corners' loads in flight together - and staged in LDS, where
-// their lanes read them; lanes with a third or later address load their own
-// entry.  Per lane the arithmetic and its order are those of one fetch per
-// pixel.  Every lane of the wave must call this (the staging is
-// cooperative); `active` = false lanes add nothing.
 // Two neighbouring CAV cells (dword alignment suffices for the 8-byte load).
 struct __attribute__((aligned(4))) CellPair {
   uint32_t a, b;
 };
 
+// The caches at the 8 corners of cell (x0, ay, az) of the atlas, offsets x
+// fastest: (0,0,0),(1,0,0),(0,1,0),(1,1,0),(0,0,1),(1,0,1),(0,1,1),(1,1,1).
+// The two cells of a pair (x, x + 1) are neighbours in the CAV row, so each
+// pair is one 8-byte load when both lie in the row; texelFetch outside the CAV
+// reads 0 -> address 0xFFFFFFFF, as inactive lanes get.  A wave whose cells all
+// lie inside loads without branches, its four pairs in flight together.
+__device__ __forceinline__ void corner_caches(const ApplyArgs& a, bool active, int x0, int ay, int az,
+                                              uint32_t* addr) {
+  const int R = a.R, CR = a.C * a.R;
+  const bool in = x0 >= 0 && x0 + 1 < CR && ay >= 0 && ay + 1 < R && az >= 0 && az + 1 < R;
+  if (__ballot(active && !in) == 0ull) {
+    const uint32_t at = active ? static_cast<uint32_t>((az * R + ay) * CR + x0) : 0u;
+    CellPair q[4];
+#pragma unroll
+    for (int p = 0; p < 4; ++p)
+      q[p] = *reinterpret_cast<const CellPair*>(a.cav + at + static_cast<uint32_t>(((p >> 1) * R + (p & 1)) * CR));
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      addr[2 * p] = active ? q[p].a - 1u : 0xFFFFFFFFu;
+      addr[2 * p + 1] = active ? q[p].b - 1u : 0xFFFFFFFFu;
+    }
+    return;
+  }
+#pragma unroll
+  for (int p = 0; p < 4; ++p) {
+    const int y = ay + (p & 1), z = az + (p >> 1);
+    const bool row = active && y >= 0 && z >= 0 && y < R && z < R;
+    uint32_t v0 = 0u, v1 = 0u;
+    if (row) {
+      const uint32_t* r = a.cav + (static_cast<uint32_t>(z) * R + y) * CR;
+      if (x0 >= 0 && x0 < CR) v0 = r[x0];
+      if (x0 + 1 >= 0 && x0 + 1 < CR) v1 = r[x0 + 1];
+    }
+    addr[2 * p] = v0 - 1u;
+    addr[2 * p + 1] = v1 - 1u;
+  }
+}
+
+// ComputeLightingFromCaches, cacheApply.frag:28-118.  The lanes of a wave
+// (8x8 pixels) mostly share their 8 caches (2.1 distinct addresses per
+// corner on a 1080p frame), and 8 x 7 per-lane 16-byte loads keep the
+// texture address and data units busy.  So per corner the wave's first two
+// distinct entries are fetched once - lanes 0-27 and 32-59 load one float
+// each, the 8 corners' loads in flight together - and staged in LDS, where
+// their lanes read them; lanes with a third or later address load their own
+// entry, lanes without a cache (an unclaimed cell, one past the live caches)
+// read zeros.  Bound by vector instructions in large images (3840x2160: 175 us)
+// and by the chain of loads in small ones, so the loads stand outside of
+// branches: 320x180 19.5 -> 14.6 us, 256x256 14.1 -> 10.6, 1920x1080 52 -> 51 (66
+// with the sums on the matrix unit, 4x4x1 with an entry broadcast).  Per lane the
+// arithmetic and its order are those of one fetch per pixel.  Every lane of
+// the wave must call this (the staging is cooperative); `active` = false lanes
+// add nothing.  stage: 8 x 64 floats of the wave, then 32 zeros.
 template <bool kSpec>
 __device__ __forceinline__ void lighting(const ApplyArgs& a, bool active, f3 wp, f3 n, int c, const drv_cascade& k,
                                          const float* diffuse, uint32_t live, const SpecPixel& sp, float* stage,
                                          float* out) {
+  out[0] = out[1] = out[2] = 0.0f;
+  if (__ballot(active) == 0ull) return;
   const float acx = (wp.x - k.min[0]) / k.world_voxel_size;
   const float acy = (wp.y - k.min[1]) / k.world_voxel_size;
   const float acz = (wp.z - k.min[2]) / k.world_voxel_size;
@@ -206,34 +251,31 @@ __device__ __forceinline__ void lighting(const ApplyArgs& a, bool active, f3 wp,
   const float jx = 1.0f - ix, jy = 1.0f - iy, jz = 1.0f - iz;
   const float w[8] = {jx * jy * jz, ix * jy * jz, jx * iy * jz, ix * iy * jz,
                       jx * jy * iz, ix * jy * iz, jx * iy * iz, ix * iy * iz};
-  const int R = a.R, CR = a.C * a.R;
   uint32_t addr[8];
-  // Offsets x fastest: (0,0,0),(1,0,0),(0,1,0),(1,1,0),(0,0,1),(1,0,1),
-  // (0,1,1),(1,1,1).  The two cells of a pair (x, x + 1) are neighbours in
-  // the CAV row, so each pair is one 8-byte load (4-byte aligned) when both
-  // lie in the row; texelFetch outside the CAV reads 0 -> address 0xFFFFFFFF.
-  const int x0 = ax + R * c;
-#pragma unroll
-  for (int p = 0; p < 4; ++p) {
-    const int y = ay + (p & 1), z = az + (p >> 1);
-    const bool row = active && y >= 0 && z >= 0 && y < R && z < R;
-    uint32_t v0 = 0u, v1 = 0u;
-    if (row) {
-      const uint32_t* r = a.cav + (static_cast<uint32_t>(z) * R + y) * CR;
-      if (x0 >= 0 && x0 + 1 < CR) {
-        const CellPair q = *reinterpret_cast<const CellPair*>(r + x0);
-        v0 = q.a;
-        v1 = q.b;
-      } else {
-        if (x0 >= 0 && x0 < CR) v0 = r[x0];
-        if (x0 + 1 >= 0 && x0 + 1 < CR) v1 = r[x0 + 1];
-      }
-    }
-    addr[2 * p] = v0 - 1u;
-    addr[2 * p + 1] = v1 - 1u;
-  }
+  corner_caches(a, active, ax + a.R * c, ay, az, addr);
+  const uint32_t lane = __lane_id();
+  const uint32_t sub = lane & 31u;
   const int nq = a.sh2 ? 8 : 4;
-  float acc[3] = {0.0f, 0.0f, 0.0f};
+  const bool fetches = sub < static_cast<uint32_t>(4 * (nq - 1));  // entry floats 4 .. 4 nq - 1 are read
+  const float* entry = a.caches + 4u + sub;
+  uint32_t from[8];  // the entry's place in the stage (0: first address, 32: second), kOwn or kNone
+  constexpr uint32_t kOwn = 1u, kNone = 2u;
+  float part[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const bool ok = addr[i] < live;
+    const uint64_t pa = __ballot(ok);
+    const uint32_t ua = static_cast<uint32_t>(__builtin_amdgcn_readlane(
+        static_cast<int>(addr[i]), pa != 0ull ? static_cast<int>(__builtin_ctzll(pa)) : 0));
+    const bool in_a = addr[i] == ua;
+    const uint64_t pb = __ballot(ok && !in_a);
+    const uint32_t ub = static_cast<uint32_t>(__builtin_amdgcn_readlane(
+        static_cast<int>(addr[i]), pb != 0ull ? static_cast<int>(__builtin_ctzll(pb)) : 0));
+    from[i] = !ok ? kNone : in_a ? 0u : addr[i] == ub ? 32u : kOwn;
+    // Entries that nothing reads (no address, no such float) are entry 0's.
+    const uint32_t ea = pa != 0ull ? ua : 0u, eb = pb != 0ull ? ub : ea;
+    part[i] = entry[static_cast<size_t>(lane < 32u ? ea : eb) * static_cast<uint32_t>(fetches ? a.stride : 0)];
+  }
   float spec[3] = {0.0f, 0.0f, 0.0f};
   if (kSpec) {
 #pragma unroll
@@ -252,44 +294,24 @@ __device__ __forceinline__ void lighting(const ApplyArgs& a, bool active, f3 wp,
       }
     }
   }
-  // An address past the live caches (unclaimed cell, overflow) adds zero.
-  const uint32_t lane = __lane_id();
-  const uint32_t sub = lane & 31u;
-  const uint32_t nf = static_cast<uint32_t>(4 * (nq - 1));  // entry floats 4 .. 4 + nf - 1 are read
-  uint32_t from[8];  // 0: first address, 1: second, 2: own load, 3: none
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const bool ok = addr[i] < live;
-    uint64_t pend = __ballot(ok);
-    uint32_t ua = 0u, ub = 0u;
-    bool in_a = false, in_b = false, have = false;
-    if (pend != 0ull) {
-      ua = static_cast<uint32_t>(
-          __builtin_amdgcn_readlane(static_cast<int>(addr[i]), static_cast<int>(__builtin_ctzll(pend))));
-      in_a = ok && addr[i] == ua;
-      pend &= ~__ballot(in_a);
-      have = lane < 32u;
-    }
-    if (pend != 0ull) {
-      ub = static_cast<uint32_t>(
-          __builtin_amdgcn_readlane(static_cast<int>(addr[i]), static_cast<int>(__builtin_ctzll(pend))));
-      in_b = ok && !in_a && addr[i] == ub;
-      have = true;
-    }
-    from[i] = in_a ? 0u : in_b ? 1u : ok ? 2u : 3u;
-    const uint32_t u = lane < 32u ? ua : ub;
-    const bool load = have && sub < nf;
-    stage[i * 64 + lane] = load ? a.caches[static_cast<size_t>(u) * a.stride + 4u + sub] : 0.0f;
-  }
+  for (int i = 0; i < 8; ++i) stage[i * 64 + lane] = part[i];
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  float acc[3] = {0.0f, 0.0f, 0.0f};
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    if (from[i] == 3u) continue;
     // q[4..7] (the L2 bands) are loaded and read only with sh2.
+    const float4* st = reinterpret_cast<const float4*>(stage + (from[i] == kNone ? 512u : i * 64u + (from[i] & 32u)));
     float4 q[8];
-    if (from[i] == 2u) {
+#pragma unroll
+    for (int j = 1; j < 4; ++j) q[j] = st[j - 1];
+    if (a.sh2) {
+#pragma unroll
+      for (int j = 4; j < 8; ++j) q[j] = st[j - 1];
+    }
+    if (from[i] == kOwn) {
       const float4* e4 = reinterpret_cast<const float4*>(a.caches + static_cast<size_t>(addr[i]) * a.stride);
 #pragma unroll
       for (int j = 1; j < 4; ++j) q[j] = e4[j];
@@ -297,20 +319,13 @@ __device__ __forceinline__ void lighting(const ApplyArgs& a, bool active, f3 wp,
 #pragma unroll
         for (int j = 4; j < 8; ++j) q[j] = e4[j];
       }
-    } else {
-      const float4* st = reinterpret_cast<const float4*>(stage + i * 64 + 32 * from[i]);
-#pragma unroll
-      for (int j = 1; j < 4; ++j) q[j] = st[j - 1];
-      if (a.sh2) {
-#pragma unroll
-        for (int j = 4; j < 8; ++j) q[j] = st[j - 1];
-      }
     }
     float irr[3];
     cache_irradiance(a, q, n, irr);
-    acc[0] = __builtin_fmaf(irr[0], w[i], acc[0]);
-    acc[1] = __builtin_fmaf(irr[1], w[i], acc[1]);
-    acc[2] = __builtin_fmaf(irr[2], w[i], acc[2]);
+    const float wi = from[i] == kNone ? 0.0f : w[i];
+    acc[0] = __builtin_fmaf(irr[0], wi, acc[0]);
+    acc[1] = __builtin_fmaf(irr[1], wi, acc[1]);
+    acc[2] = __builtin_fmaf(irr[2], wi, acc[2]);
   }
   __builtin_amdgcn_wave_barrier();  // the stage is rewritten by the next call
   out[0] = acc[0] * diffuse[0] * kInvPi;
@@ -328,10 +343,12 @@ __device__ __forceinline__ void lighting(const ApplyArgs& a, bool active, f3 wp,
 template <bool kSpec>
 __global__ __launch_bounds__(256) void k_apply(ApplyArgs a) {
   __shared__ float lut[256];
-  __shared__ __align__(16) float stage[4][8 * 64];  // per wave: the shared entries of each corner
+  __shared__ __align__(16) float stage[4][8 * 64 + 32];  // per wave: the shared entries of each corner, zeros
   lut[threadIdx.x] = a.srgb_lut[threadIdx.x];
-  const int x = blockIdx.x * 16 + (threadIdx.x & 15);
-  const int y = blockIdx.y * 16 + (threadIdx.x >> 4);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (lane < 32) stage[wave][8 * 64 + lane] = 0.0f;
+  const int x = blockIdx.x * 16 + 8 * (wave & 1) + (lane & 7);
+  const int y = blockIdx.y * 16 + 8 * (wave >> 1) + (lane >> 3);
   const bool inside = x < a.width && y < a.height;
   const size_t p = inside ? static_cast<size_t>(y) * a.width + x : 0;
   const float d = a.depth[p];
@@ -388,7 +405,7 @@ __global__ __launch_bounds__(256) void k_apply(ApplyArgs a) {
       sp.two = true;
     }
   }
-  float* st = stage[threadIdx.x >> 6];
+  float* st = stage[wave];
   float col[3];
   lighting<kSpec>(a, valid, wp, n, c, k, diffuse, live, sp, st, col);
   if (a.transitions) {  // cacheApply.frag:172-185

@@ -164,6 +164,38 @@ def test_allocation_overflow_counts_and_clamps():
     assert rel_l2(df.out.cpu().numpy(), ref) < RGB_TOL
 
 
+# Waves with cells at the volume's faces (a cascade that ends inside the view;
+# one cell, whose pairs lie outside), three and more caches at a corner (fine
+# cells), windows that end inside a wave's 8x8 pixels.
+@pytest.mark.parametrize("cav,cascades,size,width,height,sh", [
+    (1, 1, 12.0, 64, 48, 2), (1, 2, 8.0, 33, 17, 1), (4, 1, 9.0, 67, 41, 2), (16, 1, 8.0, 129, 70, 1),
+    (64, 1, 10.0, 120, 64, 2), (120, 4, 1.0, 71, 9, 2),
+])
+def test_apply_cell_edges_match_oracle(cav, cascades, size, width, height, sh):
+    orc = _orc()
+    fi = frame_inputs("cornell_256", width=width, height=height)
+    over = dict(cav_resolution=cav, cav_cascades=cascades, cascade0_world_size=size, sh_bands=sh)
+    w = fi.workload.with_(**over)
+    df = _device(fi)
+    announce(f"apply {over} {width}x{height}")
+    r = _renderer(fi, **over)
+    r.set_frame(fi.frame())
+    r.update_volume(w.eye, fi.bbox[:3], fi.bbox[3:])
+    r.voxelize_scene(df.positions, len(fi.positions))
+    r.allocate_caches(df.gbuffer())
+    r.light_caches_rsm(df.rsm(), fi.light)
+    r.apply_caches(df.gbuffer(), df.out)
+    _, live = r.cache_count()
+    vol = orc.update_volume(w.config(), w.eye, fi.bbox[:3], fi.bbox[3:])
+    ref = orc.apply(w.config(), vol, fi.frame(), orc.sh_constants(), fi, r.read_cav(), r.read_caches(live), live)
+    out = df.out.cpu().numpy()
+    if cav == 1:  # the one cell's corners lie outside the volume: no pixel finds a cache but its own cell's
+        assert np.abs(out - ref).max() <= RGB_TOL * max(1.0, np.abs(ref).max())
+    else:
+        assert np.abs(ref).max() > 0.0
+        assert rel_l2(out, ref) < RGB_TOL
+
+
 def test_allocation_reuses_address_volume_across_frames():
     """A renderer that allocates frame A, then frame B (a G-buffer with its
     upper half cleared and its lower half shifted), then A again holds the
