@@ -695,6 +695,12 @@ __device__ __forceinline__ void pack_normal16i(const float* n, int16_t* out) {
 
 __device__ __forceinline__ uint8_t srgb_encode(float c) {
   c = fminf(1.0f, fmaxf(0.0f, c));
+  // Settled in FP32 unless the value lies near a step: the hardware's log2 and
+  // exp2 keep 255 s within 2e-4 (equal for every float in [0, 1]).
+  const float q = c <= 0.0031308f ? 12.92f * c
+                                  : 1.055f * __builtin_amdgcn_exp2f(__builtin_amdgcn_logf(c) * (1.0f / 2.4f)) - 0.055f;
+  const float v = q * 255.0f + 0.5f, low = floorf(v);
+  if (v - low > 0.002f && v - low < 0.998f) return static_cast<uint8_t>(low);
   const double s = c <= 0.0031308 ? 12.92 * c : 1.055 * pow(static_cast<double>(c), 1.0 / 2.4) - 0.055;
   return static_cast<uint8_t>(floor(s * 255.0 + 0.5));
 }
@@ -712,19 +718,49 @@ struct GbufArgs {
   uint8_t* albedo_srgb;
 };
 
-// shader/fillgbuffer.frag: depth, packed normal, sRGB albedo.
+// shader/fillgbuffer.frag: depth, packed normal, sRGB albedo.  A thread shades
+// four pixels, so that every texture is read and written in words (a pixel and
+// three byte stores for each thread, with pow in FP64: 38 us at 1920x1080, now 22).
+__device__ __forceinline__ void shade_gbuffer(const GbufArgs& a, uint32_t t, int16_t* n, uint8_t* al) {
+  n[0] = n[1] = 0;
+  al[0] = al[1] = al[2] = 0;
+  if (t == 0xffffffffu) return;
+  pack_normal16i(a.normals + 3 * static_cast<size_t>(t), n);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) al[k] = srgb_encode(a.albedo[3 * static_cast<size_t>(t) + k]);
+}
+
 __global__ __launch_bounds__(256) void k_gbuffer_resolve(GbufArgs a) {
-  const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= static_cast<size_t>(a.w) * a.h) return;
-  const uint32_t t = a.tri[i];
-  a.depth[i] = static_cast<float>(__longlong_as_double(static_cast<long long>(a.zbits[i])));
-  if (t == 0xffffffffu) {
-    a.normal[2 * i] = a.normal[2 * i + 1] = 0;
-    a.albedo_srgb[3 * i] = a.albedo_srgb[3 * i + 1] = a.albedo_srgb[3 * i + 2] = 0;
+  const size_t i = 4 * (static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x);
+  const size_t n = static_cast<size_t>(a.w) * a.h;
+  if (i >= n) return;
+  if (i + 4 > n) {
+    for (size_t p = i; p < n; ++p) {
+      a.depth[p] = static_cast<float>(__longlong_as_double(static_cast<long long>(a.zbits[p])));
+      shade_gbuffer(a, a.tri[p], a.normal + 2 * p, a.albedo_srgb + 3 * p);
+    }
     return;
   }
-  pack_normal16i(a.normals + 3 * static_cast<size_t>(t), a.normal + 2 * i);
-  for (int k = 0; k < 3; ++k) a.albedo_srgb[3 * i + k] = srgb_encode(a.albedo[3 * static_cast<size_t>(t) + k]);
+  const uint4 t4 = *reinterpret_cast<const uint4*>(a.tri + i);
+  const double2 z0 = *reinterpret_cast<const double2*>(a.zbits + i), z1 = *reinterpret_cast<const double2*>(a.zbits + i + 2);
+  *reinterpret_cast<float4*>(a.depth + i) = make_float4(static_cast<float>(z0.x), static_cast<float>(z0.y),
+                                                        static_cast<float>(z1.x), static_cast<float>(z1.y));
+  const uint32_t t[4] = {t4.x, t4.y, t4.z, t4.w};
+  uint32_t nw[4], aw[3] = {0u, 0u, 0u};
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    int16_t nn[2];
+    uint8_t al[3];
+    shade_gbuffer(a, t[k], nn, al);
+    nw[k] = static_cast<uint16_t>(nn[0]) | (static_cast<uint32_t>(static_cast<uint16_t>(nn[1])) << 16);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) aw[(3 * k + c) / 4] |= static_cast<uint32_t>(al[c]) << (8 * ((3 * k + c) % 4));
+  }
+  *reinterpret_cast<uint4*>(a.normal + 2 * i) = make_uint4(nw[0], nw[1], nw[2], nw[3]);
+  uint32_t* out = reinterpret_cast<uint32_t*>(a.albedo_srgb + 3 * i);
+  out[0] = aw[0];
+  out[1] = aw[1];
+  out[2] = aw[2];
 }
 
 struct RsmArgs {
@@ -780,25 +816,27 @@ __global__ __launch_bounds__(256) void k_rsm_resolve(RsmArgs a) {
   pack_normal16i(a.normals + 3 * static_cast<size_t>(t), a.normal + 2 * i);
 }
 
+// One texel of a level as it is stored.
+struct RsmTexel {
+  uint16_t flux[3];
+  int16_t normal[2];
+  uint16_t dls[2];
+};
+
 // shader/downsamplersm.frag:15-33: flux summed over 2x2, normal the
 // normalized mean repacked, (d, d^2) averaged.
-__global__ __launch_bounds__(256) void k_rsm_downsample(int res, const uint16_t* flux, const int16_t* normal,
-                                                        const uint16_t* dls, uint16_t* flux_out, int16_t* normal_out,
-                                                        uint16_t* dls_out) {
-  const int r2 = res / 2;
-  const size_t o = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (o >= static_cast<size_t>(r2) * r2) return;
-  const int x = static_cast<int>(o % r2), y = static_cast<int>(o / r2);
-  const size_t s[4] = {static_cast<size_t>(2 * y) * res + 2 * x, static_cast<size_t>(2 * y) * res + 2 * x + 1,
-                       static_cast<size_t>(2 * y + 1) * res + 2 * x, static_cast<size_t>(2 * y + 1) * res + 2 * x + 1};
+__device__ __forceinline__ RsmTexel downsample(const RsmTexel* s) {
+  RsmTexel o;
+#pragma unroll
   for (int k = 0; k < 3; ++k) {
-    const float a = half_to_float(flux[3 * s[0] + k]) + half_to_float(flux[3 * s[1] + k]);
-    const float b = half_to_float(flux[3 * s[2] + k]) + half_to_float(flux[3 * s[3] + k]);
-    flux_out[3 * o + k] = f32_to_f16(a + b);
+    const float a = half_to_float(s[0].flux[k]) + half_to_float(s[1].flux[k]);
+    const float b = half_to_float(s[2].flux[k]) + half_to_float(s[3].flux[k]);
+    o.flux[k] = f32_to_f16(a + b);
   }
   float n[3] = {0.0f, 0.0f, 0.0f};
+#pragma unroll
   for (int j = 0; j < 4; ++j) {
-    const f3 u = unpack_normal16i(normal[2 * s[j]], normal[2 * s[j] + 1]);
+    const f3 u = unpack_normal16i(s[j].normal[0], s[j].normal[1]);
     n[0] += u.x;
     n[1] += u.y;
     n[2] += u.z;
@@ -806,11 +844,56 @@ __global__ __launch_bounds__(256) void k_rsm_downsample(int res, const uint16_t*
   const float l = sqrtf(n[0] * n[0] + n[1] * n[1] + n[2] * n[2]);
   if (l > 0.0f)
     for (float& v : n) v /= l;
-  pack_normal16i(n, normal_out + 2 * o);
+  pack_normal16i(n, o.normal);
+#pragma unroll
   for (int k = 0; k < 2; ++k) {
-    const float a = half_to_float(dls[2 * s[0] + k]) + half_to_float(dls[2 * s[1] + k]);
-    const float b = half_to_float(dls[2 * s[2] + k]) + half_to_float(dls[2 * s[3] + k]);
-    dls_out[2 * o + k] = f32_to_f16((a + b) * 0.25f);
+    const float a = half_to_float(s[0].dls[k]) + half_to_float(s[1].dls[k]);
+    const float b = half_to_float(s[2].dls[k]) + half_to_float(s[3].dls[k]);
+    o.dls[k] = f32_to_f16((a + b) * 0.25f);
+  }
+  return o;
+}
+
+// Up to kRsmLevels levels above the level of res^2 texels at the start of the
+// textures: a workgroup takes a square of 2^levels texels a side and keeps each
+// level in LDS for the next (a launch for each level of a 256^2 RSM took 50 us,
+// two launches 27; the time is the chain of sine, cosine and arc tangent).
+constexpr int kRsmLevels = 5;
+
+__global__ __launch_bounds__(256) void k_rsm_downsample(int res, int levels, uint16_t* flux, int16_t* normal,
+                                                        uint16_t* dls) {
+  __shared__ RsmTexel tile[2][256];
+  const int across = res >> levels;
+  const int bx = static_cast<int>(blockIdx.x) % across, by = static_cast<int>(blockIdx.x) / across;
+  const int t = static_cast<int>(threadIdx.x);
+  size_t off = 0;  // of the level below, in texels
+  for (int l = 1; l <= levels; ++l) {
+    const int lb = levels - l, side = 1 << lb, r = res >> (l - 1), r2 = r / 2;
+    const size_t next = off + static_cast<size_t>(r) * r;
+    if (t < side * side) {
+      const int x = t & (side - 1), y = t >> lb;
+      RsmTexel s[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int sx = 2 * x + (j & 1), sy = 2 * y + (j >> 1);
+        if (l == 1) {
+          const size_t p = off + static_cast<size_t>(by * 2 * side + sy) * r + (bx * 2 * side + sx);
+          for (int k = 0; k < 3; ++k) s[j].flux[k] = flux[3 * p + k];
+          for (int k = 0; k < 2; ++k) s[j].normal[k] = normal[2 * p + k];
+          for (int k = 0; k < 2; ++k) s[j].dls[k] = dls[2 * p + k];
+        } else {
+          s[j] = tile[l & 1][sy * 2 * side + sx];
+        }
+      }
+      const RsmTexel o = downsample(s);
+      tile[(l + 1) & 1][t] = o;
+      const size_t p = next + static_cast<size_t>(by * side + y) * r2 + (bx * side + x);
+      for (int k = 0; k < 3; ++k) flux[3 * p + k] = o.flux[k];
+      for (int k = 0; k < 2; ++k) normal[2 * p + k] = o.normal[k];
+      for (int k = 0; k < 2; ++k) dls[2 * p + k] = o.dls[k];
+    }
+    __syncthreads();
+    off = next;
   }
 }
 
@@ -902,7 +985,7 @@ void launch_render_gbuffer(const float* positions, const float* albedo, const fl
   a.normal = normal;
   a.albedo_srgb = albedo_srgb;
   const size_t n = static_cast<size_t>(w) * h;
-  hipLaunchKernelGGL(k_gbuffer_resolve, dim3((n + 255) / 256), dim3(256), 0, s, a);
+  hipLaunchKernelGGL(k_gbuffer_resolve, dim3((n + 1023) / 1024), dim3(256), 0, s, a);
 }
 
 void launch_render_rsm(const float* positions, const float* albedo, const float* normals, uint32_t n_tri,
@@ -931,12 +1014,13 @@ void launch_render_rsm(const float* positions, const float* albedo, const float*
   hipLaunchKernelGGL(k_rsm_resolve, dim3((n + 255) / 256), dim3(256), 0, s, a);
   // Mip chain: level l + 1 from level l, packed one after another.
   size_t off = 0;
-  for (int r = res; r > 1; r /= 2) {
-    const size_t n_in = static_cast<size_t>(r) * r, n_out = n_in / 4;
-    hipLaunchKernelGGL(k_rsm_downsample, dim3((n_out + 255) / 256), dim3(256), 0, s, r, flux + 3 * off,
-                       normal + 2 * off, dls + 2 * off, flux + 3 * (off + n_in), normal + 2 * (off + n_in),
-                       dls + 2 * (off + n_in));
-    off += n_in;
+  int left = __builtin_ctz(static_cast<unsigned>(res));
+  for (int r = res; left > 0;) {
+    const int levels = std::min(left, kRsmLevels), across = r >> levels;
+    hipLaunchKernelGGL(k_rsm_downsample, dim3(static_cast<unsigned>(across) * across), dim3(256), 0, s, r, levels,
+                       flux + 3 * off, normal + 2 * off, dls + 2 * off);
+    for (int l = 0; l < levels; ++l, r /= 2) off += static_cast<size_t>(r) * r;
+    left -= levels;
   }
 }
 

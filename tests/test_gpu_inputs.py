@@ -82,6 +82,29 @@ def test_rsm_chain_matches_host_producer(name):
             _normals_close(gn, nrm, 2e-2, 4)
 
 
+# Less than, just, and more than the five levels of one launch; three launches.
+@pytest.mark.parametrize("res", [8, 16, 32, 128, 2048])
+def test_rsm_mip_launches_match_host_producer(res):
+    from dataclasses import replace
+
+    from dynamicradiancevolume_amd.workloads import CORNELL_256
+
+    fi = frame_inputs("cornell_256", light=replace(CORNELL_256.light, rsm_resolution=res))
+    announce(f"device RSM mips {res}")
+    cfg = fi.workload.config()
+    from dynamicradiancevolume_amd.pipeline import Renderer
+
+    r = Renderer(cfg)
+    df = _device(fi)
+    r.render_rsm(df.scene(), fi.light)
+    assert len(fi.rsm_levels) == res.bit_length()
+    for level, (flux, nrm, dls) in enumerate(fi.rsm_levels):
+        gf, gn, gd = r.read_rsm(level, res)
+        np.testing.assert_array_equal(gf, flux)
+        np.testing.assert_array_equal(gd, dls)
+        _normals_close(gn, nrm, *((1e-4, 1) if level == 0 else (2e-2, 4)))
+
+
 def test_frame_from_device_inputs_matches_host_inputs():
     from dynamicradiancevolume_amd.pipeline import entries_sh
 
