@@ -193,8 +193,8 @@ struct Tuning {
 constexpr int kSpecMaxLevels = 6;  // S <= 32
 struct SpecAtlas {
   uint32_t* atlas = nullptr;
-  Vpl* vpls_lanes = nullptr;  // lane-interleaved VPL records of the current light
-  size_t vpls_lanes_cap = 0;
+  float4* vpl_units = nullptr;  // VPL records of the current light by units
+  size_t vpl_units_cap = 0;     // VPLs
   float* work = nullptr;   // [max_caches][S * S][3]
   float* spill = nullptr;  // [max_caches][2S + 1][3]
   uint32_t width = 0, per_row = 0;
@@ -233,19 +233,21 @@ struct GatherPlan {
   Counter* counter;
   uint32_t quantum, max_splits, target_items;
 };
+constexpr uint32_t kVplUnit = 16;  // consecutive VPLs; divides every read level's count (8x8 is the smallest)
 inline GatherPlan gather_plan(Counter* counter, uint32_t interval, uint32_t max_splits, int grid) {
   return GatherPlan{counter, interval > 64u ? interval : 64u, max_splits, static_cast<uint32_t>(grid) * 4u};
 }
 
 // flux_cut: INDIRECT_SPECULAR skips VALs whose flux sums below 0.001
 // (cacheLightingRSM.comp:240-243); their flux is stored as zero.
-// vpls_lanes (optional): the same records lane-interleaved for the specular
-// gather, record m at (m % per_lane) * 64 + m / per_lane, per_lane = n / 64.
+// vpl_units (optional): the same records for the specular gather, by units of
+// kVplUnit VPLs: three tables [place in the unit][unit] of (position, disc
+// area), (flux, whether any VPL of the unit has flux) and (normal, 0).
 // plan (optional): the gather's split plan, written by the first thread.
 // march (optional, with blocks): kMarchSteps MarchStep records per shadow
 // block, planned for the voxel levels of `vox`.
 void launch_prepare_vpls(const drv_rsm& rsm, const drv_spot_light& light, Vpl* vpls, ShadowBlock* blocks,
-                         int flux_cut, Vpl* vpls_lanes, const GatherPlan* plan, hipStream_t s,
+                         int flux_cut, float4* vpl_units, const GatherPlan* plan, hipStream_t s,
                          MarchStep* march = nullptr, const VoxelView* vox = nullptr);
 // march (optional): the blocks' march plans; without them (or with a tuning
 // other than one block walk at one step per batch) the rays plan their own
@@ -346,7 +348,7 @@ void launch_apply(const drv_config& cfg, const drv_volume& vol, const drv_frame&
 
 // Specular gather of one light into the work sums (first != 0: overwrite),
 // then quantization, mips and hole filling of every live cache's region.
-void launch_specular(const float* cam, const float* caches, int stride, const Counter* counter, const Vpl* vpls,
+void launch_specular(const float* cam, const float* caches, int stride, const Counter* counter, const float4* vpl_units,
                      uint32_t n_vpl, const float* vis, uint32_t vis_pitch, uint32_t interval, const SpecAtlas& at,
                      int first, int grid, hipStream_t s);
 

@@ -478,7 +478,7 @@ void build_split_descs(const SplitViewHost* views, uint32_t n_views, void* host_
     a.block = 1 << static_cast<int>(h.light.indirect_shadow_lod);
     a.flux_cut = 0;
     a.vpls = h.vpls;
-    a.vpls_lanes = nullptr;
+    a.vpl_units = nullptr;
     a.plan = nullptr;
     a.blocks = h.blocks;
     a.march = h.blocks ? h.march : nullptr;

@@ -365,7 +365,7 @@ __global__ __launch_bounds__(256) void k_reduce(float* caches, int stride, const
 }  // namespace
 
 void launch_prepare_vpls(const drv_rsm& rsm, const drv_spot_light& light, Vpl* vpls, ShadowBlock* blocks,
-                         int flux_cut, Vpl* vpls_lanes, const GatherPlan* plan, hipStream_t s, MarchStep* march,
+                         int flux_cut, float4* vpl_units, const GatherPlan* plan, hipStream_t s, MarchStep* march,
                          const VoxelView* vox) {
   PrepArgs a;
   for (int i = 0; i < 16; ++i) a.inv_lvp[i] = light.inverse_light_view_projection[i];
@@ -385,7 +385,7 @@ void launch_prepare_vpls(const drv_rsm& rsm, const drv_spot_light& light, Vpl* v
   a.block = 1 << static_cast<int>(light.indirect_shadow_lod);
   a.flux_cut = flux_cut;
   a.vpls = vpls;
-  a.vpls_lanes = vpls_lanes;
+  a.vpl_units = vpl_units;
   a.plan = plan ? plan->counter : nullptr;
   a.quantum = plan ? plan->quantum : 0u;
   a.max_splits = plan ? plan->max_splits : 0u;

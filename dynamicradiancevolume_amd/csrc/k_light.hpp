@@ -30,7 +30,7 @@ struct PrepArgs {
   int block;  // B = 2^lod texels per block side
   int flux_cut;
   Vpl* vpls;
-  Vpl* vpls_lanes;  // optional lane-interleaved copy: [m % per_lane][m / per_lane], per_lane = n / 64
+  float4* vpl_units;  // optional copy by units of kVplUnit (see launch_prepare_vpls)
   // Optional split plan of the gather (k_plan_gather), done by the first thread.
   Counter* plan;
   uint32_t quantum, max_splits, target_items;
@@ -122,9 +122,14 @@ __device__ __forceinline__ void prepare_vpl(const PrepArgs& a, uint32_t m, uint3
   v.nz = nrm.z;
   v.pad1 = 0.0f;
   a.vpls[m] = v;
-  if (a.vpls_lanes) {
-    const uint32_t per_lane = n / 64u;
-    a.vpls_lanes[static_cast<size_t>(m % per_lane) * 64u + m / per_lane] = v;
+  if (a.vpl_units) {
+    bits |= __shfl_xor(bits, 4);
+    bits |= __shfl_xor(bits, 8);
+    const size_t units = n / kVplUnit;
+    float4* u = a.vpl_units + (m % kVplUnit) * units + m / kVplUnit;
+    u[0] = make_float4(v.px, v.py, v.pz, v.disc_area);
+    u[kVplUnit * units] = make_float4(v.fr, v.fg, v.fb, __uint_as_float(bits));
+    u[2 * kVplUnit * units] = make_float4(v.nx, v.ny, v.nz, 0.0f);
   }
   // Mean normal of a block's VPLs: the B x B texel square of a block is the
   // `interval` Morton-consecutive VPLs m .. m + interval - 1, i.e. adjacent
