@@ -1601,17 +1601,8 @@ int batch_split(drv_batch* b, const drv_rsm* rsms, const drv_spot_light* lights)
   const uint32_t nv = static_cast<uint32_t>(n);
   drvk::launch_batch_split_prepare(b->d_split, nv, b->d_totals, b->sh_bands, b->shadow, max_vpl, max_march,
                                    static_cast<uint32_t>(grid) * 4u, b->stream);
-  if (b->shadow && b->cpw == DRV_BATCH_SPLIT_GATHER) {
-    // Each view's visibility with the single-view kernel and launch shape.
-    for (size_t v = 0; v < n; ++v) {
-      drv_ctx* ctx = b->views[v];
-      drvk::launch_visibility(ctx->vol, hv[v].vox, ctx->caches, b->stride, ctx->counter, ctx->blocks,
-                              hv[v].n_blocks, ctx->visibility, hv[v].vis_pitch, nullptr, ctx->tune,
-                              persistent_grid(ctx), b->stream, ctx->march);
-    }
-  } else if (b->shadow) {
+  if (b->shadow)
     drvk::launch_batch_split_visibility(b->d_split, nv, b->d_totals, b->stride, grid, b->stream);
-  }
   batch_voxels_read(b);
   drvk::launch_batch_split_gather(b->d_split, nv, b->d_totals, b->stride, b->sh_bands, b->shadow, v0->shc, grid,
                                   b->stream);

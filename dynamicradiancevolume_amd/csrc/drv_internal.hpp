@@ -171,7 +171,6 @@ struct SplitViewHost {
 // Item totals of the three queued launches of a batched split pass.
 struct SplitTotals {
   uint32_t vis, gather, reduce;
-  uint32_t vis_head;  // next visibility item to hand out (reset by the plan)
 };
 
 // Launch shapes chosen per context (drv_set_tuning).

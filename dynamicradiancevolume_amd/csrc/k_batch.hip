@@ -21,7 +21,7 @@
 //
 // The split queue (caches per wave DRV_BATCH_SPLIT_QUEUE) runs the
 // single-view kernels' work items of every view in one launch per stage
-// instead: VPL records of every view, a one-thread plan (split counts and
+// instead: VPL records of every view, a one-workgroup plan (split counts and
 // item offsets from the live counts), then the cone-traced visibility, the SH
 // gather and the reduction, each persistent over the concatenated items of
 // all views.  Small views no longer leave the GPU idle behind their own
@@ -238,9 +238,11 @@ __global__ __launch_bounds__(256) void k_split_prepare(const SplitDev* views, ui
 // counts are loaded in parallel (a chain of dependent loads per view in one
 // thread took ~1 us per view), then one thread walks the LDS copy.
 constexpr uint32_t kPlanChunk = 1024;
-// Shadow blocks of one visibility item of the split queue (a lane traces its
-// cache towards them one after the other).
-constexpr uint32_t kSplitBpi = 4;
+// Visibility items of the split queue: two neighbouring 64-cache tiles by two
+// neighbouring shadow blocks (one of each for a wave), as k_visibility_planned.
+__device__ __forceinline__ uint32_t vis_items(uint32_t tiles, uint32_t n_blocks) {
+  return ((tiles + 1u) / 2u) * ((n_blocks + 1u) / 2u);
+}
 __global__ __launch_bounds__(256) void k_split_plan(SplitDev* views, uint32_t n_views, uint32_t target_items,
                                                     int shadow, int sh2, SplitTotals* totals) {
   __shared__ uint32_t live_s[kPlanChunk];
@@ -289,7 +291,7 @@ __global__ __launch_bounds__(256) void k_split_plan(SplitDev* views, uint32_t n_
         d.vis_begin = run[0];
         d.gather_begin = run[1];
         d.reduce_begin = run[2];
-        if (shadow) run[0] += tiles * ((d.n_blocks + kSplitBpi - 1u) / kSplitBpi);
+        if (shadow) run[0] += vis_items(tiles, d.n_blocks);
         run[1] += tiles * groups;
         run[2] += tiles * n_jc;
       }
@@ -300,7 +302,6 @@ __global__ __launch_bounds__(256) void k_split_plan(SplitDev* views, uint32_t n_
     totals->vis = run[0];
     totals->gather = run[1];
     totals->reduce = run[2];
-    totals->vis_head = 0u;
   }
 }
 
@@ -341,7 +342,7 @@ __device__ __forceinline__ VisView vis_view(const SplitDev* views, uint32_t v) {
   w.begin = d->vis_begin;
   w.tiles = d->tiles;
   w.n_blocks = d->n_blocks;
-  w.end = w.begin + w.tiles * ((w.n_blocks + kSplitBpi - 1u) / kSplitBpi);
+  w.end = w.begin + vis_items(w.tiles, w.n_blocks);
   w.live = d->live;
   w.pitch = d->vis_pitch;
   w.caches = d->caches;
@@ -359,51 +360,39 @@ __device__ __forceinline__ VisView vis_view(const SplitDev* views, uint32_t v) {
   return w;
 }
 
-// Items a wave takes from the visibility queue at a time: 1 or 2 contend
-// for the queue head, 8 and more put the items of more views in flight at
-// once (each view traces its own voxel copy).
-constexpr uint32_t kVisChunk = 4;
-
-// Cone-traced visibility of every view: items (view, group of kSplitBpi
-// shadow blocks, 64-cache tile), group-major within a view, handed out in
-// chunks of kVisChunk consecutive items by an atomic queue head, so a wave's
-// items mostly share a view and a block group (its descriptor, block records
-// and march records stay in SGPRs and the scalar cache) and the waves that
-// finish first take more.  Each lane loads its cache once per item and traces
-// it towards the group's blocks with the code of k_visibility_planned (the
-// view's march plan), so the values are those of the single-view kernels.
+// Cone-traced visibility of every view: the workgroup items of all views, view
+// after view and in k_visibility_planned's order within one, so that at a time
+// one or two views are traced (each has its own voxel copy), and only the last
+// one's tail leaves the GPU idle.  The traces are those of k_visibility_planned
+// (the view's march plan).  Sixteen views of 5000 caches and 256 blocks: 569 us
+// against 690 for sixteen launches of it, which waves that took four blocks each
+// from an atomic queue did not reach either; with a quarter of the workgroups
+// 635, with four times as many 598.
 __global__ __launch_bounds__(256) void k_split_visibility(const SplitDev* views, uint32_t n_views, int stride,
-                                                          SplitTotals* totals) {
+                                                          const SplitTotals* totals) {
   const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t items = totals->vis;
   VisView w;
   w.begin = w.end = 0u;
-  while (true) {
-    uint32_t base = 0u;
-    if (lane == 0u) base = atomicAdd(&totals->vis_head, kVisChunk);
-    base = __builtin_amdgcn_readfirstlane(__shfl(base, 0));
-    if (base >= items) break;
-    const uint32_t stop = min(items, base + kVisChunk);
-    for (uint32_t item = base; item < stop; ++item) {
-      if (item < w.begin || item >= w.end) w = vis_view(views, split_view<0>(views, n_views, item));
-      const uint32_t local = item - w.begin;
-      const uint32_t group = local / w.tiles, tile = local - group * w.tiles;
-      const uint32_t cache = tile * 64u + lane;
-      const bool valid = cache < w.live;
-      const float* e = w.caches + static_cast<size_t>(valid ? cache : w.live - 1u) * stride;
-      const f3 wp = make3(e[0], e[1], e[2]);
-      const float vsz = w.voxel_size * static_cast<float>(w.vox.res), inv_vsz = 1.0f / vsz;
-      const f3 vpos = make3(volume_coord(wp.x - w.vmin[0], vsz, inv_vsz), volume_coord(wp.y - w.vmin[1], vsz, inv_vsz),
-                            volume_coord(wp.z - w.vmin[2], vsz, inv_vsz));
-      const __amdgpu_buffer_rsrc_t cr = corner_rsrc(w.vox);
-      const uint32_t b0 = group * kSplitBpi, b1 = min(w.n_blocks, b0 + kSplitBpi);
-      for (uint32_t b = b0; b < b1; ++b) {
-        const Trace t =
-            w.fidx ? trace_planned<false, true>(w.vox, cr, w.blocks, w.march, b, w.voxel_size, wp, vpos, valid)
-                   : trace_planned<false, false>(w.vox, cr, w.blocks, w.march, b, w.voxel_size, wp, vpos, valid);
-        if (valid) w.vis[static_cast<size_t>(b) * w.pitch + cache] = trace_visibility(t);
-      }
-    }
+  for (uint32_t item = blockIdx.x; item < items; item += gridDim.x) {
+    if (item < w.begin || item >= w.end) w = vis_view(views, split_view<0>(views, n_views, item));
+    const uint32_t local = item - w.begin, tile_pairs = (w.tiles + 1u) / 2u;
+    const uint32_t pair = local / tile_pairs;
+    const uint32_t tile = 2u * (local - pair * tile_pairs) + (wave & 1u), b = 2u * pair + (wave >> 1);
+    if (tile >= w.tiles || b >= w.n_blocks) continue;
+    const uint32_t cache = tile * 64u + lane;
+    const bool valid = cache < w.live;
+    const float* e = w.caches + static_cast<size_t>(valid ? cache : w.live - 1u) * stride;
+    const f3 wp = make3(e[0], e[1], e[2]);
+    const float vsz = w.voxel_size * static_cast<float>(w.vox.res), inv_vsz = 1.0f / vsz;
+    const f3 vpos = make3(volume_coord(wp.x - w.vmin[0], vsz, inv_vsz), volume_coord(wp.y - w.vmin[1], vsz, inv_vsz),
+                          volume_coord(wp.z - w.vmin[2], vsz, inv_vsz));
+    const __amdgpu_buffer_rsrc_t cr = corner_rsrc(w.vox);
+    const Trace t =
+        w.fidx ? trace_planned<false, true>(w.vox, cr, w.blocks, w.march, b, w.voxel_size, wp, vpos, valid)
+               : trace_planned<false, false>(w.vox, cr, w.blocks, w.march, b, w.voxel_size, wp, vpos, valid);
+    if (valid) w.vis[static_cast<size_t>(b) * w.pitch + cache] = trace_visibility(t);
   }
 }
 
@@ -512,7 +501,7 @@ void launch_batch_split_prepare(void* descs, uint32_t n_views, SplitTotals* tota
 
 void launch_batch_split_visibility(void* descs, uint32_t n_views, SplitTotals* totals, int stride, int grid,
                                    hipStream_t s) {
-  hipLaunchKernelGGL(k_split_visibility, dim3(grid), dim3(256), 0, s, static_cast<SplitDev*>(descs), n_views, stride,
+  hipLaunchKernelGGL(k_split_visibility, dim3(4 * grid), dim3(256), 0, s, static_cast<SplitDev*>(descs), n_views, stride,
                      totals);
 }
 
