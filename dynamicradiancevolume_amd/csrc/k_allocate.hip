@@ -57,6 +57,7 @@ struct AllocArgs {
   Counter* counter;
   float4* phantoms;  // positions of appended corners outside the CAV, [capacity]
   int width, height, R, C;
+  float inv_width, inv_height;
   uint32_t capacity;
   int transitions;
 };
@@ -80,9 +81,9 @@ __device__ __forceinline__ Cell cell_of(const AllocArgs& a, const drv_cascade& k
     qy = (wp.y - k.min[1]) * s;
     qz = (wp.z - k.min[2]) * s;
   } else {
-    qx = (wp.x - k.min[0]) / k.world_voxel_size;
-    qy = (wp.y - k.min[1]) / k.world_voxel_size;
-    qz = (wp.z - k.min[2]) / k.world_voxel_size;
+    qx = cell_coordinate(wp.x - k.min[0], k);
+    qy = cell_coordinate(wp.y - k.min[1], k);
+    qz = cell_coordinate(wp.z - k.min[2], k);
   }
   const int R = a.R;
   Cell e;
@@ -177,8 +178,9 @@ __device__ __forceinline__ void mark_corners(const AllocArgs& a, bool active, in
 
 // 16x16 pixel tiles per pass-1 workgroup (one: 4K 89 us, two: 79).  Bound by
 // instructions and the wait for the depths: 4K 97 us, 79 since waves without a
-// leader skip the marks and the cascade is found without branches; 1080p 26 and
-// 22 us.
+// leader skip the marks and the cascade is found without branches, 72 with the
+// cascades in LDS and without IEEE divisions by the cell size and the window;
+// 1080p 26, 22 and 21 us.
 constexpr int kAllocTiles = 2;
 
 template <bool kPow2>
@@ -188,6 +190,8 @@ __global__ __launch_bounds__(256) void k_allocate(AllocArgs a) {
   // lists are built before one barrier.  The leader rule stays per tile.
   __shared__ int list[kAllocTiles][256];
   __shared__ int list2[kAllocTiles][256];
+  __shared__ drv_cascade cascades[DRV_MAX_CASCADES];
+  stage_cascades(a.vol, cascades);
   const int t = threadIdx.x;
   const int lx = t & 15, ly = t >> 4;
   const int y = blockIdx.y * 16 + ly;
@@ -197,6 +201,7 @@ __global__ __launch_bounds__(256) void k_allocate(AllocArgs a) {
     const int x = (blockIdx.x * kAllocTiles + h) * 16 + lx;
     d[h] = (x < a.width && y < a.height) ? a.depth[static_cast<size_t>(y) * a.width + x] : 0.0f;
   }
+  __syncthreads();  // the cascades
   int own[kAllocTiles], own2[kAllocTiles], c[kAllocTiles];
   Cell e[kAllocTiles], e2[kAllocTiles];
 #pragma unroll
@@ -209,15 +214,15 @@ __global__ __launch_bounds__(256) void k_allocate(AllocArgs a) {
     e2[h] = Cell{0, 0, 0, -1};
     // Pixels outside the image read depth 0: no geometry, as in the reference.
     if (d[h] > 0.0001f) {
-      const f3 wp = unproject_pixel(a.inv_vp, a.width, a.height, x, y, d[h]);
+      const f3 wp = unproject_pixel(a.inv_vp, a.width, a.height, a.inv_width, a.inv_height, x, y, d[h]);
       c[h] = cascade_of(a.vol, a.C, wp);
-      const drv_cascade k = cascade_at(a.vol, c[h]);
+      const drv_cascade k = cascades[c[h]];
       e[h] = cell_of<kPow2>(a, k, wp, c[h]);
       own[h] = e[h].flat;
       if (a.transitions) {
         const float tr = cascade_transition(a.vol, k, wp);
         if (tr > 0.0f && c[h] < a.C - 1) {
-          e2[h] = cell_of<kPow2>(a, cascade_at(a.vol, c[h] + 1), wp, c[h] + 1);
+          e2[h] = cell_of<kPow2>(a, cascades[c[h] + 1], wp, c[h] + 1);
           own2[h] = e2[h].flat;
         }
       }
@@ -618,6 +623,8 @@ void launch_allocate(const drv_config& cfg, const drv_volume& vol, const drv_fra
   a.phantoms = phantoms;
   a.width = cfg.width;
   a.height = cfg.height;
+  a.inv_width = 1.0f / static_cast<float>(cfg.width);
+  a.inv_height = 1.0f / static_cast<float>(cfg.height);
   a.R = cfg.cav_resolution;
   a.C = cfg.cav_cascades;
   a.capacity = static_cast<uint32_t>(cfg.max_caches);

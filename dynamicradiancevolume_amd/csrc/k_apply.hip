@@ -34,6 +34,7 @@ struct ApplyArgs {
   const float* srgb_lut;
   float* out;
   int width, height, R, C, stride, sh2, transitions, accumulate;
+  float inv_width, inv_height;
   // INDIRECT_SPECULAR
   const uint8_t* roughness_metallic;  // RG8 or null (roughness 1, metallic 0)
   const uint32_t* atlas;
@@ -230,9 +231,9 @@ __device__ __forceinline__ void corner_caches(const ApplyArgs& a, bool active, i
 // each, the 8 corners' loads in flight together - and staged in LDS, where
 // their lanes read them; lanes with a third or later address load their own
 // entry, lanes without a cache (an unclaimed cell, one past the live caches)
-// read zeros.  Bound by vector instructions in large images (3840x2160: 175 us)
+// read zeros.  Bound by vector instructions in large images (3840x2160: 167 us)
 // and by the chain of loads in small ones, so the loads stand outside of
-// branches: 320x180 19.5 -> 14.6 us, 256x256 14.1 -> 10.6, 1920x1080 52 -> 51 (66
+// branches: 320x180 19.5 -> 14.1 us, 256x256 14.1 -> 9.8, 1920x1080 52 -> 47 (66
 // with the sums on the matrix unit, 4x4x1 with an entry broadcast).  Per lane the
 // arithmetic and its order are those of one fetch per pixel.  Every lane of
 // the wave must call this (the staging is cooperative); `active` = false lanes
@@ -243,9 +244,9 @@ __device__ __forceinline__ void lighting(const ApplyArgs& a, bool active, f3 wp,
                                          float* out) {
   out[0] = out[1] = out[2] = 0.0f;
   if (__ballot(active) == 0ull) return;
-  const float acx = (wp.x - k.min[0]) / k.world_voxel_size;
-  const float acy = (wp.y - k.min[1]) / k.world_voxel_size;
-  const float acz = (wp.z - k.min[2]) / k.world_voxel_size;
+  const float acx = cell_coordinate(wp.x - k.min[0], k);
+  const float acy = cell_coordinate(wp.y - k.min[1], k);
+  const float acz = cell_coordinate(wp.z - k.min[2], k);
   const int ax = to_int(acx), ay = to_int(acy), az = to_int(acz);
   const float ix = acx - static_cast<float>(ax), iy = acy - static_cast<float>(ay), iz = acz - static_cast<float>(az);
   const float jx = 1.0f - ix, jy = 1.0f - iy, jz = 1.0f - iz;
@@ -257,7 +258,7 @@ __device__ __forceinline__ void lighting(const ApplyArgs& a, bool active, f3 wp,
   const uint32_t sub = lane & 31u;
   const int nq = a.sh2 ? 8 : 4;
   const bool fetches = sub < static_cast<uint32_t>(4 * (nq - 1));  // entry floats 4 .. 4 nq - 1 are read
-  const float* entry = a.caches + 4u + sub;
+  const float* entry = a.caches + 4u + (fetches ? sub : 0u);
   uint32_t from[8];  // the entry's place in the stage (0: first address, 32: second), kOwn or kNone
   constexpr uint32_t kOwn = 1u, kNone = 2u;
   float part[8];
@@ -344,7 +345,9 @@ template <bool kSpec>
 __global__ __launch_bounds__(256) void k_apply(ApplyArgs a) {
   __shared__ float lut[256];
   __shared__ __align__(16) float stage[4][8 * 64 + 32];  // per wave: the shared entries of each corner, zeros
+  __shared__ drv_cascade cascades[DRV_MAX_CASCADES];  // looked up by lane
   lut[threadIdx.x] = a.srgb_lut[threadIdx.x];
+  stage_cascades(a.vol, cascades);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (lane < 32) stage[wave][8 * 64 + lane] = 0.0f;
   const int x = blockIdx.x * 16 + 8 * (wave & 1) + (lane & 7);
@@ -364,9 +367,9 @@ __global__ __launch_bounds__(256) void k_apply(ApplyArgs a) {
   // the (cooperative) cache fetches, inactive.
   const bool valid = inside && !(d < 0.00001f);
   const uint32_t live = a.counter->live;
-  const f3 wp = unproject_pixel(a.inv_vp, a.width, a.height, x, y, d);
+  const f3 wp = unproject_pixel(a.inv_vp, a.width, a.height, a.inv_width, a.inv_height, x, y, d);
   const int c = cascade_of(a.vol, a.C, wp);
-  const drv_cascade& k = a.vol.cascades[c];
+  const drv_cascade k = cascades[c];
   const f3 n = shading_normal(static_cast<int16_t>(nrm & 0xFFFFu), static_cast<int16_t>(nrm >> 16));
   float diffuse[3] = {lut[al0], lut[al1], lut[al2]};
   SpecPixel sp{};
@@ -414,7 +417,7 @@ __global__ __launch_bounds__(256) void k_apply(ApplyArgs a) {
     if (__ballot(two) != 0ull) {
       float col2[3];
       const int c2 = two ? c + 1 : c;
-      lighting<kSpec>(a, two, wp, n, c2, a.vol.cascades[c2], diffuse, live, sp, st, col2);
+      lighting<kSpec>(a, two, wp, n, c2, cascades[c2], diffuse, live, sp, st, col2);
       if (two) {
         col[0] = col[0] * (1.0f - t) + col2[0] * t;
         col[1] = col[1] * (1.0f - t) + col2[1] * t;
@@ -458,6 +461,8 @@ void launch_apply(const drv_config& cfg, const drv_volume& vol, const drv_frame&
   a.out = out_rgb;
   a.width = cfg.width;
   a.height = cfg.height;
+  a.inv_width = 1.0f / static_cast<float>(cfg.width);
+  a.inv_height = 1.0f / static_cast<float>(cfg.height);
   a.R = cfg.cav_resolution;
   a.C = cfg.cav_cascades;
   a.stride = entry_stride(cfg.sh_bands);

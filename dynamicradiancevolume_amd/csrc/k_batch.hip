@@ -386,8 +386,8 @@ __global__ __launch_bounds__(256) void k_split_visibility(const SplitDev* views,
     const float* e = w.caches + static_cast<size_t>(valid ? cache : w.live - 1u) * stride;
     const f3 wp = make3(e[0], e[1], e[2]);
     const float vsz = w.voxel_size * static_cast<float>(w.vox.res), inv_vsz = 1.0f / vsz;
-    const f3 vpos = make3(volume_coord(wp.x - w.vmin[0], vsz, inv_vsz), volume_coord(wp.y - w.vmin[1], vsz, inv_vsz),
-                          volume_coord(wp.z - w.vmin[2], vsz, inv_vsz));
+    const f3 vpos = make3(quotient(wp.x - w.vmin[0], vsz, inv_vsz), quotient(wp.y - w.vmin[1], vsz, inv_vsz),
+                          quotient(wp.z - w.vmin[2], vsz, inv_vsz));
     const __amdgpu_buffer_rsrc_t cr = corner_rsrc(w.vox);
     const Trace t =
         w.fidx ? trace_planned<false, true>(w.vox, cr, w.blocks, w.march, b, w.voxel_size, wp, vpos, valid)

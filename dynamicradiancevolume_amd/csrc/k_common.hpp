@@ -47,14 +47,34 @@ __device__ __forceinline__ void mat_vec(const float* m, float x, float y, float 
 
 // Pixel centre (x + 0.5, y + 0.5) with reverse-Z depth -> world position
 // (cacheGather.comp:113-119, cacheApply.frag:134-135).
-__device__ __forceinline__ f3 unproject_pixel(const float* inv_vp, int w, int h, int x, int y, float depth) {
-  const float px = static_cast<float>(x) + 0.5f;
-  const float py = static_cast<float>(y) + 0.5f;
-  const float sx = px / static_cast<float>(w) * 2.0f - 1.0f;
-  const float sy = py / static_cast<float>(h) * 2.0f - 1.0f;
+__device__ __forceinline__ f3 unproject_screen(const float* inv_vp, float sx, float sy, float depth) {
   float v[4];
   mat_vec(inv_vp, sx, sy, depth, 1.0f, v);
   return make3(v[0] / v[3], v[1] / v[3], v[2] / v[3]);
+}
+
+__device__ __forceinline__ f3 unproject_pixel(const float* inv_vp, int w, int h, int x, int y, float depth) {
+  const float px = static_cast<float>(x) + 0.5f;
+  const float py = static_cast<float>(y) + 0.5f;
+  return unproject_screen(inv_vp, px / static_cast<float>(w) * 2.0f - 1.0f, py / static_cast<float>(h) * 2.0f - 1.0f,
+                          depth);
+}
+
+// d / size with inv = 1 / size correctly rounded: a quotient estimate corrected
+// by its exact remainder is the correctly rounded quotient (Markstein), in 3
+// instructions instead of 11.  Finite quotients only.
+__device__ __forceinline__ float quotient(float d, float size, float inv) {
+  const float q = d * inv;
+  return __builtin_fmaf(__builtin_fmaf(-q, size, d), inv, q);
+}
+
+// unproject_pixel with inv_w = 1 / w and inv_h = 1 / h.
+__device__ __forceinline__ f3 unproject_pixel(const float* inv_vp, int w, int h, float inv_w, float inv_h, int x, int y,
+                                              float depth) {
+  const float px = static_cast<float>(x) + 0.5f;
+  const float py = static_cast<float>(y) + 0.5f;
+  return unproject_screen(inv_vp, quotient(px, static_cast<float>(w), inv_w) * 2.0f - 1.0f,
+                          quotient(py, static_cast<float>(h), inv_h) * 2.0f - 1.0f, depth);
 }
 
 // ComputeAddressVolumeCascade, shader/lightcache.glsl:109-122: the first cascade
@@ -71,26 +91,24 @@ __device__ __forceinline__ int cascade_of(const drv_volume& vol, int n, f3 wp) {
   return found;
 }
 
-// The lane's cascade c of n, chosen out of scalar loads where a lookup by lane
-// would wait for a memory load of each member (the allocation; a kernel that is
-// bound by instructions is better off with the loads).  Most waves see one or
-// two cascades.
-__device__ __forceinline__ drv_cascade cascade_at(const drv_volume& vol, int c) {
-  drv_cascade k = vol.cascades[0];
-#pragma unroll
-  for (int i = 1; i < DRV_MAX_CASCADES; ++i) {
-    const bool me = c == i;
-    if (__ballot(me) == 0ull) continue;
-    const drv_cascade& s = vol.cascades[i];
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      k.min[j] = me ? s.min[j] : k.min[j];
-      k.decision_min[j] = me ? s.decision_min[j] : k.decision_min[j];
-      k.decision_max[j] = me ? s.decision_max[j] : k.decision_max[j];
-    }
-    k.world_voxel_size = me ? s.world_voxel_size : k.world_voxel_size;
-  }
-  return k;
+// The cascades in LDS, for lookups by lane: from the kernel's arguments each
+// would be a memory load on the way to the address volume.  pad0 holds
+// 1 / world_voxel_size.  The caller synchronises the workgroup (of 64 threads or
+// more).
+__device__ __forceinline__ void stage_cascades(const drv_volume& vol, drv_cascade* out) {
+  constexpr uint32_t kWords = sizeof(drv_cascade) / sizeof(uint32_t) * DRV_MAX_CASCADES;
+  static_assert(kWords <= 64u, "one word for each thread");
+  if (threadIdx.x < kWords)
+    reinterpret_cast<uint32_t*>(out)[threadIdx.x] = reinterpret_cast<const uint32_t*>(vol.cascades)[threadIdx.x];
+  __builtin_amdgcn_wave_barrier();  // the same wave's LDS stores stay in order
+  if (threadIdx.x < DRV_MAX_CASCADES) out[threadIdx.x].pad0 = 1.0f / vol.cascades[threadIdx.x].world_voxel_size;
+}
+
+// Coordinate d (from the volume's corner) in cells of a staged cascade.
+__device__ __forceinline__ float cell_coordinate(float d, const drv_cascade& k) {
+  const float estimate = d * k.pad0;
+  const float q = __builtin_fmaf(__builtin_fmaf(-estimate, k.world_voxel_size, d), k.pad0, estimate);
+  return __builtin_isinf(estimate) ? estimate : q;
 }
 
 // ComputeAddressVolumeCascadeTransition, shader/lightcache.glsl:125-134.

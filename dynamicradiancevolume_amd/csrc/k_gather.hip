@@ -201,8 +201,8 @@ __global__ __launch_bounds__(256) void k_visibility_planned(VisArgs a) {
     const float* e = a.caches + static_cast<size_t>(valid ? cache : live - 1u) * a.stride;
     const f3 wp = make3(e[0], e[1], e[2]);
     // cacheLightingRSM.comp:103-104
-    const f3 vpos = make3(volume_coord(wp.x - a.vmin[0], vsz, inv_vsz), volume_coord(wp.y - a.vmin[1], vsz, inv_vsz),
-                          volume_coord(wp.z - a.vmin[2], vsz, inv_vsz));
+    const f3 vpos = make3(quotient(wp.x - a.vmin[0], vsz, inv_vsz), quotient(wp.y - a.vmin[1], vsz, inv_vsz),
+                          quotient(wp.z - a.vmin[2], vsz, inv_vsz));
     const uint32_t b0 = group * bpi;
     const uint32_t b1 = min(a.n_blocks, b0 + bpi);
     for (uint32_t b = b0; b < b1; ++b) {

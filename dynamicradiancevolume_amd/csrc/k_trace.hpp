@@ -212,14 +212,6 @@ __device__ __forceinline__ bool march_planned(MarchSteps pl, const MarchStep& fi
   return stopped;
 }
 
-// (wp - vmin) / vsz of a cache (cacheLightingRSM.comp:103-104) with inv = 1 / vsz
-// correctly rounded: a quotient estimate corrected by its exact remainder is
-// the correctly rounded quotient (Markstein), the value of the division.
-__device__ __forceinline__ float volume_coord(float d, float vsz, float inv) {
-  const float q = d * inv;
-  return __builtin_fmaf(__builtin_fmaf(-q, vsz, d), inv, q);
-}
-
 // The whole trace (samples 0 .. 31) of cache wp towards block b, the same for
 // every lane of the wave; lanes with live = false take no samples.
 template <bool kCount = false, bool kFloatIndex = false>
