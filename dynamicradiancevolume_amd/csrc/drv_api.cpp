@@ -1501,6 +1501,13 @@ struct drv_batch {
 
 namespace {
 
+// With more shadow blocks than this in a view, DRV_BATCH_SPLIT_GATHER gives every
+// view a visibility launch of its own; with fewer such a launch leaves the GPU
+// idle behind its slowest rays for too long.  Per view of a captured batch, one
+// launch / launches: 256 blocks 112 / 118 us (320x180), 152 / 157 (1280x720); 1024
+// blocks 250 / 239 and 280 / 272; 64 views of 256-2048 blocks at 720p-4K 18.9 /
+// 13.5 ms.
+constexpr uint32_t kQueuedBlocks = 512;
 constexpr size_t kBatchPartialFloats = size_t(1) << 28;  // 1 GiB of split partials at most
 
 int bfail(drv_batch* b, int code, const std::string& msg) {
@@ -1601,8 +1608,19 @@ int batch_split(drv_batch* b, const drv_rsm* rsms, const drv_spot_light* lights)
   const uint32_t nv = static_cast<uint32_t>(n);
   drvk::launch_batch_split_prepare(b->d_split, nv, b->d_totals, b->sh_bands, b->shadow, max_vpl, max_march,
                                    static_cast<uint32_t>(grid) * 4u, b->stream);
-  if (b->shadow)
+  bool large = false;
+  for (const drvk::SplitViewHost& d : hv) large = large || d.n_blocks > kQueuedBlocks;
+  if (b->shadow && b->cpw == DRV_BATCH_SPLIT_GATHER && large) {
+    // Each view's visibility with the single-view kernel and launch shape.
+    for (size_t v = 0; v < n; ++v) {
+      drv_ctx* ctx = b->views[v];
+      drvk::launch_visibility(ctx->vol, hv[v].vox, ctx->caches, b->stride, ctx->counter, ctx->blocks,
+                              hv[v].n_blocks, ctx->visibility, hv[v].vis_pitch, nullptr, ctx->tune,
+                              persistent_grid(ctx), b->stream, ctx->march);
+    }
+  } else if (b->shadow) {
     drvk::launch_batch_split_visibility(b->d_split, nv, b->d_totals, b->stride, grid, b->stream);
+  }
   batch_voxels_read(b);
   drvk::launch_batch_split_gather(b->d_split, nv, b->d_totals, b->stride, b->sh_bands, b->shadow, v0->shc, grid,
                                   b->stream);

@@ -365,7 +365,7 @@ __device__ __forceinline__ VisView vis_view(const SplitDev* views, uint32_t v) {
 // one or two views are traced (each has its own voxel copy), and only the last
 // one's tail leaves the GPU idle.  The traces are those of k_visibility_planned
 // (the view's march plan).  Sixteen views of 5000 caches and 256 blocks: 569 us
-// against 690 for sixteen launches of it, which waves that took four blocks each
+// against 690 for sixteen launches of it (large views: see the caller), which waves that took four blocks each
 // from an atomic queue did not reach either; with a quarter of the workgroups
 // 635, with four times as many 598.
 __global__ __launch_bounds__(256) void k_split_visibility(const SplitDev* views, uint32_t n_views, int stride,
