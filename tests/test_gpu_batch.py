@@ -16,7 +16,7 @@ import pytest
 import torch
 
 from canon import rel_l2
-from conftest import announce
+from conftest import announce, frame_inputs
 
 pytestmark = pytest.mark.gpu
 
@@ -196,6 +196,41 @@ def test_split_queue_visibility_and_sh_equal_single_views(mode):
         o1 = np.lexsort(pos1.view(np.uint32).T)
         np.testing.assert_array_equal(pos1[o1], pos0[o0])
         np.testing.assert_array_equal(r.read_visibility(live, nb)[o1], v0[o0])
+    b.close()
+
+
+# One visibility launch for all views up to 512 shadow blocks (an odd count of
+# tiles and of blocks among them), one for each view as soon as a view has more.
+@pytest.mark.parametrize("lights", [((64, 2), (64, 2)), ((64, 2), (32, 5), (8, 0)), ((64, 2), (128, 2)),
+                                    ((128, 2), (128, 2))])
+def test_split_gather_visibility_of_small_and_large_views(lights):
+    from dataclasses import replace
+
+    from dynamicradiancevolume_amd.pipeline import Batch
+    from dynamicradiancevolume_amd.workloads import CORNELL_256
+
+    frames = [frame_inputs("cornell_256", width=160 + 32 * i, height=96,
+                           light=replace(CORNELL_256.light, rsm_resolution=res, indirect_shadow_lod=lod))
+              for i, (res, lod) in enumerate(lights)]
+    announce(f"split gather of views with lights {lights}")
+    ref = []
+    rs1, dfs1 = _group(frames, 1)
+    for r, df, fi in zip(rs1, dfs1, frames):
+        r.render_frame(df)
+        _, live = r.cache_count()
+        nb = fi.n_vpl // int(fi.light.indirect_shadow_sample_interval)
+        ref.append((r.read_visibility(live, nb), r.read_caches(live)[:, :3].copy()))
+        r.close()
+    rs, dfs = _group(frames, 1)
+    b = Batch(rs)
+    b.set_tuning(-2, 1024)
+    b.render_frame(dfs)
+    for (v0, pos0), r in zip(ref, rs):
+        _, live = r.cache_count()
+        pos1 = r.read_caches(live)[:, :3].copy()
+        o0, o1 = (np.lexsort(p.view(np.uint32).T) for p in (pos0, pos1))
+        np.testing.assert_array_equal(pos1[o1], pos0[o0])
+        np.testing.assert_array_equal(r.read_visibility(live, v0.shape[1])[o1], v0[o0])
     b.close()
 
 
