@@ -191,16 +191,18 @@ struct __attribute__((aligned(4))) CellPair {
 // pair is one 8-byte load when both lie in the row; texelFetch outside the CAV
 // reads 0 -> address 0xFFFFFFFF, as inactive lanes get.  A wave whose cells all
 // lie inside loads without branches, its four pairs in flight together.
-__device__ __forceinline__ void corner_caches(const ApplyArgs& a, bool active, int x0, int ay, int az,
+// Coordinates are unsigned, so that -1 + 1 is cell 0 and every other one below
+// zero or saturated (a pixel far outside, at infinity) lies past the end.
+__device__ __forceinline__ void corner_caches(const ApplyArgs& a, bool active, uint32_t x0, uint32_t ay, uint32_t az,
                                               uint32_t* addr) {
-  const int R = a.R, CR = a.C * a.R;
-  const bool in = x0 >= 0 && x0 + 1 < CR && ay >= 0 && ay + 1 < R && az >= 0 && az + 1 < R;
+  const uint32_t R = static_cast<uint32_t>(a.R), CR = static_cast<uint32_t>(a.C * a.R);
+  const bool in = x0 < CR - 1u && ay < R - 1u && az < R - 1u;
   if (__ballot(active && !in) == 0ull) {
-    const uint32_t at = active ? static_cast<uint32_t>((az * R + ay) * CR + x0) : 0u;
+    const uint32_t at = active ? (az * R + ay) * CR + x0 : 0u;
     CellPair q[4];
 #pragma unroll
-    for (int p = 0; p < 4; ++p)
-      q[p] = *reinterpret_cast<const CellPair*>(a.cav + at + static_cast<uint32_t>(((p >> 1) * R + (p & 1)) * CR));
+    for (uint32_t p = 0; p < 4u; ++p)
+      q[p] = *reinterpret_cast<const CellPair*>(a.cav + at + ((p >> 1) * R + (p & 1u)) * CR);
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
       addr[2 * p] = active ? q[p].a - 1u : 0xFFFFFFFFu;
@@ -209,14 +211,14 @@ __device__ __forceinline__ void corner_caches(const ApplyArgs& a, bool active, i
     return;
   }
 #pragma unroll
-  for (int p = 0; p < 4; ++p) {
-    const int y = ay + (p & 1), z = az + (p >> 1);
-    const bool row = active && y >= 0 && z >= 0 && y < R && z < R;
+  for (uint32_t p = 0; p < 4u; ++p) {
+    const uint32_t y = ay + (p & 1u), z = az + (p >> 1);
+    const bool row = active && y < R && z < R;
     uint32_t v0 = 0u, v1 = 0u;
     if (row) {
-      const uint32_t* r = a.cav + (static_cast<uint32_t>(z) * R + y) * CR;
-      if (x0 >= 0 && x0 < CR) v0 = r[x0];
-      if (x0 + 1 >= 0 && x0 + 1 < CR) v1 = r[x0 + 1];
+      const uint32_t* r = a.cav + (z * R + y) * CR;
+      if (x0 < CR) v0 = r[x0];
+      if (x0 + 1u < CR) v1 = r[x0 + 1u];
     }
     addr[2 * p] = v0 - 1u;
     addr[2 * p + 1] = v1 - 1u;
@@ -253,7 +255,8 @@ __device__ __forceinline__ void lighting(const ApplyArgs& a, bool active, f3 wp,
   const float w[8] = {jx * jy * jz, ix * jy * jz, jx * iy * jz, ix * iy * jz,
                       jx * jy * iz, ix * jy * iz, jx * iy * iz, ix * iy * iz};
   uint32_t addr[8];
-  corner_caches(a, active, ax + a.R * c, ay, az, addr);
+  corner_caches(a, active, static_cast<uint32_t>(ax) + static_cast<uint32_t>(a.R * c), static_cast<uint32_t>(ay),
+                static_cast<uint32_t>(az), addr);
   const uint32_t lane = __lane_id();
   const uint32_t sub = lane & 31u;
   const int nq = a.sh2 ? 8 : 4;

@@ -196,6 +196,36 @@ def test_apply_cell_edges_match_oracle(cav, cascades, size, width, height, sh):
         assert rel_l2(out, ref) < RGB_TOL
 
 
+# Pixels that unproject to cells past the 32-bit range along one axis, the
+# others inside the volume, and to infinity: no cache is there to light them.
+@pytest.mark.parametrize("cascades", [1, 4])
+@pytest.mark.parametrize("far", ["x", "y", "z", "inf"])
+def test_apply_of_pixels_beyond_the_integer_range_finds_no_cache(far, cascades):
+    fi = frame_inputs("cornell_256", width=64, height=48)
+    over = dict(cav_cascades=cascades, cascade0_world_size=8.0)
+    w = fi.workload.with_(**over)
+    df = _device(fi)
+    announce(f"apply far along {far}, {cascades} cascades")
+    r = _renderer(fi, **over)
+    r.set_frame(fi.frame())
+    r.update_volume(w.eye, fi.bbox[:3], fi.bbox[3:])
+    r.voxelize_scene(df.positions, len(fi.positions))
+    r.allocate_caches(df.gbuffer())
+    r.light_caches_rsm(df.rsm(), fi.light)
+    frame = fi.frame()
+    rows = [[0.01, 0.01, 0.0, e] for e in w.eye] + [[0.0, 0.0, 0.0, 0.0 if far == "inf" else 1.0]]
+    if far != "inf":
+        rows["xyz".index(far)] = [1e30, 1e25, 0.0, 0.0]
+    frame.inverse_view_projection[:] = [v for row in rows for v in row]
+    r.set_frame(frame)
+    df.out.fill_(7.0)
+    r.apply_caches(df.gbuffer(), df.out)
+    assert not df.out.cpu().numpy().any()
+    r.set_frame(fi.frame())
+    r.apply_caches(df.gbuffer(), df.out)
+    assert df.out.cpu().numpy().any()
+
+
 def test_allocation_reuses_address_volume_across_frames():
     """A renderer that allocates frame A, then frame B (a G-buffer with its
     upper half cleared and its lower half shifted), then A again holds the
