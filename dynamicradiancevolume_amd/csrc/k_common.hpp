@@ -8,6 +8,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <stddef.h>
 #include <stdint.h>
 
 #include "../../include/drv.h"
@@ -93,15 +94,17 @@ __device__ __forceinline__ int cascade_of(const drv_volume& vol, int n, f3 wp) {
 
 // The cascades in LDS, for lookups by lane: from the kernel's arguments each
 // would be a memory load on the way to the address volume.  pad0 holds
-// 1 / world_voxel_size.  The caller synchronises the workgroup (of 64 threads or
-// more).
+// 1 / world_voxel_size.  Every word has one writer, so the caller's barrier is
+// all the order they need; the workgroup has 64 threads or more.
 __device__ __forceinline__ void stage_cascades(const drv_volume& vol, drv_cascade* out) {
-  constexpr uint32_t kWords = sizeof(drv_cascade) / sizeof(uint32_t) * DRV_MAX_CASCADES;
-  static_assert(kWords <= 64u, "one word for each thread");
-  if (threadIdx.x < kWords)
-    reinterpret_cast<uint32_t*>(out)[threadIdx.x] = reinterpret_cast<const uint32_t*>(vol.cascades)[threadIdx.x];
-  __builtin_amdgcn_wave_barrier();  // the same wave's LDS stores stay in order
-  if (threadIdx.x < DRV_MAX_CASCADES) out[threadIdx.x].pad0 = 1.0f / vol.cascades[threadIdx.x].world_voxel_size;
+  constexpr uint32_t kWords = sizeof(drv_cascade) / sizeof(uint32_t);
+  static_assert(kWords * DRV_MAX_CASCADES <= 64u, "one word for each thread");
+  const uint32_t t = threadIdx.x, c = t / kWords;
+  if (t >= kWords * DRV_MAX_CASCADES) return;
+  const float inv = 1.0f / vol.cascades[c].world_voxel_size;
+  reinterpret_cast<uint32_t*>(out)[t] = t - c * kWords == offsetof(drv_cascade, pad0) / sizeof(uint32_t)
+                                            ? __float_as_uint(inv)
+                                            : reinterpret_cast<const uint32_t*>(vol.cascades)[t];
 }
 
 // Coordinate d (from the volume's corner) in cells of a staged cascade.

@@ -196,6 +196,44 @@ def test_apply_cell_edges_match_oracle(cav, cascades, size, width, height, sh):
         assert rel_l2(out, ref) < RGB_TOL
 
 
+def test_cascades_of_unrelated_cell_sizes_match_oracle():
+    """Four cascades whose cell sizes are neither powers of two nor multiples
+    of each other, all of them in a tile's view: every pixel looks its own
+    cascade up, in the allocation and in the apply."""
+    orc = _orc()
+    fi = frame_inputs("cornell_256", width=160, height=96)
+    over = dict(cav_resolution=24, cav_cascades=4, cascade0_world_size=1.0, sh_bands=2)
+    w = fi.workload.with_(**over)
+    cfg = w.config()
+    df = _device(fi)
+    announce("cascades of unrelated cell sizes")
+    r = _renderer(fi, **over)
+    r.set_frame(fi.frame())
+    r.update_volume(w.eye, fi.bbox[:3], fi.bbox[3:])
+    v = r.volume()
+    for c, half in enumerate((0.9, 2.3, 5.3, 9.7)):
+        k = v.cascades[c]
+        for i in range(3):
+            k.min[i], k.max[i] = w.eye[i] - half, w.eye[i] + half
+            k.decision_min[i], k.decision_max[i] = w.eye[i] - 0.8 * half, w.eye[i] + 0.8 * half
+        k.world_voxel_size = 2.0 * half / 24
+    r.set_volume(v)
+    r.voxelize_scene(df.positions, len(fi.positions))
+    r.allocate_caches(df.gbuffer())
+    count, cav, entries = orc.allocate(cfg, v, fi.frame(), fi.depth)
+    demanded, live = r.cache_count()
+    assert demanded == count
+    got, want = (canonical(count, *x, cfg.max_caches) for x in ((r.read_cav(), r.read_caches(live)), (cav, entries)))
+    assert got[3] and want[3] and got[2] == want[2]
+    np.testing.assert_array_equal(got[0], want[0])
+    np.testing.assert_array_equal(got[1], want[1])
+    r.light_caches_rsm(df.rsm(), fi.light)
+    r.apply_caches(df.gbuffer(), df.out)
+    ref = orc.apply(cfg, v, fi.frame(), orc.sh_constants(), fi, r.read_cav(), r.read_caches(live), live)
+    assert np.abs(ref).max() > 0.0
+    assert rel_l2(df.out.cpu().numpy(), ref) < RGB_TOL
+
+
 # Pixels that unproject to cells past the 32-bit range along one axis, the
 # others inside the volume, and to infinity: no cache is there to light them.
 @pytest.mark.parametrize("cascades", [1, 4])
