@@ -29,12 +29,23 @@ struct Counter {
 constexpr int kGatherTile = 64;    // caches per gather / cone-trace tile (one per lane)
 constexpr uint32_t kMaxSplits = 256;  // VPL splits of the SH gather (each at least 64 VPLs)
 
+// What a group of VPLs that light passes skip by its flux bits must hold: none is
+// odd.  Odd is a VPL with a position or disc area at or past these bounds, and
+// any NaN or infinity (half flux and depth have both): such a VPL counts for
+// every receiver, also for those it faces away from (infinity times zero), and
+// in the shader's order of operations.  No group of finite half fluxes has all
+// bits set.
+constexpr uint32_t kOddFlux = 0xffffffffu;
+constexpr float kFarPosition = 0x1p29f, kFarArea = 0x1p61f;
+
 // One VPL ("LightInfo", cacheLightingRSM.comp:34-40) packed for LDS staging.
 struct Vpl {
   float px, py, pz, disc_area;
   float fr, fg, fb;
-  uint32_t quad_flux;  // the bits of all flux of the aligned group of four VPLs or'ed: 0 = the group is dark
-  float nx, ny, nz, pad1;
+  uint32_t quad_flux;  // the bits of all flux of the aligned group of four VPLs or'ed: 0 = the group is dark;
+                       // kOddFlux: the group holds an odd VPL
+  float nx, ny, nz;
+  uint32_t wave_odd;  // not 0: the aligned group of 64 VPLs holds an odd one
 };
 
 // One shadow block (cacheLightingRSM.comp:171-192): averaged VAL position and

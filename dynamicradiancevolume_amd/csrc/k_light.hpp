@@ -88,8 +88,10 @@ __device__ __forceinline__ float block_aperture(const PrepArgs& a, const float d
 }
 
 // The VPL record m (and the shadow block record when m starts a block) of
-// the light in `a`, n = R^2 VPLs; every lane of a wave must call it with
-// m < n (n is a multiple of 64, so whole waves are in or out).
+// the light in `a`, n VPLs, one per lane in order.  Lanes at and past n do not call
+// it, so what neighbouring lanes exchange is whole where n holds whole groups of
+// them: quad_flux from n = 4 on (nothing reads it of fewer VPLs), the light
+// passes' units and blocks from their least n of 64 on.
 __device__ __forceinline__ void prepare_vpl(const PrepArgs& a, uint32_t m, uint32_t n) {
   uint32_t x, y;
   morton_decode(m, x, y);
@@ -112,15 +114,17 @@ __device__ __forceinline__ void prepare_vpl(const PrepArgs& a, uint32_t m, uint3
   // cacheLightingRSM.comp:240-243: with INDIRECT_SPECULAR a VAL whose flux
   // sums below 0.001 is skipped (`continue`); a zero flux adds nothing.
   if (a.flux_cut && (v.fr + v.fg) + v.fb < 0.001f) v.fr = v.fg = v.fb = 0.0f;
-  // Whether any VPL of the aligned group of four has flux (adjacent lanes).
-  uint32_t bits = __float_as_uint(v.fr) | __float_as_uint(v.fg) | __float_as_uint(v.fb);
+  // Whether any VPL of the aligned group of four has flux or is odd (adjacent lanes).
+  const bool odd = !(fabsf(v.px) < kFarPosition && fabsf(v.py) < kFarPosition && fabsf(v.pz) < kFarPosition &&
+                     fabsf(v.disc_area) < kFarArea && fabsf(v.fr) + fabsf(v.fg) + fabsf(v.fb) < kFarArea);
+  uint32_t bits = odd ? kOddFlux : __float_as_uint(v.fr) | __float_as_uint(v.fg) | __float_as_uint(v.fb);
   bits |= __shfl_xor(bits, 1);
   bits |= __shfl_xor(bits, 2);
   v.quad_flux = bits;
   v.nx = nrm.x;
   v.ny = nrm.y;
   v.nz = nrm.z;
-  v.pad1 = 0.0f;
+  v.wave_odd = __ballot(odd) != 0ull ? 1u : 0u;
   a.vpls[m] = v;
   if (a.vpl_units) {
     bits |= __shfl_xor(bits, 4);
