@@ -213,12 +213,14 @@ __device__ __forceinline__ void gather_quad(ShSums& acc, const Vpl* vpls, uint32
   }
   asm volatile("" : "+s"(p[0]), "+s"(p[1]), "+s"(p[2]), "+s"(p[3]), "+s"(f[0]), "+s"(f[1]), "+s"(f[2]), "+s"(f[3]),
                     "+s"(n[0]), "+s"(n[1]), "+s"(n[2]), "+s"(n[3]));
-  if (__float_as_uint(f[0].w) == 0u) return;  // Vpl::quad_flux
+  const uint32_t quad_flux = __float_as_uint(f[0].w);
+  if (quad_flux == 0u) return;
+  const uint64_t every = quad_flux == kOddFlux ? ~0ull : 0ull;  // an odd VPL counts whichever way it faces
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     const float tx = p[k].x - wx, ty = p[k].y - wy, tz = p[k].z - wz;
     const float nd = -__builtin_fmaf(n[k].z, tz, __builtin_fmaf(n[k].y, ty, n[k].x * tx));
-    if ((__ballot(nd > 0.0f) & lit[kUnit ? k : 0]) != 0ull)
+    if (((__ballot(nd > 0.0f) | every) & lit[kUnit ? k : 0]) != 0ull)
       sh_accumulate<kSh2>(acc, p[k].w, f[k].x, f[k].y, f[k].z, tx, ty, tz, nd, shadowing[kUnit ? k : 0]);
   }
 }
