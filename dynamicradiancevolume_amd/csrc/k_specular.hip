@@ -125,7 +125,8 @@ __global__ __launch_bounds__(256) void k_specular_gather(SpecGatherArgs a) {
           const bool in = u < u1;
           const uint32_t uc = in ? u : u0;
           const float sh = unit_shadowing(a, uc, c);
-          const bool lit = in && sh != 0.0f && __float_as_uint(fluxes[uc].w) != 0u;
+          const uint32_t flux = __float_as_uint(fluxes[uc].w);
+          const bool lit = in && ((sh != 0.0f && flux != 0u) || flux == kOddFlux);  // zero times an odd VAL counts
           const uint64_t m = __ballot(lit);
           const uint32_t at = queued + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32),
                                                                  __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0u));
