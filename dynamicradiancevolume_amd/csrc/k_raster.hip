@@ -274,7 +274,7 @@ __global__ __launch_bounds__(256) void k_raster_id_big(RasterArgs a) {
 // ---- the tiled raster ----------------------------------------------------
 //
 // For windows of many tiles.  Triangles are binned to the 16x16-pixel tiles
-// their pixel boxes touch (count, scan, fill); then one workgroup per tile
+// their pixel boxes touch (count, start, fill); then one workgroup per tile
 // keeps the tile's pixels in registers, one pixel per lane (a wave owns 8x8),
 // and walks the tile's triangles, 256 at a time: every thread sets up one
 // triangle in LDS, then every wave tests those that may touch it.  A pixel
@@ -283,6 +283,16 @@ __global__ __launch_bounds__(256) void k_raster_id_big(RasterArgs a) {
 // planes with an error margin whether all its pixels are outside or behind, the
 // wave then for its lanes; the FP64 test, with the operations of raster_piece,
 // runs when a lane is left.
+//
+// Triangles of more than kTileSpan tiles are records that every tile looks
+// through and gathers to whole batches.  Lists and records have fixed room
+// (tile_room): what finds none is drawn by the two passes above before the tiles,
+// whose pixels then start from that, so a scene past the room costs no more than
+// the two passes.  1920x1080 / 3840x2160, two passes for all of it and this:
+// 200000 triangles of some 50 tiles (twice the room) 5.4 / 5.4 and 0.32 / 0.62 ms,
+// 1.0M of some 30 (four times) 23 / 23 and 1.4 / 1.9, 30000 of 1000 tiles 8.2 / 8.6
+// and 0.89 / 2.8.  (With 4 n + 2^16 pairs and all others as records that each tile
+// took in batches of 256, hits or not: 8.5 / 15.9, 23 / 53 and 4.4 / 12.9 ms.)
 //
 // 1920x1080, 1.0M triangles in 2000 boxes (74M box pixels, 18 layers deep):
 // the two passes 1660 us, of it atomics and FP64 tests of hidden fragments;
@@ -306,17 +316,29 @@ struct TilePair {
 constexpr uint32_t kNoTile = 0xffffffffu;
 
 struct TileArgs {
-  RasterArgs r;
+  RasterArgs r;         // r.big: triangles that found no room
   int tiles_x, tiles_y;
   uint32_t capacity;    // pairs
-  uint32_t* head;       // {wide records, clipped triangles, pairs, records in lists}, then the counts
+  uint32_t wide_capacity, cut_capacity;  // records
+  uint32_t* head;       // {wide records, clipped triangles, pairs, records in lists, r.n_big, room taken by lists, 0, 0}, then the counts
   uint32_t* count;      // [tiles]
   uint32_t* start;      // [tiles]
   uint32_t* clip;       // [n_tri] triangles that reach behind the near plane
   TilePair* pairs;      // [capacity]
   uint32_t* lists;      // [capacity] items by tile
-  TileRecord* records;  // [2 n_tri] from the front the wide ones, which every tile looks at, from the back those in lists
+  TileRecord* wide;     // [wide_capacity] what every tile looks at
+  TileRecord* cut;      // [cut_capacity] what the lists hold of clipped triangles
 };
+constexpr uint32_t kHeadWords = 8;
+
+// A triangle without room in the lists or the records.
+__device__ __forceinline__ void leave_out(const TileArgs& a, uint32_t t) { a.r.big[atomicAdd(a.r.n_big, 1u)] = t; }
+// A triangle's piece for every tile to look at; false: no room.
+__device__ __forceinline__ bool add_wide(const TileArgs& a, const TileRecord& rec) {
+  const uint32_t i = atomicAdd(&a.head[0], 1u);
+  if (i < a.wide_capacity) a.wide[i] = rec;
+  return i < a.wide_capacity;
+}
 
 __device__ __forceinline__ TileRecord tile_record(const Setup& st, uint32_t t, uint32_t piece) {
   const uint32_t x0 = st.px0 / kTile, x1 = (st.px0 + st.bw - 1) / kTile;
@@ -386,12 +408,13 @@ __global__ __launch_bounds__(1024) void k_tile_count(TileArgs a) {
   first_y[threadIdx.x] = rec.y & 0xffffu;
   width[threadIdx.x] = (rec.x >> 16) - (rec.x & 0xffffu) + 1u;
   __syncthreads();
+  bool out = big && !add_wide(a, rec);
   if (sum != 0u && (group_base > a.capacity || sum > a.capacity - group_base)) {
-    // Triangles whose pairs would pass the capacity are left to the records.
     if (threadIdx.x == 0u) drop_pairs(a, group_base, sum);
-    big = big || tiles != 0u;
+    out = out || tiles != 0u;
     sum = 0u;
   }
+  if (out) leave_out(a, t);
   for (uint32_t i0 = 0; i0 < sum; i0 += 1024u) {
     // Pair i: the first thread whose pairs end behind it, then its tile.
     const uint32_t i = i0 + threadIdx.x;
@@ -419,7 +442,6 @@ __global__ __launch_bounds__(1024) void k_tile_count(TileArgs a) {
     before = __shfl(before, static_cast<int>(leader));
     if (on) a.pairs[group_base + i] = TilePair{blockIdx.x * 1024u + owner, tile, before + rank};
   }
-  if (big) a.records[atomicAdd(&a.head[0], 1u)] = rec;
 }
 
 // The pieces of triangles cut by the near plane.
@@ -429,61 +451,74 @@ __global__ __launch_bounds__(256) void k_tile_clip(TileArgs a) {
     const uint32_t t = a.clip[i];
     ScreenTri sc[2];
     const int m = project_clip(a.r.positions + 9 * static_cast<size_t>(t), a.r.vp, a.r.w, a.r.h, sc);
+    bool out = false;  // whole, though one piece may be in the lists: the same fragments
     for (int k = 0; k < m; ++k) {
       const Setup st = setup_piece(sc[k], a.r.w, a.r.h);
       if (!st.ok) continue;
       const TileRecord rec = tile_record(st, t, static_cast<uint32_t>(k));
       const uint32_t tiles = list_tiles(rec);
-      uint32_t slot = tiles != 0u ? atomicAdd(&a.head[2], tiles) : 0u;
-      if (tiles == 0u || slot > a.capacity || tiles > a.capacity - slot) {
-        drop_pairs(a, slot, tiles);
-        a.records[atomicAdd(&a.head[0], 1u)] = rec;
+      if (tiles == 0u) {
+        out = !add_wide(a, rec) || out;
         continue;
       }
-      const uint32_t r = 2u * a.r.n_tri - 1u - atomicAdd(&a.head[3], 1u);
-      a.records[r] = rec;
+      uint32_t slot = atomicAdd(&a.head[2], tiles);
+      const bool fits = slot <= a.capacity && tiles <= a.capacity - slot;
+      const uint32_t r = fits ? atomicAdd(&a.head[3], 1u) : a.cut_capacity;
+      if (r >= a.cut_capacity) {
+        drop_pairs(a, slot, tiles);
+        out = true;
+        continue;
+      }
+      a.cut[r] = rec;
       for (uint32_t y = rec.y & 0xffffu; y <= rec.y >> 16; ++y)
         for (uint32_t x = rec.x & 0xffffu; x <= rec.x >> 16; ++x, ++slot) {
           const uint32_t tile = y * static_cast<uint32_t>(a.tiles_x) + x;
           a.pairs[slot] = TilePair{kRecordItem | r, tile, atomicAdd(&a.count[tile], 1u)};
         }
     }
+    if (out) leave_out(a, t);
   }
 }
 
-// Where each tile's list begins: exclusive scan of the counts, one workgroup.
-__global__ __launch_bounds__(1024) void k_tile_scan(TileArgs a) {
-  __shared__ uint32_t wave_total[16];
-  const uint32_t n = static_cast<uint32_t>(a.tiles_x) * static_cast<uint32_t>(a.tiles_y);
-  const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
-  uint32_t carry = 0;
-  for (uint32_t i0 = 0; i0 < n; i0 += 1024u) {
-    const uint32_t i = i0 + threadIdx.x;
-    const uint32_t c = i < n ? a.count[i] : 0u;
-    uint32_t s = c;
-    for (int o = 1; o < 64; o <<= 1) {
-      const uint32_t u = __shfl_up(s, o);
-      if (static_cast<int>(lane) >= o) s += u;
+// Where each tile's list begins, in any order of the tiles: a wave takes the room
+// of its 64 at once (one workgroup that scanned all counts took 9 us at 1920x1080
+// and 25 at 3840x2160).  The workgroups after those of the tiles empty the pixels
+// if triangles are left to the two passes.
+__global__ __launch_bounds__(256) void k_tile_start(TileArgs a) {
+  const uint32_t n = static_cast<uint32_t>(a.tiles_x) * static_cast<uint32_t>(a.tiles_y), groups = (n + 255u) / 256u;
+  if (blockIdx.x >= groups) {
+    if (*a.r.n_big == 0u) return;
+    const size_t pixels = static_cast<size_t>(a.r.w) * a.r.h, step = (gridDim.x - groups) * size_t(256);
+    for (size_t i = (blockIdx.x - groups) * size_t(256) + threadIdx.x; i < pixels; i += step) {
+      a.r.zbits[i] = 0ull;
+      a.r.tri[i] = 0xffffffffu;
     }
-    if (lane == 63u) wave_total[w] = s;
-    __syncthreads();
-    uint32_t before = carry, all = 0;
-    for (uint32_t k = 0; k < 16u; ++k) {
-      before += k < w ? wave_total[k] : 0u;
-      all += wave_total[k];
-    }
-    if (i < n) a.start[i] = before + s - c;
-    carry += all;
-    __syncthreads();
+    return;
   }
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x, lane = threadIdx.x & 63u;
+  const uint32_t c = i < n ? a.count[i] : 0u;
+  uint32_t upto = c;
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t u = __shfl_up(upto, o);
+    if (static_cast<int>(lane) >= o) upto += u;
+  }
+  uint32_t base = 0u;
+  if (lane == 63u) base = atomicAdd(&a.head[5], upto);
+  base = __shfl(base, 63);
+  if (i < n) a.start[i] = base + upto - c;
 }
 
+// The pairs into the tiles' lists, and the depth pass of the triangles left to
+// the two passes.
 __global__ __launch_bounds__(256) void k_tile_fill(TileArgs a) {
   const uint32_t n = min(a.head[2], a.capacity);
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
     const TilePair p = a.pairs[i];
     if (p.tile != kNoTile) a.lists[a.start[p.tile] + p.rank] = p.item;
   }
+  raster_big(a.r, [&](uint32_t, size_t i, double z) {
+    atomicMax(&a.r.zbits[i], static_cast<unsigned long long>(__double_as_longlong(z)));
+  });
 }
 
 // A batch of triangles in LDS: what raster_piece reads, and FP32 planes
@@ -500,7 +535,10 @@ struct TileBatch {
   uint2 box_tri[256];   // columns | rows << 16 of the tile inside the pixel box; index
   float zmax[4][256];   // above every depth in the wave's 8x8 pixels
   uint8_t touch[256];   // bit per wave: may cover a pixel of it
+  uint16_t queue[512];  // wide records that touch the tile
+  uint16_t found[4];
 };
+static_assert(sizeof(TileBatch) <= 40960, "four workgroups on a CU");
 
 // g bounds the terms that c and the FP64 test were summed from.
 __device__ __forceinline__ void tile_plane(float* out, double a, double b, double c, double g) {
@@ -580,37 +618,60 @@ __global__ __launch_bounds__(256, 4) void k_tile_raster(TileArgs a) {
   const float fx = static_cast<float>(lx) + 0.5f, fy = static_cast<float>(ly) + 0.5f;
   const uint32_t bit = (1u << lx) | (0x10000u << ly);
   double z = 0.0;                      // a fragment must beat the cleared depth 0
-  float zlow = inside ? 0.0f : 1e38f;  // below z
   uint32_t id = 0xffffffffu;
+  const size_t pixel = static_cast<size_t>(py) * a.r.w + px;
+  if (*a.r.n_big != 0u && inside) {  // what the two passes drew
+    z = __longlong_as_double(static_cast<long long>(a.r.zbits[pixel]));
+    id = a.r.tri[pixel];
+  }
+  float zlow = inside ? static_cast<float>(z) * (1.0f - 0x1p-20f) : 1e38f;  // below z
 
-  // First the wide records, then the tile's list.
-  const uint32_t n_wide = a.head[0], wide_span = (n_wide + 255u) & ~255u;
+  // First the wide records, gathered to whole batches, then the tile's list.
+  const uint32_t n_wide = min(a.head[0], a.wide_capacity);
   const uint32_t begin = a.start[blockIdx.x], n_list = a.count[blockIdx.x];
-  for (uint32_t i0 = 0; i0 < wide_span + n_list; i0 += 256u) {
-    const uint32_t i = i0 + tid;
-    uint32_t item = 0u, piece = 2u;
-    bool valid;
-    if (i0 < wide_span) {
-      valid = i < n_wide;
-      if (valid) {
-        const TileRecord rec = a.records[i];
+  uint32_t looked = 0u, queued = 0u, taken = 0u;
+  while (looked < n_wide || queued != 0u || taken < n_list) {
+    while (looked < n_wide && queued < 256u) {
+      const uint32_t i = looked + tid;
+      bool hit = i < n_wide;
+      if (hit) {
+        const TileRecord rec = a.wide[i];
         const uint32_t tx = static_cast<uint32_t>(tile_x), ty = static_cast<uint32_t>(tile_y);
-        valid = tx >= (rec.x & 0xffffu) && tx <= (rec.x >> 16) && ty >= (rec.y & 0xffffu) && ty <= (rec.y >> 16);
+        hit = tx >= (rec.x & 0xffffu) && tx <= (rec.x >> 16) && ty >= (rec.y & 0xffffu) && ty <= (rec.y >> 16);
+      }
+      looked += 256u;
+      if (!__syncthreads_or(hit)) continue;
+      const uint64_t hits = __ballot(hit);
+      if (lane == 0u) e.found[w] = static_cast<uint16_t>(__popcll(hits));
+      __syncthreads();
+      uint32_t at = queued + static_cast<uint32_t>(__popcll(hits & ((1ull << lane) - 1ull)));
+#pragma unroll
+      for (uint32_t k = 0; k < 4u; ++k) {
+        at += k < w ? e.found[k] : 0u;
+        queued += e.found[k];
+      }
+      if (hit) e.queue[at] = static_cast<uint16_t>(i);
+      __syncthreads();
+    }
+    const uint32_t n_queue = min(queued, 256u), n_items = min(256u - n_queue, n_list - taken);
+    const bool from_queue = tid < n_queue, valid = tid < n_queue + n_items;
+    uint32_t item = 0u, piece = 2u;
+    uint16_t left = 0u;
+    if (valid) {
+      if (!from_queue) item = a.lists[begin + taken + (tid - n_queue)];
+      if (from_queue || (item & kRecordItem)) {
+        const TileRecord rec = from_queue ? a.wide[e.queue[tid]] : a.cut[item & ~kRecordItem];
         item = rec.tri;
         piece = rec.piece;
       }
-      if (!__syncthreads_or(valid)) continue;
-    } else {
-      valid = i - wide_span < n_list;
-      if (valid) {
-        item = a.lists[begin + (i - wide_span)];
-        if (item & kRecordItem) {
-          const TileRecord rec = a.records[item & ~kRecordItem];
-          item = rec.tri;
-          piece = rec.piece;
-        }
-      }
     }
+    taken += n_items;
+    if (queued > 256u) {  // what is left of the queue moves up
+      left = e.queue[256u + tid];
+      __syncthreads();
+      e.queue[tid] = left;
+    }
+    queued -= n_queue;
     uint32_t touch = 0u;
     if (valid) {
       ScreenTri q;
@@ -660,9 +721,8 @@ __global__ __launch_bounds__(256, 4) void k_tile_raster(TileArgs a) {
     __syncthreads();
   }
   if (!inside) return;
-  const size_t o = static_cast<size_t>(py) * a.r.w + px;
-  a.r.zbits[o] = static_cast<unsigned long long>(__double_as_longlong(z));
-  a.r.tri[o] = id;
+  a.r.zbits[pixel] = static_cast<unsigned long long>(__double_as_longlong(z));
+  a.r.tri[pixel] = id;
 }
 
 // ---- formats (bit-exact restatements of the host producer's) ------------
@@ -922,7 +982,21 @@ int tile_count(int w, int h) { return ((w + kTile - 1) / kTile) * ((h + kTile - 
 bool tiled(int w, int h, uint32_t n_tri) {
   return tile_count(w, h) >= kMinTiles && w <= 65536 && h <= 65536 && n_tri <= (1u << 24);
 }
-uint32_t pair_capacity(uint32_t n_tri) { return 4u * n_tri + 65536u; }
+
+// Room of the tiled raster's lists and records; what passes it is drawn by the
+// two passes before the tiles.
+struct TileRoom {
+  uint32_t pairs, wide, cut;
+};
+TileRoom tile_room(int w, int h, uint32_t n_tri) {
+  constexpr uint64_t kWideLooks = 1u << 30;  // of all tiles at wide records: ~1 ms
+  const uint64_t n = n_tri, tiles = static_cast<uint64_t>(tile_count(w, h));
+  TileRoom r;
+  r.pairs = static_cast<uint32_t>(std::min<uint64_t>(2 * kTileSpan * n, 4 * n + (1u << 22)));
+  r.cut = static_cast<uint32_t>(std::min<uint64_t>(2 * n, 65536));
+  r.wide = static_cast<uint32_t>(std::min<uint64_t>({2 * n, 65536, std::max<uint64_t>(256, kWideLooks / tiles)}));
+  return r;
+}
 
 // Depth and winning triangle of every pixel into zbits / tri; work: the
 // raster's lists (raster_work_words).
@@ -945,21 +1019,30 @@ void raster(const float* positions, uint32_t n_tri, const float* vp, int w, int 
     t.tiles_x = (w + kTile - 1) / kTile;
     t.tiles_y = (h + kTile - 1) / kTile;
     const size_t tiles = static_cast<size_t>(t.tiles_x) * t.tiles_y, n = n_tri;
-    t.capacity = pair_capacity(n_tri);
-    t.records = reinterpret_cast<TileRecord*>(work);
-    t.head = work + 8 * n;
-    t.count = t.head + 4;
+    const TileRoom room = tile_room(w, h, n_tri);
+    t.capacity = room.pairs;
+    t.wide_capacity = room.wide;
+    t.cut_capacity = room.cut;
+    t.wide = reinterpret_cast<TileRecord*>(work);
+    t.cut = t.wide + room.wide;
+    t.head = reinterpret_cast<uint32_t*>(t.cut + room.cut);
+    t.count = t.head + kHeadWords;
     t.start = t.count + tiles;
     t.clip = t.start + tiles;
     t.lists = t.clip + n;
     t.pairs = reinterpret_cast<TilePair*>(t.lists + t.capacity);
-    launch_fill_u32(t.head, 4 + tiles, 0u, s);
+    t.r.n_big = t.head + 4;
+    t.r.big = reinterpret_cast<uint32_t*>(t.pairs + t.capacity);
+    // Everything fits that could come: no triangle is left to the two passes.
+    const bool roomy = room.pairs == 2 * kTileSpan * n && room.wide == 2 * n && room.cut == 2 * n;
+    launch_fill_u32(t.head, kHeadWords + tiles, 0u, s);
     if (n_tri != 0) {
       hipLaunchKernelGGL(k_tile_count, dim3((n_tri + 1023) / 1024), dim3(1024), 0, s, t);
       hipLaunchKernelGGL(k_tile_clip, dim3(256), dim3(256), 0, s, t);
     }
-    hipLaunchKernelGGL(k_tile_scan, dim3(1), dim3(1024), 0, s, t);
+    hipLaunchKernelGGL(k_tile_start, dim3(static_cast<unsigned>((tiles + 255) / 256) + (roomy ? 0 : 1024)), dim3(256), 0, s, t);
     if (n_tri != 0) hipLaunchKernelGGL(k_tile_fill, dim3(1024), dim3(256), 0, s, t);
+    if (!roomy) hipLaunchKernelGGL(k_raster_id_big, dim3(1024), dim3(256), 0, s, t.r);
     hipLaunchKernelGGL(k_tile_raster, dim3(static_cast<unsigned>(tiles)), dim3(256), 0, s, t);
     return;
   }
@@ -977,8 +1060,9 @@ void raster(const float* positions, uint32_t n_tri, const float* vp, int w, int 
 
 size_t raster_work_words(int w, int h, uint32_t n_tri) {
   if (!tiled(w, h, n_tri)) return static_cast<size_t>(n_tri) + 1;
-  return 9 * static_cast<size_t>(n_tri) + 4 + 2 * static_cast<size_t>(tile_count(w, h)) +
-         4 * static_cast<size_t>(pair_capacity(n_tri));
+  const TileRoom room = tile_room(w, h, n_tri);
+  return kHeadWords + 2 * static_cast<size_t>(n_tri) + 2 * static_cast<size_t>(tile_count(w, h)) +
+         4 * (static_cast<size_t>(room.pairs) + room.wide + room.cut);
 }
 
 void launch_render_gbuffer(const float* positions, const float* albedo, const float* normals, uint32_t n_tri,
