@@ -14,6 +14,7 @@
 #include "../../include/drv.h"
 #include "drv_internal.hpp"
 #include "mat4.hpp"
+#include "raster_room.hpp"
 #include "split_plan.hpp"
 
 using drvk::Counter;
@@ -128,6 +129,7 @@ struct drv_ctx {
   uint32_t* rtri = nullptr;
   uint32_t* rwork = nullptr;  // the raster's triangle lists
   size_t raster_cap = 0, raster_tri_cap = 0, rwork_cap = 0;
+  size_t rwork_refused = ~size_t{0};  // the least words of lists that did not fit
   float* g_depth = nullptr;
   int16_t* g_normal = nullptr;
   uint8_t* g_albedo = nullptr;
@@ -1094,8 +1096,14 @@ int ensure_raster(drv_ctx* ctx, int w, int h, uint32_t n_tri) {
   const size_t pixels = static_cast<size_t>(w) * h;
   int rc;
   if ((rc = ensure(ctx, &ctx->rz, &ctx->raster_cap, pixels)) != DRV_OK) return rc;
-  if ((rc = ensure(ctx, &ctx->rwork, &ctx->rwork_cap, drvk::raster_work_words(w, h, n_tri))) != DRV_OK) return rc;
-  return ensure(ctx, &ctx->rtri, &ctx->raster_tri_cap, pixels);
+  if ((rc = ensure(ctx, &ctx->rtri, &ctx->raster_tri_cap, pixels)) != DRV_OK) return rc;
+  const size_t least = drvk::raster_least_words(n_tri);
+  return drvk::reserve_raster_words(
+      drvk::raster_work_words(w, h, n_tri), least, &ctx->rwork_refused, DRV_ERR_NO_MEMORY, [&](size_t words) {
+        const int code = ensure(ctx, &ctx->rwork, &ctx->rwork_cap, words);
+        if (code != DRV_OK && words != least) (void)hipGetLastError();
+        return code;
+      });
 }
 
 bool valid_scene(const drv_scene* s) {
@@ -1116,7 +1124,8 @@ int drv_render_gbuffer(drv_ctx* ctx, const drv_scene* scene, const float view_pr
     if ((rc = dev_alloc(ctx, &ctx->g_albedo, 3 * n)) != DRV_OK) return rc;
   }
   drvk::launch_render_gbuffer(scene->positions, scene->albedo, scene->normals, scene->n_tri, view_projection, w, h,
-                              ctx->rz, ctx->rtri, ctx->rwork, ctx->g_depth, ctx->g_normal, ctx->g_albedo, ctx->stream);
+                              ctx->rz, ctx->rtri, ctx->rwork, ctx->rwork_cap, ctx->g_depth, ctx->g_normal,
+                              ctx->g_albedo, ctx->stream);
   out->depth = ctx->g_depth;
   out->normal = ctx->g_normal;
   out->albedo = ctx->g_albedo;
@@ -1141,7 +1150,7 @@ int drv_render_rsm(drv_ctx* ctx, const drv_scene* scene, const drv_spot_light* l
   if ((rc = ensure(ctx, &ctx->rsm_dls, &ctx->rsm_dls_cap, 2 * chain)) != DRV_OK) return rc;
   if ((rc = ensure(ctx, &ctx->rsm_shadow, &ctx->rsm_shadow_cap, static_cast<size_t>(res) * res)) != DRV_OK) return rc;
   drvk::launch_render_rsm(scene->positions, scene->albedo, scene->normals, scene->n_tri, *light, ctx->rz, ctx->rtri,
-                          ctx->rwork, ctx->rsm_flux, ctx->rsm_normal, ctx->rsm_dls, ctx->rsm_shadow, ctx->stream);
+                          ctx->rwork, ctx->rwork_cap, ctx->rsm_flux, ctx->rsm_normal, ctx->rsm_dls, ctx->rsm_shadow, ctx->stream);
   ctx->rsm_res = res;
   // Level l starts after the texels of levels 0..l-1.
   const int read_lod = log2i(res / light->rsm_read_resolution);

@@ -333,14 +333,16 @@ void launch_spot_select(const Counter* counter, uint32_t k, const float* caches,
 void launch_spot_error(const float* spot, uint32_t spot_cap, int stride, int sh_bands, const Counter* spot_ctr,
                        float threshold, const Counter* counter, uint32_t* stats, Counter* gate, hipStream_t s);
 
-// uint32 of the raster's work lists (`work` below, 16-byte aligned) for a w x h window.
-size_t raster_work_words(int w, int h, uint32_t n_tri);
+// work: the raster's lists (16-byte aligned, raster_room.hpp); with fewer
+// work_words than the tiles take, at least raster_least_words, in two passes.
 void launch_render_gbuffer(const float* positions, const float* albedo, const float* normals, uint32_t n_tri,
                            const float* view_proj, int w, int h, unsigned long long* zbits, uint32_t* tri,
-                           uint32_t* work, float* depth, int16_t* normal, uint8_t* albedo_srgb, hipStream_t s);
+                           uint32_t* work, size_t work_words, float* depth, int16_t* normal, uint8_t* albedo_srgb,
+                           hipStream_t s);
 void launch_render_rsm(const float* positions, const float* albedo, const float* normals, uint32_t n_tri,
                        const drv_spot_light& light, unsigned long long* zbits, uint32_t* tri, uint32_t* work,
-                       uint16_t* flux, int16_t* normal, uint16_t* dls, float* shadow, hipStream_t s);
+                       size_t work_words, uint16_t* flux, int16_t* normal, uint16_t* dls, float* shadow,
+                       hipStream_t s);
 void launch_direct(const drv_config& cfg, const drv_frame& frame, const drv_spot_light& light, const drv_gbuffer& gb,
                    const uint8_t* roughness_metallic, const float* srgb_lut, const float* shadow, int shadow_res,
                    float normal_offset, float bias, float* out_rgb, int accumulate, hipStream_t s);

@@ -18,6 +18,7 @@
 
 #include "drv_internal.hpp"
 #include "k_common.hpp"
+#include "raster_room.hpp"
 
 namespace drvk {
 namespace {
@@ -299,8 +300,6 @@ __global__ __launch_bounds__(256) void k_raster_id_big(RasterArgs a) {
 // count 47, near-plane pieces 11, scan 9, fill 8, tiles 129 us, bound by vector
 // instructions (60 % of the cycles issue one, four waves on a SIMD).
 
-constexpr int kTile = 16;
-constexpr uint32_t kTileSpan = 64;  // triangles that touch more tiles go to the records that every tile looks through
 constexpr int kTileGroups = 16;     // tiles of which a wave adds up the pairs before its atomics
 
 struct TileRecord {
@@ -329,7 +328,6 @@ struct TileArgs {
   TileRecord* wide;     // [wide_capacity] what every tile looks at
   TileRecord* cut;      // [cut_capacity] what the lists hold of clipped triangles
 };
-constexpr uint32_t kHeadWords = 8;
 
 // A triangle without room in the lists or the records.
 __device__ __forceinline__ void leave_out(const TileArgs& a, uint32_t t) { a.r.big[atomicAdd(a.r.n_big, 1u)] = t; }
@@ -969,39 +967,10 @@ __global__ __launch_bounds__(256) void k_rsm_downsample(int res, int levels, uin
   }
 }
 
-// Windows of at least this many tiles take the tiled raster: a tile is one
-// workgroup's work, and a small window's few tiles hold many triangles each
-// and leave the chip idle.  1.0M triangles, tiled / two passes: 306 / 228 us at
-// 256x256 (256 tiles; an RSM 439 / 111), 238 / 424 at 480x270 (510), 191 / 684 at
-// 640x360, 259 / 1907 at 1920x1080; 2176 large triangles: 43 / 58, 47 / 65,
-// 54 / 74, 165 / 335.
-constexpr int kMinTiles = 384;
-
-int tile_count(int w, int h) { return ((w + kTile - 1) / kTile) * ((h + kTile - 1) / kTile); }
-// Tile coordinates have 12 bits, and the pairs of 2^24 triangles count in 32.
-bool tiled(int w, int h, uint32_t n_tri) {
-  return tile_count(w, h) >= kMinTiles && w <= 65536 && h <= 65536 && n_tri <= (1u << 24);
-}
-
-// Room of the tiled raster's lists and records; what passes it is drawn by the
-// two passes before the tiles.
-struct TileRoom {
-  uint32_t pairs, wide, cut;
-};
-TileRoom tile_room(int w, int h, uint32_t n_tri) {
-  constexpr uint64_t kWideLooks = 1u << 30;  // of all tiles at wide records: ~1 ms
-  const uint64_t n = n_tri, tiles = static_cast<uint64_t>(tile_count(w, h));
-  TileRoom r;
-  r.pairs = static_cast<uint32_t>(std::min<uint64_t>(2 * kTileSpan * n, 4 * n + (1u << 22)));
-  r.cut = static_cast<uint32_t>(std::min<uint64_t>(2 * n, 65536));
-  r.wide = static_cast<uint32_t>(std::min<uint64_t>({2 * n, 65536, std::max<uint64_t>(256, kWideLooks / tiles)}));
-  return r;
-}
-
 // Depth and winning triangle of every pixel into zbits / tri; work: the
-// raster's lists (raster_work_words).
+// raster's lists, of raster_work_words or else for two passes.
 void raster(const float* positions, uint32_t n_tri, const float* vp, int w, int h, unsigned long long* zbits,
-            uint32_t* tri, uint32_t* work, hipStream_t s) {
+            uint32_t* tri, uint32_t* work, size_t work_words, hipStream_t s) {
   RasterArgs a;
   a.positions = positions;
   a.n_tri = n_tri;
@@ -1013,7 +982,7 @@ void raster(const float* positions, uint32_t n_tri, const float* vp, int w, int 
   a.n_big = work;  // work[0] counts, the list follows
   a.big = work + 1;
   const dim3 grid((n_tri + 255) / 256);
-  if (tiled(w, h, n_tri)) {
+  if (tiled(w, h, n_tri) && work_words >= raster_work_words(w, h, n_tri)) {
     TileArgs t;
     t.r = a;
     t.tiles_x = (w + kTile - 1) / kTile;
@@ -1033,16 +1002,14 @@ void raster(const float* positions, uint32_t n_tri, const float* vp, int w, int 
     t.pairs = reinterpret_cast<TilePair*>(t.lists + t.capacity);
     t.r.n_big = t.head + 4;
     t.r.big = reinterpret_cast<uint32_t*>(t.pairs + t.capacity);
-    // Everything fits that could come: no triangle is left to the two passes.
-    const bool roomy = room.pairs == 2 * kTileSpan * n && room.wide == 2 * n && room.cut == 2 * n;
     launch_fill_u32(t.head, kHeadWords + tiles, 0u, s);
     if (n_tri != 0) {
       hipLaunchKernelGGL(k_tile_count, dim3((n_tri + 1023) / 1024), dim3(1024), 0, s, t);
       hipLaunchKernelGGL(k_tile_clip, dim3(256), dim3(256), 0, s, t);
     }
-    hipLaunchKernelGGL(k_tile_start, dim3(static_cast<unsigned>((tiles + 255) / 256) + (roomy ? 0 : 1024)), dim3(256), 0, s, t);
+    hipLaunchKernelGGL(k_tile_start, dim3(static_cast<unsigned>((tiles + 255) / 256) + (room.all ? 0 : 1024)), dim3(256), 0, s, t);
     if (n_tri != 0) hipLaunchKernelGGL(k_tile_fill, dim3(1024), dim3(256), 0, s, t);
-    if (!roomy) hipLaunchKernelGGL(k_raster_id_big, dim3(1024), dim3(256), 0, s, t.r);
+    if (!room.all) hipLaunchKernelGGL(k_raster_id_big, dim3(1024), dim3(256), 0, s, t.r);
     hipLaunchKernelGGL(k_tile_raster, dim3(static_cast<unsigned>(tiles)), dim3(256), 0, s, t);
     return;
   }
@@ -1058,17 +1025,11 @@ void raster(const float* positions, uint32_t n_tri, const float* vp, int w, int 
 
 }  // namespace
 
-size_t raster_work_words(int w, int h, uint32_t n_tri) {
-  if (!tiled(w, h, n_tri)) return static_cast<size_t>(n_tri) + 1;
-  const TileRoom room = tile_room(w, h, n_tri);
-  return kHeadWords + 2 * static_cast<size_t>(n_tri) + 2 * static_cast<size_t>(tile_count(w, h)) +
-         4 * (static_cast<size_t>(room.pairs) + room.wide + room.cut);
-}
-
 void launch_render_gbuffer(const float* positions, const float* albedo, const float* normals, uint32_t n_tri,
                            const float* view_proj, int w, int h, unsigned long long* zbits, uint32_t* tri,
-                           uint32_t* work, float* depth, int16_t* normal, uint8_t* albedo_srgb, hipStream_t s) {
-  raster(positions, n_tri, view_proj, w, h, zbits, tri, work, s);
+                           uint32_t* work, size_t work_words, float* depth, int16_t* normal, uint8_t* albedo_srgb,
+                           hipStream_t s) {
+  raster(positions, n_tri, view_proj, w, h, zbits, tri, work, work_words, s);
   GbufArgs a;
   a.w = w;
   a.h = h;
@@ -1085,9 +1046,10 @@ void launch_render_gbuffer(const float* positions, const float* albedo, const fl
 
 void launch_render_rsm(const float* positions, const float* albedo, const float* normals, uint32_t n_tri,
                        const drv_spot_light& light, unsigned long long* zbits, uint32_t* tri, uint32_t* work,
-                       uint16_t* flux, int16_t* normal, uint16_t* dls, float* shadow, hipStream_t s) {
+                       size_t work_words, uint16_t* flux, int16_t* normal, uint16_t* dls, float* shadow,
+                       hipStream_t s) {
   const int res = light.rsm_render_resolution;
-  raster(positions, n_tri, light.light_view_projection, res, res, zbits, tri, work, s);
+  raster(positions, n_tri, light.light_view_projection, res, res, zbits, tri, work, work_words, s);
   RsmArgs a;
   a.res = res;
   a.zbits = zbits;
