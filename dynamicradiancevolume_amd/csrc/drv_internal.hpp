@@ -45,7 +45,8 @@ struct Vpl {
   uint32_t quad_flux;  // the bits of all flux of the aligned group of four VPLs or'ed: 0 = the group is dark;
                        // kOddFlux: the group holds an odd VPL
   float nx, ny, nz;
-  uint32_t wave_odd;  // not 0: the aligned group of 64 VPLs holds an odd one
+  float least_cos;  // receivers count whose unnormalized cosine is not at most this: 0, for an odd VPL NaN (all
+                    // count); bits other than +0's: the aligned group of 64 VPLs holds an odd one
 };
 
 // One shadow block (cacheLightingRSM.comp:171-192): averaged VAL position and

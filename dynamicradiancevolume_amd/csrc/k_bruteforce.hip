@@ -170,7 +170,7 @@ __global__ __launch_bounds__(256) void k_bruteforce(BruteArgs a) {
     const ValRecord vals = (ValRecord)(a.vals);  // NOLINT(old-style-cast)
     const bool far = !(fabsf(wp.x) < kFarPosition && fabsf(wp.y) < kFarPosition && fabsf(wp.z) < kFarPosition);
     bool odd = false;
-    for (uint32_t k = g0 / 16u + lane; k < (g1 + 15u) / 16u; k += 64u) odd |= a.vals[64u * k].wave_odd != 0u;
+    for (uint32_t k = g0 / 16u + lane; k < (g1 + 15u) / 16u; k += 64u) odd |= __float_as_uint(a.vals[64u * k].least_cos) != 0u;
     const bool any_far = __ballot(far) != 0ull;
     // Two loops, so that the ordinary one pays nothing for the odd groups: 7.61 ms
     // without them and 7.59 with, 8.6 with both kinds in one loop (1920x1080 x

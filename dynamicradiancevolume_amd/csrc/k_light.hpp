@@ -124,7 +124,8 @@ __device__ __forceinline__ void prepare_vpl(const PrepArgs& a, uint32_t m, uint3
   v.nx = nrm.x;
   v.ny = nrm.y;
   v.nz = nrm.z;
-  v.wave_odd = __ballot(odd) != 0ull ? 1u : 0u;
+  const uint64_t any_odd = __ballot(odd);
+  v.least_cos = odd ? __builtin_nanf("") : any_odd != 0ull ? -0.0f : 0.0f;
   a.vpls[m] = v;
   if (a.vpl_units) {
     bits |= __shfl_xor(bits, 4);
@@ -192,9 +193,9 @@ typedef const __attribute__((address_space(4))) float4v* VplRecord;  // 3 per VP
 // Four VPLs first .. first + 3 for the 64 caches of a wave; shadowing[k] is
 // VPL k's and lit[k] holds the lanes it may reach (kUnit; otherwise the four
 // share shadowing[0] and lit[0], one shadow block's).  A VPL whose front faces
-// none of those lanes adds exact zeros (finite flux and distances) and is
-// skipped after the sign of its cosine, as are four VPLs without flux: the
-// RSM's texels outside the light's cone.  Of a wave's (64 caches x VPL) steps
+// none of those lanes adds exact zeros and is skipped after the sign of its
+// cosine (Vpl::least_cos: unless its flux or distance is not finite), as are four
+// VPLs without flux: the RSM's texels outside the light's cone.  Of a wave's (64 caches x VPL) steps
 // that its shadow blocks leave, 29 of 60 % remain on boxes_1080p, 19 of 48 % on
 // boxes_1080p_dense (a step is 48 VALU instructions, the test 7); the kernel
 // went from 99 to 62 and from 796 to 325 us with the item order of k_gather.
@@ -211,16 +212,14 @@ __device__ __forceinline__ void gather_quad(ShSums& acc, const Vpl* vpls, uint32
     f[k] = r[3 * k + 1];
     n[k] = r[3 * k + 2];
   }
-  asm volatile("" : "+s"(p[0]), "+s"(p[1]), "+s"(p[2]), "+s"(p[3]), "+s"(f[0]), "+s"(f[1]), "+s"(f[2]), "+s"(f[3]),
-                    "+s"(n[0]), "+s"(n[1]), "+s"(n[2]), "+s"(n[3]));
-  const uint32_t quad_flux = __float_as_uint(f[0].w);
-  if (quad_flux == 0u) return;
-  const uint64_t every = quad_flux == kOddFlux ? ~0ull : 0ull;  // an odd VPL counts whichever way it faces
+  asm volatile("" ::"s"(p[0]), "s"(p[1]), "s"(p[2]), "s"(p[3]), "s"(f[0]), "s"(f[1]), "s"(f[2]), "s"(f[3]), "s"(n[0]),
+               "s"(n[1]), "s"(n[2]), "s"(n[3]));
+  if (__float_as_uint(f[0].w) == 0u) return;  // Vpl::quad_flux
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     const float tx = p[k].x - wx, ty = p[k].y - wy, tz = p[k].z - wz;
     const float nd = -__builtin_fmaf(n[k].z, tz, __builtin_fmaf(n[k].y, ty, n[k].x * tx));
-    if (((__ballot(nd > 0.0f) | every) & lit[kUnit ? k : 0]) != 0ull)
+    if ((__ballot(!(nd <= n[k].w)) & lit[kUnit ? k : 0]) != 0ull)
       sh_accumulate<kSh2>(acc, p[k].w, f[k].x, f[k].y, f[k].z, tx, ty, tz, nd, shadowing[kUnit ? k : 0]);
   }
 }
