@@ -1510,9 +1510,9 @@ struct drv_batch {
 
 namespace {
 
-// With more shadow blocks than this in a view, DRV_BATCH_SPLIT_GATHER gives every
-// view a visibility launch of its own; with fewer such a launch leaves the GPU
-// idle behind its slowest rays for too long.  Per view of a captured batch, one
+// A view of more shadow blocks than this has a visibility launch of its own with
+// DRV_BATCH_SPLIT_GATHER; with fewer such a launch leaves the GPU idle behind its
+// slowest rays for too long.  Per view of a captured batch, one
 // launch / launches: 256 blocks 112 / 118 us (320x180), 152 / 157 (1280x720); 1024
 // blocks 250 / 239 and 280 / 272; 64 views of 256-2048 blocks at 720p-4K 18.9 /
 // 13.5 ms.
@@ -1615,20 +1615,21 @@ int batch_split(drv_batch* b, const drv_rsm* rsms, const drv_spot_light* lights)
   drv_ctx* v0 = b->views[0];
   const int grid = persistent_grid(v0);
   const uint32_t nv = static_cast<uint32_t>(n);
+  const uint32_t most = b->cpw == DRV_BATCH_SPLIT_GATHER ? kQueuedBlocks : 0xffffffffu;
   drvk::launch_batch_split_prepare(b->d_split, nv, b->d_totals, b->sh_bands, b->shadow, max_vpl, max_march,
-                                   static_cast<uint32_t>(grid) * 4u, b->stream);
-  bool large = false;
-  for (const drvk::SplitViewHost& d : hv) large = large || d.n_blocks > kQueuedBlocks;
-  if (b->shadow && b->cpw == DRV_BATCH_SPLIT_GATHER && large) {
-    // Each view's visibility with the single-view kernel and launch shape.
+                                   static_cast<uint32_t>(grid) * 4u, most, b->stream);
+  if (b->shadow) {
+    bool queued = false;
     for (size_t v = 0; v < n; ++v) {
       drv_ctx* ctx = b->views[v];
-      drvk::launch_visibility(ctx->vol, hv[v].vox, ctx->caches, b->stride, ctx->counter, ctx->blocks,
-                              hv[v].n_blocks, ctx->visibility, hv[v].vis_pitch, nullptr, ctx->tune,
-                              persistent_grid(ctx), b->stream, ctx->march);
+      if (hv[v].n_blocks > most)  // the single-view kernel and launch shape
+        drvk::launch_visibility(ctx->vol, hv[v].vox, ctx->caches, b->stride, ctx->counter, ctx->blocks,
+                                hv[v].n_blocks, ctx->visibility, hv[v].vis_pitch, nullptr, ctx->tune,
+                                persistent_grid(ctx), b->stream, ctx->march);
+      else
+        queued = true;
     }
-  } else if (b->shadow) {
-    drvk::launch_batch_split_visibility(b->d_split, nv, b->d_totals, b->stride, grid, b->stream);
+    if (queued) drvk::launch_batch_split_visibility(b->d_split, nv, b->d_totals, b->stride, grid, b->stream);
   }
   batch_voxels_read(b);
   drvk::launch_batch_split_gather(b->d_split, nv, b->d_totals, b->stride, b->sh_bands, b->shadow, v0->shc, grid,
@@ -1884,8 +1885,17 @@ int drv_batch_autotune(drv_batch* b, const drv_rsm* rsms, const drv_spot_light* 
   uint32_t best_tile = keep_tile;
   const int32_t cpws[6] = {0, DRV_BATCH_SPLIT_QUEUE, DRV_BATCH_SPLIT_GATHER, 64, 32, 16};
   const bool per_view_only = b->specular || any_surrogate(b);
+  // Without a view that has a visibility launch of its own the split queues are
+  // one and the same: the one that tells such views apart is kept.
+  bool large = false;
+  for (size_t v = 0; v < n; ++v) {
+    uint32_t n_vpl = 0, interval = 0, n_blocks = 0;
+    large = large || (validate_light(b->views[v], &rsms[v], &lights[v], &n_vpl, &interval, &n_blocks) == DRV_OK &&
+                      n_blocks > kQueuedBlocks);
+  }
   for (int32_t cpw : cpws) {
     if (per_view_only && cpw != 0) continue;  // env-map or surrogate views: per-view passes only
+    if (!large && cpw == DRV_BATCH_SPLIT_QUEUE) continue;
     // Per-view passes and the split queue have no VPL tile: one candidate.
     for (uint32_t tile = cpw <= 0 ? max_vpl : 256; tile <= max_vpl; tile *= 2) {
       b->cpw = cpw;

@@ -321,9 +321,11 @@ void build_split_descs(const SplitViewHost* views, uint32_t n_views, void* host_
 // The split queue's launches: VPL/block/march records and the plan of every
 // view; the queued visibility; the queued SH gather and reduction.
 // max_march: the most march records of any view (n_blocks x kMarchSteps,
-// 0 without indirect shadows).
+// 0 without indirect shadows); most_blocks: views of more shadow blocks have no
+// items in the queued visibility.
 void launch_batch_split_prepare(void* descs, uint32_t n_views, SplitTotals* totals, int sh_bands, int shadow,
-                                uint32_t max_vpl, uint32_t max_march, uint32_t target_items, hipStream_t s);
+                                uint32_t max_vpl, uint32_t max_march, uint32_t target_items, uint32_t most_blocks,
+                                hipStream_t s);
 void launch_batch_split_visibility(void* descs, uint32_t n_views, SplitTotals* totals, int stride, int grid,
                                    hipStream_t s);
 void launch_batch_split_gather(void* descs, uint32_t n_views, SplitTotals* totals, int stride, int sh_bands,

@@ -239,13 +239,14 @@ __global__ __launch_bounds__(256) void k_split_prepare(const SplitDev* views, ui
 // thread took ~1 us per view), then one thread walks the LDS copy.
 constexpr uint32_t kPlanChunk = 1024;
 // Visibility items of the split queue: two neighbouring 64-cache tiles by two
-// neighbouring shadow blocks (one of each for a wave), as k_visibility_planned.
-__device__ __forceinline__ uint32_t vis_items(uint32_t tiles, uint32_t n_blocks) {
-  return ((tiles + 1u) / 2u) * ((n_blocks + 1u) / 2u);
+// neighbouring shadow blocks (one of each for a wave), as k_visibility_planned;
+// none for a view of more than `most_blocks`, which has a launch of its own.
+__device__ __forceinline__ uint32_t vis_items(uint32_t tiles, uint32_t n_blocks, uint32_t most_blocks) {
+  return n_blocks > most_blocks ? 0u : ((tiles + 1u) / 2u) * ((n_blocks + 1u) / 2u);
 }
 __global__ __launch_bounds__(256) void k_split_plan(SplitDev* views, uint32_t n_views, uint32_t target_items,
-                                                    int shadow, int sh2, SplitTotals* totals) {
-  __shared__ uint32_t live_s[kPlanChunk];
+                                                    int shadow, int sh2, uint32_t most_blocks, SplitTotals* totals) {
+  __shared__ uint32_t live_s[kPlanChunk], vis_s[kPlanChunk];
   __shared__ uint32_t all_tiles_s;
   __shared__ uint32_t s_s;
   __shared__ uint32_t run[3];  // running vis, gather, reduce offsets
@@ -282,6 +283,7 @@ __global__ __launch_bounds__(256) void k_split_plan(SplitDev* views, uint32_t n_
       const uint32_t quantum = d.interval > 64u ? d.interval : 64u;
       d.splits = plan_split_count(d.live, d.n_vpl, quantum, min(s_s, d.max_splits), 0xffffffffu);
       live_s[i] = (d.tiles << 9) | ((d.splits + 3u) / 4u);  // tiles < 2^23, groups <= 64
+      vis_s[i] = shadow ? vis_items(d.tiles, d.n_blocks, most_blocks) : 0u;
     }
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -291,7 +293,7 @@ __global__ __launch_bounds__(256) void k_split_plan(SplitDev* views, uint32_t n_
         d.vis_begin = run[0];
         d.gather_begin = run[1];
         d.reduce_begin = run[2];
-        if (shadow) run[0] += vis_items(tiles, d.n_blocks);
+        run[0] += vis_s[i];
         run[1] += tiles * groups;
         run[2] += tiles * n_jc;
       }
@@ -342,7 +344,7 @@ __device__ __forceinline__ VisView vis_view(const SplitDev* views, uint32_t v) {
   w.begin = d->vis_begin;
   w.tiles = d->tiles;
   w.n_blocks = d->n_blocks;
-  w.end = w.begin + vis_items(w.tiles, w.n_blocks);
+  w.end = w.begin + vis_items(w.tiles, w.n_blocks, 0xffffffffu);  // no item of another view finds it
   w.live = d->live;
   w.pitch = d->vis_pitch;
   w.caches = d->caches;
@@ -490,13 +492,14 @@ void build_split_descs(const SplitViewHost* views, uint32_t n_views, void* host_
 }
 
 void launch_batch_split_prepare(void* descs, uint32_t n_views, SplitTotals* totals, int sh_bands, int shadow,
-                                uint32_t max_vpl, uint32_t max_march, uint32_t target_items, hipStream_t s) {
+                                uint32_t max_vpl, uint32_t max_march, uint32_t target_items, uint32_t most_blocks,
+                                hipStream_t s) {
   SplitDev* d = static_cast<SplitDev*>(descs);
   const uint32_t vpl_groups = (max_vpl + 255u) / 256u;
   hipLaunchKernelGGL(k_split_prepare, dim3(vpl_groups + (max_march + 255u) / 256u, n_views), dim3(256), 0, s, d,
                      vpl_groups);
   hipLaunchKernelGGL(k_split_plan, dim3(1), dim3(256), 0, s, d, n_views, target_items, shadow, sh_bands >= 2 ? 1 : 0,
-                     totals);
+                     most_blocks, totals);
 }
 
 void launch_batch_split_visibility(void* descs, uint32_t n_views, SplitTotals* totals, int stride, int grid,

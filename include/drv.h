@@ -459,9 +459,9 @@ typedef struct drv_batch drv_batch;
  * items of every view, and the gather's VPL splits are planned over all views
  * together. */
 #define DRV_BATCH_SPLIT_QUEUE (-1)
-/* The split queue with the cone-traced visibility of each view in a launch of
- * its own (the single-view kernel) where a view has more than 512 shadow blocks,
- * and the other stages queued over all views. */
+/* The split queue with the cone-traced visibility of every view of more than
+ * 512 shadow blocks in a launch of its own (the single-view kernel); the other
+ * views' visibility and the other stages are queued over all views. */
 #define DRV_BATCH_SPLIT_GATHER (-2)
 
 /* A batch keeps pointers to its views (all on one stream): destroy it before
@@ -476,8 +476,8 @@ const char* drv_batch_last_error(const drv_batch* batch);
  * Caches per wavefront 0 selects per-view passes instead of the fused queue:
  * each view's own cone trace, SH gather and reduction (drv_light_caches)
  * back to back on the shared stream; DRV_BATCH_SPLIT_QUEUE selects the split
- * queue and DRV_BATCH_SPLIT_GATHER the split queue with per-view visibility
- * launches for large views (the VPL tile is then unused). */
+ * queue and DRV_BATCH_SPLIT_GATHER the split queue with visibility launches of
+ * their own for large views (the VPL tile is then unused). */
 int drv_batch_set_tuning(drv_batch* batch, int32_t caches_per_wave, int32_t vpl_tile, int32_t waves_per_cu);
 int drv_batch_get_tuning(const drv_batch* batch, int32_t* caches_per_wave, int32_t* vpl_tile, int32_t* waves_per_cu);
 /* rsms[i], lights[i] belong to view i. */
