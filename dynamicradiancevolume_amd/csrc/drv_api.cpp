@@ -531,7 +531,7 @@ int drv_destroy(drv_ctx* ctx) {
   dev_free(ctx->alloc_touched);
   dev_free(ctx->cav);
   dev_free(ctx->spec.atlas);
-  dev_free(ctx->spec.vpl_units);
+  dev_free(ctx->spec.vpl_runs);
   dev_free(ctx->spec.work);
   dev_free(ctx->spec.spill);
   dev_free(ctx->vox_target);
@@ -891,19 +891,20 @@ int drv_light_caches(drv_ctx* ctx, const drv_rsm* rsm, const drv_spot_light* lig
   }
   record(ctx, 5);
   const int specular = ctx->cfg.indirect_specular;
-  if (specular && n_vpl > ctx->spec.vpl_units_cap) {
-    dev_free(ctx->spec.vpl_units);
-    ctx->spec.vpl_units_cap = 0;
-    if ((rc = dev_alloc(ctx, &ctx->spec.vpl_units, static_cast<size_t>(n_vpl) * 3)) != DRV_OK) return rc;
-    ctx->spec.vpl_units_cap = n_vpl;
+  if (specular && n_vpl > ctx->spec.vpl_runs_cap) {
+    dev_free(ctx->spec.vpl_runs);
+    ctx->spec.vpl_runs_cap = 0;
+    if ((rc = dev_alloc(ctx, &ctx->spec.vpl_runs, static_cast<size_t>(n_vpl) * 3)) != DRV_OK) return rc;
+    ctx->spec.vpl_runs_cap = n_vpl;
   }
   // The gather's split plan rides on the VPL preparation (one launch less).
   const drvk::GatherPlan plan = drvk::gather_plan(ctx->counter, interval,
                                                   static_cast<uint32_t>(ctx->tune.gather_max_splits), grid);
   const drvk::VoxelView vview = voxel_view(ctx);
   drvk::launch_prepare_vpls(*rsm, *light, ctx->vpls, shadow ? ctx->blocks : nullptr, specular,
-                            specular ? ctx->spec.vpl_units : nullptr, &plan, ctx->stream,
-                            shadow ? ctx->march : nullptr, &vview);
+                            specular ? ctx->spec.vpl_runs : nullptr, &plan, ctx->stream,
+                            shadow ? ctx->march : nullptr, &vview,
+                            drvk::specular_queue(n_vpl, interval, shadow));
   record(ctx, 6);
   join_voxels_for_read(ctx);
   if (use_net) {
@@ -931,7 +932,7 @@ int drv_light_caches(drv_ctx* ctx, const drv_rsm* rsm, const drv_spot_light* lig
   if (specular) {
     // renderer.cpp:553-558: LightCachesRSM with the env-map writes, then
     // PrepareSpecularEnvmaps.
-    drvk::launch_specular(ctx->frame.camera_position, ctx->caches, stride, ctx->counter, ctx->spec.vpl_units, n_vpl,
+    drvk::launch_specular(ctx->frame.camera_position, ctx->caches, stride, ctx->counter, ctx->spec.vpl_runs, n_vpl,
                           shadow ? ctx->visibility : nullptr, static_cast<uint32_t>(cap), interval, ctx->spec,
                           ctx->spec_first ? 1 : 0, ctx->cu_count * 8, ctx->stream);
     ctx->spec_first = false;

@@ -204,8 +204,8 @@ struct Tuning {
 constexpr int kSpecMaxLevels = 6;  // S <= 32
 struct SpecAtlas {
   uint32_t* atlas = nullptr;
-  float4* vpl_units = nullptr;  // VPL records of the current light by units
-  size_t vpl_units_cap = 0;     // VPLs
+  float4* vpl_runs = nullptr;  // VPL records of the current light by runs
+  size_t vpl_runs_cap = 0;     // VPLs
   float* work = nullptr;   // [max_caches][S * S][3]
   float* spill = nullptr;  // [max_caches][2S + 1][3]
   uint32_t width = 0, per_row = 0;
@@ -245,21 +245,24 @@ struct GatherPlan {
   uint32_t quantum, max_splits, target_items;
 };
 constexpr uint32_t kVplUnit = 16;  // consecutive VPLs; divides every read level's count (8x8 is the smallest)
+// Whether the specular gather queues units of kVplUnit VPLs; else 64 runs of n_vpl / 64.
+bool specular_queue(uint32_t n_vpl, uint32_t interval, bool shadow);
 inline GatherPlan gather_plan(Counter* counter, uint32_t interval, uint32_t max_splits, int grid) {
   return GatherPlan{counter, interval > 64u ? interval : 64u, max_splits, static_cast<uint32_t>(grid) * 4u};
 }
 
 // flux_cut: INDIRECT_SPECULAR skips VALs whose flux sums below 0.001
 // (cacheLightingRSM.comp:240-243); their flux is stored as zero.
-// vpl_units (optional): the same records for the specular gather, by units of
-// kVplUnit VPLs: three tables [place in the unit][unit] of (position, disc
-// area), (flux, whether any VPL of the unit has flux) and (normal, 0).
+// vpl_runs (optional): the same records for the specular gather.  With `queue`
+// by units of kVplUnit VPLs: three tables [place in the unit][unit] of (position,
+// disc area), (flux, whether any VPL of the unit has flux) and (normal, 0).  Else
+// by 64 runs of consecutive VPLs: these three of a VPL at [place in the run][run].
 // plan (optional): the gather's split plan, written by the first thread.
 // march (optional, with blocks): kMarchSteps MarchStep records per shadow
 // block, planned for the voxel levels of `vox`.
 void launch_prepare_vpls(const drv_rsm& rsm, const drv_spot_light& light, Vpl* vpls, ShadowBlock* blocks,
-                         int flux_cut, float4* vpl_units, const GatherPlan* plan, hipStream_t s,
-                         MarchStep* march = nullptr, const VoxelView* vox = nullptr);
+                         int flux_cut, float4* vpl_runs, const GatherPlan* plan, hipStream_t s,
+                         MarchStep* march = nullptr, const VoxelView* vox = nullptr, bool queue = false);
 // march (optional): the blocks' march plans; without them (or with a tuning
 // other than one block walk at one step per batch) the rays plan their own
 // samples, with the same values.
@@ -363,7 +366,7 @@ void launch_apply(const drv_config& cfg, const drv_volume& vol, const drv_frame&
 
 // Specular gather of one light into the work sums (first != 0: overwrite),
 // then quantization, mips and hole filling of every live cache's region.
-void launch_specular(const float* cam, const float* caches, int stride, const Counter* counter, const float4* vpl_units,
+void launch_specular(const float* cam, const float* caches, int stride, const Counter* counter, const float4* vpl_runs,
                      uint32_t n_vpl, const float* vis, uint32_t vis_pitch, uint32_t interval, const SpecAtlas& at,
                      int first, int grid, hipStream_t s);
 

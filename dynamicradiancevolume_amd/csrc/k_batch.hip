@@ -469,7 +469,9 @@ void build_split_descs(const SplitViewHost* views, uint32_t n_views, void* host_
     a.block = 1 << static_cast<int>(h.light.indirect_shadow_lod);
     a.flux_cut = 0;
     a.vpls = h.vpls;
-    a.vpl_units = nullptr;
+    a.vpl_runs = nullptr;
+    a.run = 0u;
+    a.run_tables = false;
     a.plan = nullptr;
     a.blocks = h.blocks;
     a.march = h.blocks ? h.march : nullptr;

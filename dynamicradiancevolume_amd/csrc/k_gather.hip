@@ -365,8 +365,8 @@ __global__ __launch_bounds__(256) void k_reduce(float* caches, int stride, const
 }  // namespace
 
 void launch_prepare_vpls(const drv_rsm& rsm, const drv_spot_light& light, Vpl* vpls, ShadowBlock* blocks,
-                         int flux_cut, float4* vpl_units, const GatherPlan* plan, hipStream_t s, MarchStep* march,
-                         const VoxelView* vox) {
+                         int flux_cut, float4* vpl_runs, const GatherPlan* plan, hipStream_t s, MarchStep* march,
+                         const VoxelView* vox, bool queue) {
   PrepArgs a;
   for (int i = 0; i < 16; ++i) a.inv_lvp[i] = light.inverse_light_view_projection[i];
   for (int i = 0; i < 3; ++i) a.light_pos[i] = light.light_position[i];
@@ -385,7 +385,9 @@ void launch_prepare_vpls(const drv_rsm& rsm, const drv_spot_light& light, Vpl* v
   a.block = 1 << static_cast<int>(light.indirect_shadow_lod);
   a.flux_cut = flux_cut;
   a.vpls = vpls;
-  a.vpl_units = vpl_units;
+  a.vpl_runs = vpl_runs;
+  a.run = queue ? kVplUnit : static_cast<uint32_t>(a.R) * static_cast<uint32_t>(a.H) / 64u;
+  a.run_tables = queue;
   a.plan = plan ? plan->counter : nullptr;
   a.quantum = plan ? plan->quantum : 0u;
   a.max_splits = plan ? plan->max_splits : 0u;

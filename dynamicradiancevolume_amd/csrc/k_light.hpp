@@ -30,7 +30,9 @@ struct PrepArgs {
   int block;  // B = 2^lod texels per block side
   int flux_cut;
   Vpl* vpls;
-  float4* vpl_units;  // optional copy by units of kVplUnit (see launch_prepare_vpls)
+  float4* vpl_runs;  // optional copy by runs (see launch_prepare_vpls)
+  uint32_t run;
+  bool run_tables;
   // Optional split plan of the gather (k_plan_gather), done by the first thread.
   Counter* plan;
   uint32_t quantum, max_splits, target_items;
@@ -127,14 +129,15 @@ __device__ __forceinline__ void prepare_vpl(const PrepArgs& a, uint32_t m, uint3
   const uint64_t any_odd = __ballot(odd);
   v.least_cos = odd ? __builtin_nanf("") : any_odd != 0ull ? -0.0f : 0.0f;
   a.vpls[m] = v;
-  if (a.vpl_units) {
+  if (a.vpl_runs) {
     bits |= __shfl_xor(bits, 4);
     bits |= __shfl_xor(bits, 8);
-    const size_t units = n / kVplUnit;
-    float4* u = a.vpl_units + (m % kVplUnit) * units + m / kVplUnit;
+    const size_t place = (m % a.run) * (n / a.run) + m / a.run;
+    float4* u = a.vpl_runs + (a.run_tables ? place : 3 * place);
+    const size_t next = a.run_tables ? n : 1u;
     u[0] = make_float4(v.px, v.py, v.pz, v.disc_area);
-    u[kVplUnit * units] = make_float4(v.fr, v.fg, v.fb, __uint_as_float(bits));
-    u[2 * kVplUnit * units] = make_float4(v.nx, v.ny, v.nz, 0.0f);
+    u[next] = make_float4(v.fr, v.fg, v.fb, __uint_as_float(bits));
+    u[2 * next] = make_float4(v.nx, v.ny, v.nz, 0.0f);
   }
   // Mean normal of a block's VPLs: the B x B texel square of a block is the
   // `interval` Morton-consecutive VPLs m .. m + interval - 1, i.e. adjacent

@@ -14,17 +14,17 @@
 //
 // MI355X design.  Two waves own one cache at a time and keep a map each in LDS
 // in FP32 (the reference read-modify-writes the R11G11B10F image once per
-// VAL).  Their lanes take units of 16 Morton-consecutive VALs, and only those
-// that light the cache: a wave tests 64 units at a time for shadowing and flux,
-// queues the rest in LDS and works off the queue 64 at a time, so that no lane
-// idles beside dark units (80 % of the units of a cache of specular_1080p).
-// Neighbouring VALs of a unit mostly reflect into the same texel, so a lane
-// sums runs in registers and adds a run into the LDS map only when its texel
-// changes (LDS float atomics to one address serialize, which made per-VAL adds
-// four times slower).  The light's FP32 sums go to a per-cache work buffer that
-// accumulates over the lights of a frame; the finalize kernel (one workgroup
-// per cache) quantizes, builds the mips and fills holes in LDS and writes every
-// level of the cache's atlas region once.
+// VAL).  Their lanes take runs of Morton-consecutive VALs: mostly they reflect
+// into the same texel, so a lane sums in registers and adds into the LDS map only
+// when its texel changes (LDS float atomics to one address serialize, which made
+// per-VAL adds four times slower).  With shadows in blocks of at least 16 VALs the
+// runs are units of 16, and only those that light the cache: a wave tests 64 units
+// at a time for shadowing and flux, queues the rest and works off the queue 64 at
+// a time, so that no lane idles beside dark units (80 % of the units of a cache of
+// specular_1080p).  Otherwise a lane's run is a 64th of the VALs.  The light's
+// FP32 sums go to a per-cache work buffer that accumulates over the lights of a
+// frame; the finalize kernel (one workgroup per cache) quantizes, builds the mips
+// and fills holes in LDS and writes every level of the cache's atlas region once.
 //
 // Texel index S: ivec2(HemisphericalProjection(h) * S + 0.5) reaches S for
 // half vectors near the horizon, so the reference's image store lands in
@@ -51,7 +51,7 @@ struct SpecGatherArgs {
   const float* caches;
   int stride;
   const Counter* counter;
-  const float4* units;  // VPLs by units (launch_prepare_vpls)
+  const float4* runs;  // VPLs by runs (launch_prepare_vpls)
   uint32_t n_vpl;
   const float* vis;  // [block][vis_pitch] or null (unshadowed)
   uint32_t vis_pitch;
@@ -70,45 +70,70 @@ __device__ __forceinline__ int texel_index(float p, int S) {
   return static_cast<int>(fminf(fmaxf(__builtin_fmaf(p, fs, 0.5f), 0.0f), fs));
 }
 
-// A unit that waits for a lane: its number and its shadowing.
-struct SpecEntry {
-  uint32_t unit;
-  float shadowing;
+// A lane's sum over the VALs in a row that reflect into one texel.
+struct TexelSum {
+  int tex = -1;
+  float r = 0.0f, g = 0.0f, b = 0.0f;
+  __device__ __forceinline__ void flush(float* map) const {
+    if (tex < 0) return;
+    float* t = map + tex * 3;
+    atomicAdd(t, r);
+    atomicAdd(t + 1, g);
+    atomicAdd(t + 2, b);
+  }
 };
 
-// The shadowing of unit u for cache c: its block's, or with blocks smaller than
-// a unit whether any of them is lit (1 or 0; the steps look theirs up).
-__device__ __forceinline__ float unit_shadowing(const SpecGatherArgs& a, uint32_t u, uint32_t c) {
-  if (!a.vis) return 1.0f;
-  const float* v = a.vis + static_cast<size_t>(u * kVplUnit >> a.interval_log2) * a.vis_pitch + c;
-  if (a.interval >= kVplUnit) return *v;
-  float any = 0.0f;
-  for (uint32_t k = 0; k < kVplUnit; k += a.interval, v += a.vis_pitch) any = *v != 0.0f ? 1.0f : any;
-  return any;
+// One VAL (position and disc area, flux, normal) of cache wp.
+__device__ __forceinline__ void specular_val(TexelSum& run, float* map, int S, const f3& wp, const LocalFrame& fr,
+                                             float4 vp, float4 vf, float4 vn, float shadowing) {
+  // radianceIn, cacheLightingRSM.comp:246-264 (the SH gather's expressions)
+  const float tx0 = vp.x - wp.x, ty0 = vp.y - wp.y, tz0 = vp.z - wp.z;
+  const float d2 = __builtin_fmaf(tz0, tz0, __builtin_fmaf(ty0, ty0, tx0 * tx0));
+  const float inv = __builtin_amdgcn_rsqf(d2);
+  const float tx = tx0 * inv, ty = ty0 * inv, tz = tz0 * inv;
+  const float nd = -__builtin_fmaf(vn.z, tz, __builtin_fmaf(vn.y, ty, vn.x * tx));
+  const float f = fminf(1.0f, fmaxf(0.0f, nd)) * shadowing * __builtin_amdgcn_rcpf(d2 + vp.w);
+  // cacheLightingRSM.comp:281-335
+  const f3 l = to_local(fr, tx, ty, tz);
+  const float hz0 = l.z + 1.0f;
+  const float hi = __builtin_amdgcn_rsqf(__builtin_fmaf(hz0, hz0, __builtin_fmaf(l.y, l.y, l.x * l.x)));
+  const float hx = l.x * hi, hy = l.y * hi, hz = hz0 * hi;
+  float proj[2];
+  hemi_projection(hx, hy, hz, proj);
+  const int ix = texel_index(proj[0], S), iy = texel_index(proj[1], S);
+  const float k = f * fminf(1.0f, fmaxf(0.0f, __builtin_fmaf(hz, l.z, __builtin_fmaf(hy, l.y, hx * l.x))));
+  const float cr = vf.x * k, cg = vf.y * k, cb = vf.z * k;
+  if (cr == 0.0f && cg == 0.0f && cb == 0.0f) return;  // changes nothing
+  const int tex = iy * (S + 1) + ix;
+  if (tex != run.tex) {
+    run.flush(map);
+    run.tex = tex;
+    run.r = cr;
+    run.g = cg;
+    run.b = cb;
+  } else {
+    run.r += cr;
+    run.g += cg;
+    run.b += cb;
+  }
 }
 
-// Dynamic LDS: 4 maps of (S+1)^2 RGB floats, 4 queues of 128 units.  Wave half h
-// of a cache's two takes the units of the half h of the RSM into its own map,
-// and the pair writes map 0 + map 1 out (a fixed order), so twice as many
-// waves, each half as long, balance the SIMDs.  16384 VALs, 16x16 maps, 5775
-// caches, 21 % of whose units are lit: 270 us with 256 VALs in a row for each of
-// a cache's lanes, 140 (63 % of the cycles issue a vector instruction).
+// Dynamic LDS: 4 maps of (S+1)^2 RGB floats.  Wave half h of a cache's two takes
+// the half h of the units (kQueue) or of every lane's run into its own map, and
+// the pair writes map 0 + map 1 out (a fixed order), so twice as many waves, each
+// half as long, balance the SIMDs.  The queue is 128 units, two in each lane's
+// registers (in LDS it took a third of the waves of 32x32 maps).
+template <bool kQueue>
 __global__ __launch_bounds__(256) void k_specular_gather(SpecGatherArgs a) {
   extern __shared__ float lds[];
   const int S = a.S, S1 = S + 1;
   const uint32_t map_floats = static_cast<uint32_t>(S1 * S1 * 3);
   const uint32_t lane = threadIdx.x & 63u, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t pair = w >> 1, half = w & 1u;
-  SpecEntry* queue = reinterpret_cast<SpecEntry*>(lds) + w * 128u;
-  float* maps = lds + 4u * 128u * 2u;
-  float* map = maps + w * map_floats;
-  const float* map0 = maps + (2u * pair) * map_floats;
+  float* map = lds + w * map_floats;
+  const float* map0 = lds + (2u * pair) * map_floats;
   const float* map1 = map0 + map_floats;
   const uint32_t live = a.counter->live;
-  const uint32_t n_units = a.n_vpl / kVplUnit, mid = n_units / 2u;
-  const uint32_t u0 = half ? mid : 0u, u1 = half ? n_units : mid;
-  const size_t table = static_cast<size_t>(kVplUnit) * n_units;
-  const float4 *positions = a.units, *fluxes = a.units + table, *normals = a.units + 2 * table;
   for (uint32_t base = blockIdx.x * 2u; base < live; base += gridDim.x * 2u) {  // workgroup-uniform
     const uint32_t c = base + pair;
     const bool active = c < live;
@@ -118,90 +143,68 @@ __global__ __launch_bounds__(256) void k_specular_gather(SpecGatherArgs a) {
       const float* e = a.caches + static_cast<size_t>(c) * a.stride;
       const f3 wp = make3(e[0], e[1], e[2]);
       const LocalFrame fr = local_view_space(a.cam, wp);
-      uint32_t next = u0, queued = 0u;
-      while (next < u1 || queued != 0u) {
-        if (next < u1) {
-          const uint32_t u = next + lane;
-          const bool in = u < u1;
-          const uint32_t uc = in ? u : u0;
-          const float sh = unit_shadowing(a, uc, c);
-          const uint32_t flux = __float_as_uint(fluxes[uc].w);
-          const bool lit = in && ((sh != 0.0f && flux != 0u) || flux == kOddFlux);  // zero times an odd VAL counts
-          const uint64_t m = __ballot(lit);
-          const uint32_t at = queued + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32),
-                                                                 __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0u));
-          if (lit) queue[at] = SpecEntry{u, sh};
-          queued += static_cast<uint32_t>(__popcll(m));
-          next += 64u;
-          wave_lds_sync();
-          if (queued < 64u && next < u1) continue;
-          if (queued == 0u) break;
-        }
-        const uint32_t n = min(queued, 64u);
-        SpecEntry q = queue[lane];
-        if (lane >= n) q = SpecEntry{u0, 0.0f};
-        const SpecEntry rest = queue[64u + lane];
-        wave_lds_sync();
-        if (n + lane < queued) queue[lane] = rest;
-        queued -= n;
-        float shadowing = q.shadowing;
-        const bool small = a.vis && a.interval < kVplUnit && lane < n;
-        int run_tex = -1;
-        float run_r = 0.0f, run_g = 0.0f, run_b = 0.0f;
-#pragma unroll 2
-        for (uint32_t i = 0; i < kVplUnit; ++i) {
-          const size_t r = static_cast<size_t>(i) * n_units + q.unit;
-          const float4 vp = positions[r], vf = fluxes[r], vn = normals[r];
-          // Blocks smaller than a unit: the shadowing changes inside it.
-          if (small && (i & (a.interval - 1u)) == 0u)
-            shadowing = a.vis[static_cast<size_t>((q.unit * kVplUnit + i) >> a.interval_log2) * a.vis_pitch + c];
-          // radianceIn, cacheLightingRSM.comp:246-264 (the SH gather's expressions)
-          const float tx0 = vp.x - wp.x, ty0 = vp.y - wp.y, tz0 = vp.z - wp.z;
-          const float d2 = __builtin_fmaf(tz0, tz0, __builtin_fmaf(ty0, ty0, tx0 * tx0));
-          const float inv = __builtin_amdgcn_rsqf(d2);
-          const float tx = tx0 * inv, ty = ty0 * inv, tz = tz0 * inv;
-          const float nd = -__builtin_fmaf(vn.z, tz, __builtin_fmaf(vn.y, ty, vn.x * tx));
-          const float f = fminf(1.0f, fmaxf(0.0f, nd)) * shadowing * __builtin_amdgcn_rcpf(d2 + vp.w);
-          // cacheLightingRSM.comp:281-335
-          const f3 l = to_local(fr, tx, ty, tz);
-          const float hz0 = l.z + 1.0f;
-          const float hi = __builtin_amdgcn_rsqf(__builtin_fmaf(hz0, hz0, __builtin_fmaf(l.y, l.y, l.x * l.x)));
-          const float hx = l.x * hi, hy = l.y * hi, hz = hz0 * hi;
-          float proj[2];
-          hemi_projection(hx, hy, hz, proj);
-          const int ix = texel_index(proj[0], S), iy = texel_index(proj[1], S);
-          const float k = f * fminf(1.0f, fmaxf(0.0f, __builtin_fmaf(hz, l.z, __builtin_fmaf(hy, l.y, hx * l.x))));
-          // Run accumulation: consecutive VALs of a lane mostly hit the same
-          // texel, so the lane sums in registers and adds the run into the map
-          // when the texel changes (zero contributions change nothing).
-          const float cr = vf.x * k, cg = vf.y * k, cb = vf.z * k;
-          if (!(cr == 0.0f && cg == 0.0f && cb == 0.0f)) {
-            const int tex = iy * S1 + ix;
-            if (tex != run_tex) {
-              if (run_tex >= 0) {
-                float* t = map + run_tex * 3;
-                atomicAdd(t, run_r);
-                atomicAdd(t + 1, run_g);
-                atomicAdd(t + 2, run_b);
-              }
-              run_tex = tex;
-              run_r = cr;
-              run_g = cg;
-              run_b = cb;
-            } else {
-              run_r += cr;
-              run_g += cg;
-              run_b += cb;
+      if (kQueue) {
+        const uint32_t units = a.n_vpl / kVplUnit, mid = units / 2u, u1 = half ? units : mid;
+        const float4 *positions = a.runs, *fluxes = a.runs + a.n_vpl, *normals = fluxes + a.n_vpl;
+        uint32_t next = half ? mid : 0u, queued = 0u;
+        uint32_t unit = next, more_unit = 0u;  // entries `lane` and 64 + lane of the queue
+        float lit_by = 0.0f, more_lit_by = 0.0f;
+        while (next < u1 || queued != 0u) {
+          if (next < u1) {
+            const uint32_t u = min(next + lane, u1 - 1u);
+            const float sh = a.vis[static_cast<size_t>(u * kVplUnit >> a.interval_log2) * a.vis_pitch + c];
+            const uint32_t flux = __float_as_uint(fluxes[u].w);
+            // (Zero times an odd VAL counts.)
+            const bool lit = next + lane < u1 && ((sh != 0.0f && flux != 0u) || flux == kOddFlux);
+            const uint64_t m = __ballot(lit);
+            const uint32_t n = static_cast<uint32_t>(__popcll(m));
+            const uint32_t rank = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32),
+                                                            __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0u));
+            // Lit units go to the lanes from `queued` on, the others to the lanes left.
+            const int to = static_cast<int>(4u * ((queued + (lit ? rank : n + lane - rank)) & 63u));
+            const uint32_t got = static_cast<uint32_t>(__builtin_amdgcn_ds_permute(to, static_cast<int>(u)));
+            const float got_by = __builtin_bit_cast(
+                float, __builtin_amdgcn_ds_permute(to, __builtin_bit_cast(int, sh)));
+            const uint32_t place = (lane - queued) & 63u;
+            if (place < n && lane >= queued) {
+              unit = got;
+              lit_by = got_by;
+            } else if (place < n) {
+              more_unit = got;
+              more_lit_by = got_by;
             }
+            queued += n;
+            next += 64u;
+            if (queued < 64u && next < u1) continue;
+            if (queued == 0u) break;
           }
+          if (lane < queued) {
+            TexelSum run;
+#pragma unroll 2
+            for (uint32_t i = 0; i < kVplUnit; ++i) {
+              const size_t r = static_cast<size_t>(i) * units + unit;
+              specular_val(run, map, S, wp, fr, positions[r], fluxes[r], normals[r], lit_by);
+            }
+            run.flush(map);
+          }
+          queued -= min(queued, 64u);
+          unit = more_unit;
+          lit_by = more_lit_by;
         }
-        if (run_tex >= 0) {
-          float* t = map + run_tex * 3;
-          atomicAdd(t, run_r);
-          atomicAdd(t + 1, run_g);
-          atomicAdd(t + 2, run_b);
+      } else {
+        const uint32_t per_run = a.n_vpl / 64u, mid = per_run / 2u, i0 = half ? mid : 0u, i1 = half ? per_run : mid;
+        float shadowing = 1.0f;
+        TexelSum run;
+        for (uint32_t i = i0; i < i1; ++i) {
+          const uint32_t m = lane * per_run + i;
+          const float4* r = a.runs + 3 * static_cast<size_t>(i * 64u + lane);
+          const float4 vp = r[0], vf = r[1], vn = r[2];
+          // The block's shadowing changes every `interval` VALs.
+          if (a.vis && (i == i0 || (m & (a.interval - 1u)) == 0u))
+            shadowing = a.vis[static_cast<size_t>(m >> a.interval_log2) * a.vis_pitch + c];
+          specular_val(run, map, S, wp, fr, vp, vf, vn, shadowing);
         }
-        wave_lds_sync();
+        run.flush(map);
       }
     }
     __syncthreads();  // both maps of every pair are complete
@@ -349,7 +352,17 @@ __global__ __launch_bounds__(256) void k_specular_finalize(SpecFinalArgs a) {
 
 }  // namespace
 
-void launch_specular(const float* cam, const float* caches, int stride, const Counter* counter, const float4* vpl_units,
+// Units of 16 VALs in a queue where whole units can be dark and there are enough
+// of them for the lanes; else runs of a 64th of the VALs.  Queue / runs, 16x16 maps:
+// 16384 VALs in blocks of 16, 6352 caches 139 / 312 us (32x32 maps 222 / 461); 4096
+// VALs 70 / 91, 1154 caches 30 / 31 (32x32 maps 45 / 42); 1024 VALs 50 / 38 and 19 /
+// 16; 64 VALs 61 / 19.  Without shadows 329 / 308, blocks of one VAL 325 / 268 (4096
+// VALs; of four 95 / 99, 1154 caches 38 / 32), as nearly all units are lit.
+bool specular_queue(uint32_t n_vpl, uint32_t interval, bool shadow) {
+  return shadow && interval >= kVplUnit && n_vpl >= 4096u;
+}
+
+void launch_specular(const float* cam, const float* caches, int stride, const Counter* counter, const float4* vpl_runs,
                      uint32_t n_vpl, const float* vis, uint32_t vis_pitch, uint32_t interval, const SpecAtlas& at,
                      int first, int grid, hipStream_t s) {
   SpecGatherArgs g;
@@ -357,7 +370,7 @@ void launch_specular(const float* cam, const float* caches, int stride, const Co
   g.caches = caches;
   g.stride = stride;
   g.counter = counter;
-  g.units = vpl_units;
+  g.runs = vpl_runs;
   g.n_vpl = n_vpl;
   g.vis = vis;
   g.vis_pitch = vis_pitch;
@@ -367,10 +380,11 @@ void launch_specular(const float* cam, const float* caches, int stride, const Co
   g.work = at.work;
   g.spill = at.spill;
   g.first = first;
-  const size_t glds = static_cast<size_t>(4) * ((at.S + 1) * (at.S + 1) * 3 * sizeof(float) + 128 * sizeof(SpecEntry));
+  const size_t glds = static_cast<size_t>(4) * (at.S + 1) * (at.S + 1) * 3 * sizeof(float);
   // More workgroups than fit at once (each takes two caches a round): the
   // hardware deals the last ones out as others finish.
-  hipLaunchKernelGGL(k_specular_gather, dim3(4 * grid), dim3(256), glds, s, g);
+  const auto gather = specular_queue(n_vpl, interval, vis != nullptr) ? k_specular_gather<true> : k_specular_gather<false>;
+  hipLaunchKernelGGL(gather, dim3(4 * grid), dim3(256), glds, s, g);
 
   SpecFinalArgs f;
   f.counter = counter;

@@ -149,6 +149,26 @@ def test_specular_unit_and_block_sizes_match_oracle(res, lod, wide, shadow):
     r.close()
 
 
+# Both ways of the gather on either side of the rule: the queue of units from 4096
+# VALs in blocks of at least 16 on (among them 2:1 maps, whose halves end inside a
+# wave's 64 units, and one unit in a block), runs of a 64th of the VALs below; maps
+# of 4 to 32 texels a side; dark units (the light's cone ends inside the map).
+@pytest.mark.parametrize("res,lod,wide,size", [(64, 2, 1, 8), (64, 2, 0, 32), (128, 2, 1, 4), (128, 1, 1, 8),
+                                               (64, 1, 0, 32), (128, 3, 0, 16)])
+def test_specular_queue_and_runs_match_oracle(res, lod, wide, size):
+    from dynamicradiancevolume_amd.workloads import CORNELL_256
+
+    light = replace(CORNELL_256.light, rsm_resolution=res, indirect_shadow_lod=lod, rsm_wide=wide)
+    fi = frame_inputs("cornell_256", light=light, width=96, height=64)
+    fi = replace(fi, workload=fi.workload.with_(specular=1, specular_size=size))
+    announce(f"specular rsm {res} lod {lod} wide {wide} maps {size}")
+    r, df = _run(fi)
+    _, live = r.cache_count()
+    o_atlas, _, _ = _oracle_atlas(fi, r.read_caches(live)[:, :3].copy())
+    _compare_atlas(fi.workload.config(), _gpu_atlas(r), o_atlas, live)
+    r.close()
+
+
 # A VAL of infinite flux that faces away, or whose shadow block a cache does not
 # see, adds infinity times zero to the texel it would reflect into: at most the
 # caches whose texel is a neighbour's stay finite.
