@@ -421,9 +421,13 @@ void launch_visibility(const drv_volume& vol, const VoxelView& vox, const float*
   a.march = march;
   const dim3 b(256);
   if (march && tune.visibility_kernel == 0 && tune.steps_per_batch == 1) {
-    // More blocks are more items: 2048 blocks (32768 VPLs) over twice the
-    // workgroups took 755 -> 715 us (the hardware deals smaller shares), 1024
-    // blocks 121 -> 123 us.
+    // More blocks are more items, which the hardware deals in smaller shares (the
+    // number of blocks is a power of two, so the factor is 1, 2 or 4).  Factors 1 /
+    // 2 / 4 / 8 in us: 1024 blocks, 5841 caches 149 / 149 / 153 / 174, 1960 caches 142
+    // / 147 / 150 / 170; 2048 blocks at 3840x2160 755 / 715; 4096 blocks 599 / 567 /
+    // 576 / 575, in 256^3 voxels 3715 / 3276 / 2898 / 2507, 4197 caches of a closed
+    // room 662 / 604 / 562 / 571; 16384 blocks 1189 / 1153 / 1157 / 1201, 1960 caches
+    // 554 / 536 / 548 / 569.
     grid *= static_cast<int>(std::min(4u, std::max(1u, n_blocks / 1024u)));
   }
   const dim3 g(grid);

@@ -165,65 +165,49 @@ __device__ __forceinline__ MarchStep march_step(MarchSteps pl, uint32_t offset) 
   return e;
 }
 
-// Samples n0 .. n1 - 1 of a ray set up by trace_setup (the ray has taken
-// samples 0 .. n0 - 1), with the samples of its block's march plan `pl`:
-// every lane of the calling wave traces towards the same block (pl is
-// wave-uniform) and starts at n0.  Each sample is the one trace_batch takes
-// (same positions, levels, weights and transmittance updates, so the same
-// values), without the ray computing the plan itself: per step the lanes
-// only advance, fetch and blend.  Returns true when the ray stopped at one
-// of the samples (its march reached the goal or it turned opaque).  t.s
-// (samples taken) is kept only with kCount: it costs a VALU instruction per
+// The whole trace of cache wp towards block b, the same for every lane of the
+// wave, with the samples of the block's march plan; lanes with live = false take
+// no samples.  Each sample is the one trace_batch takes (same positions, levels,
+// weights and transmittance updates, so the same values), without the ray
+// computing the plan itself: per step the lanes only advance, fetch and blend.
+// t.s (samples taken) is kept only with kCount: it costs a VALU instruction per
 // sample and only the step counters read it.
-template <bool kCount = false, bool kFloatIndex = false>
-__device__ __forceinline__ bool march_planned(MarchSteps pl, const MarchStep& first, __amdgpu_buffer_rsrc_t cr,
-                                              Trace& t, int n0, int n1) {
-  // The lanes that march stay in lockstep (all start at sample n0 and take
-  // one sample per iteration until they stop), so the sample index is
-  // wave-uniform and the record load is scalar.
-  bool stopped = false;
-  uint32_t off = __builtin_amdgcn_readfirstlane(n0) * sizeof(MarchStep);
-  MarchStep next = first;
-  for (int n = n0; n < n1; ++n) {
-    const MarchStep cur = next;
-    off += sizeof(MarchStep);  // past sample 31: the next block's record, or the padding one, not used
-    t.px = __builtin_fmaf(t.dx, cur.step, t.px);
-    t.py = __builtin_fmaf(t.dy, cur.step, t.py);
-    t.pz = __builtin_fmaf(t.dz, cur.step, t.pz);
-    const Footprint f1 = footprint<kFloatIndex>(cur.lv[0], t.px, t.py, t.pz);
-    const corner_t c1 = corner_load(cr, f1.offset);
-    Footprint f2;
-    corner_t c2;
-    if (cur.two) {  // wave-uniform; both loads are issued before either record is blended
-      f2 = footprint<kFloatIndex>(cur.lv[1], t.px, t.py, t.pz);
-      c2 = corner_load(cr, f2.offset);
-    }
-    next = march_step(pl, off);  // a step ahead
-    const float o1 = blend_corner(c1, f1.ax, f1.ay, f1.az);
-    float o = o1;
-    if (cur.two) o = __builtin_fmaf(cur.frac, blend_corner(c2, f2.ax, f2.ay, f2.az) - o1, o1);
-    t.trans = __builtin_fmaf(-(t.trans * (1.0f / 255.0f)), o, t.trans);
-    if (kCount) t.s = n + 1;
-    if (cur.dist >= t.goal || t.trans <= kOpaque) {
-      stopped = true;
-      break;
-    }
-  }
-  return stopped;
-}
-
-// The whole trace (samples 0 .. 31) of cache wp towards block b, the same for
-// every lane of the wave; lanes with live = false take no samples.
 template <bool kCount = false, bool kFloatIndex = false>
 __device__ __forceinline__ Trace trace_planned(const VoxelView& vox, __amdgpu_buffer_rsrc_t cr, const ShadowBlock* blocks,
                                                const MarchStep* march, uint32_t b, float voxel_size, f3 wp, f3 vpos,
                                                bool live) {
   const MarchSteps pl = march_steps(march, b);
-  const MarchStep first = march_step(pl, 0u);
+  MarchStep next = march_step(pl, 0u);
   const ShadowBlock rec = block_record(blocks, b);
   Trace t = trace_setup(vox, voxel_size, wp, vpos, rec);
-  asm volatile("" ::"s"(first.step));  // keeps the load above the branch, beside the ones before it
-  if (live) march_planned<kCount, kFloatIndex>(pl, first, cr, t, 0, kMarchSteps);
+  asm volatile("" ::"s"(next.step));  // keeps the load above the branch, beside the ones before it
+  if (live) {
+    // The lanes that march stay in lockstep (one sample per iteration until they
+    // stop), so the sample index is wave-uniform and the record load is scalar.
+    uint32_t off = 0u;
+    for (int n = 0; n < kMarchSteps; ++n) {
+      const MarchStep cur = next;
+      off += sizeof(MarchStep);  // past sample 31: the next block's record, or the padding one, not used
+      t.px = __builtin_fmaf(t.dx, cur.step, t.px);
+      t.py = __builtin_fmaf(t.dy, cur.step, t.py);
+      t.pz = __builtin_fmaf(t.dz, cur.step, t.pz);
+      const Footprint f1 = footprint<kFloatIndex>(cur.lv[0], t.px, t.py, t.pz);
+      const corner_t c1 = corner_load(cr, f1.offset);
+      Footprint f2;
+      corner_t c2;
+      if (cur.two) {  // wave-uniform; both loads are issued before either record is blended
+        f2 = footprint<kFloatIndex>(cur.lv[1], t.px, t.py, t.pz);
+        c2 = corner_load(cr, f2.offset);
+      }
+      next = march_step(pl, off);  // a step ahead
+      const float o1 = blend_corner(c1, f1.ax, f1.ay, f1.az);
+      float o = o1;
+      if (cur.two) o = __builtin_fmaf(cur.frac, blend_corner(c2, f2.ax, f2.ay, f2.az) - o1, o1);
+      t.trans = __builtin_fmaf(-(t.trans * (1.0f / 255.0f)), o, t.trans);
+      if (kCount) t.s = n + 1;
+      if (cur.dist >= t.goal || t.trans <= kOpaque) break;
+    }
+  }
   return t;
 }
 
