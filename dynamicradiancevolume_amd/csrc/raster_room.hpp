@@ -17,10 +17,15 @@ constexpr uint32_t kHeadWords = 8;  // counters before those of the tiles
 
 // Windows of at least this many tiles take the tiled raster: a tile is one
 // workgroup's work, and a small window's few tiles hold many triangles each
-// and leave the chip idle.  1.0M triangles, tiled / two passes: 306 / 228 us at
-// 256x256 (256 tiles; an RSM 439 / 111), 238 / 424 at 480x270 (510), 191 / 684 at
-// 640x360, 259 / 1907 at 1920x1080; 2176 large triangles: 43 / 58, 47 / 65,
-// 54 / 74, 165 / 335.
+// and leave the chip idle.  us in two passes / tiled, of 1.0M, 157k, 12k and 2176
+// (large) triangles:
+//   view 256x256 (256 tiles)   155 / 402   78 / 188   65 / 77    55 / 45
+//   view 400x240 (375)         293 / 276  103 / 138   64 / 68    60 / 43
+//   view 480x270 (510)         407 / 239  121 / 125   68 / 72    66 / 45
+//   view 640x360 (920)         683 / 198  203 / 107  133 / 69   121 / 49
+//   RSM 256x256                 89 / 411   71 / 172   63 / 94    98 / 72
+//   RSM 512x512 (1024)         269 / 255  116 / 146   84 / 98   191 / 82
+//   RSM 1024x1024             1633 / 266  380 / 187  198 / 136  423 / 129
 constexpr int kMinTiles = 384;
 
 inline int tile_count(int w, int h) { return ((w + kTile - 1) / kTile) * ((h + kTile - 1) / kTile); }
