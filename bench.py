@@ -122,7 +122,7 @@ def _cpu_baseline(fi, r, n_threads: int, budget_s: float):
 # SH-error statements against the FP64 oracle: the GPU results are captured
 # during the run (cache positions and SH of a seeded subset, the device's
 # voxel mips), and the oracle evaluates them on the host in the CPU leg at
-# the end, as a checker.
+# the end.
 _FP64_PENDING = []
 
 

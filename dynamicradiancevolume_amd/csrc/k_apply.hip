@@ -233,9 +233,9 @@ __device__ __forceinline__ void corner_caches(const ApplyArgs& a, bool active, u
 // each, the 8 corners' loads in flight together - and staged in LDS, where
 // their lanes read them; lanes with a third or later address load their own
 // entry, lanes without a cache (an unclaimed cell, one past the live caches)
-// read zeros.  Bound by vector instructions in large images (3840x2160: 167 us)
+// read zeros.  Bound by vector instructions in large images (3840x2160: 165 us)
 // and by the chain of loads in small ones, so the loads stand outside of
-// branches: 320x180 19.5 -> 14.1 us, 256x256 14.1 -> 9.8, 1920x1080 52 -> 47 (66
+// branches: 320x180 19.5 -> 14.1 us, 256x256 14.1 -> 9.8, 1920x1080 52 -> 48 (66
 // with the sums on the matrix unit, 4x4x1 with an entry broadcast).  Per lane the
 // arithmetic and its order are those of one fetch per pixel.  Every lane of
 // the wave must call this (the staging is cooperative); `active` = false lanes

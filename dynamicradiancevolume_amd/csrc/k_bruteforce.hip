@@ -18,8 +18,8 @@
 //  - groups that face away from, or lie behind, the surface of every pixel of
 //    the tile are skipped after the two cosines' signs: 59 % of the groups
 //    with flux on boxes_1080p, 39 % on a 637x359 view of 300 boxes.
-// 1920x1080 x 16384 VALs, diffuse: 25.6 -> 7.7 ms; 637x359 x 4096, whole BRDF:
-// 1.78 -> 0.67 ms.  Two and four pixels per lane (fewer scalar loads per pair)
+// 1920x1080 x 16384 VALs, diffuse: 25.6 -> 7.6 ms; 637x359 x 4096, whole BRDF:
+// 1.78 -> 0.68 ms.  Two and four pixels per lane (fewer scalar loads per pair)
 // took 15.8 and 16.6 ms against 14.9 ms with one, before the second skip.
 #include <type_traits>
 

@@ -1,6 +1,6 @@
 /*
  * drv_oracle.h - CPU restatement of DynamicRadianceVolume's indirect-lighting
- * hot path.  TEST INFRASTRUCTURE ONLY: it is the checker the HIP path is
+ * hot path.  TEST INFRASTRUCTURE ONLY: it is what the HIP path is
  * compared against and the CPU baseline the benchmark times.  Nothing in the
  * product links, loads or calls it.
  *

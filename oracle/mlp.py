@@ -1,6 +1,6 @@
 """CPU restatement of the surrogate visibility network (numpy).
 
-TEST INFRASTRUCTURE ONLY: the checker that the HIP forward and training
+TEST INFRASTRUCTURE ONLY: what the HIP forward and training
 kernels are compared against.  The network has no counterpart in the
 reference; it stands in for the cone trace of
 shader/cacheLightingRSM.comp:167-231.

@@ -1,7 +1,7 @@
 """ctypes bindings of the CPU oracle (``liborc.so``).
 
 TEST INFRASTRUCTURE ONLY.  Imported by ``tests/``, ``__graft_entry__.smoke()``
-and the ``cpu_baseline`` leg of ``bench.py`` - as the checker and the CPU
+and the ``cpu_baseline`` leg of ``bench.py`` - for comparison and as the CPU
 baseline, never as a product path.
 """
 from __future__ import annotations
